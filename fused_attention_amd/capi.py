@@ -12,7 +12,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libfused_attn_gfx950.so")
 
 # every symbol include/fused_attn.h declares
-EXPORTS = ("fa_fwd", "fa_fwd_ex", "fa_fwd_strided", "fa_fwd_plan", "fa_fwd_query", "fa_fwd_reference_bias", "fa_strerror",
+EXPORTS = ("fa_fwd", "fa_fwd_ex", "fa_fwd_strided", "fa_fwd_plan", "fa_fwd_variant", "fa_fwd_query", "fa_fwd_reference_bias", "fa_strerror",
            "fa_fwd_timed", "fa_fwd_timed_ex", "fa_qkv_proj", "fa_qkv_proj_plan")
 FLAG_CAUSAL = 1
 FLAG_BF16 = 2
@@ -58,6 +58,8 @@ def load_library():
     lib.fa_qkv_proj_plan.restype = ctypes.c_int
     lib.fa_fwd_plan.argtypes = [i64, i64, i64, i64, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     lib.fa_fwd_plan.restype = ctypes.c_int
+    lib.fa_fwd_variant.argtypes = lib.fa_fwd_plan.argtypes
+    lib.fa_fwd_variant.restype = ctypes.c_int
     lib.fa_fwd_query.argtypes = [i64]
     lib.fa_fwd_query.restype = ctypes.c_int
     lib.fa_fwd_reference_bias.argtypes = [i64]
@@ -83,6 +85,16 @@ def launch_plan(B, R, L, H, causal=False, has_mask=False):
     _check(load_library().fa_fwd_plan(B, R, L, H, FLAG_CAUSAL if causal else 0, 1 if has_mask else 0, out))
     keys = ("waves", "rows_per_wave", "workgroups", "working", "per_head", "heads_per_xcd", "matrix_tile")
     return dict(zip(keys, out))
+
+
+def launch_variant(B, R, L, H, causal=False, has_mask=False):
+    """What fa_fwd_variant reports for a problem, as a dict.  Needs no GPU."""
+    out = (ctypes.c_int * 7)()
+    _check(load_library().fa_fwd_variant(B, R, L, H, FLAG_CAUSAL if causal else 0, 1 if has_mask else 0, out))
+    keys = ("kernel", "waves", "rows", "key_groups", "workgroups", "working", "per_head")
+    res = dict(zip(keys, out))
+    res["kernel"] = ("tile", "split", "group")[res["kernel"]]
+    return res
 
 
 def projection_plan(B, L, F_in, R, H):

@@ -7,6 +7,10 @@
 
 #include "../../include/fused_attn.h"
 
+#ifdef FA_TUNE
+#include <cstdio>
+#include <cstdlib>
+#endif
 #include <mutex>
 #include <utility>
 #include <vector>
@@ -23,16 +27,15 @@ struct Shape {
     int rows() const { return waves * 32 * nqb; }
 };
 
-// Three shapes, picked by how the problem's workgroups fill the 256 compute units:
-//   {8, 2}  eight 64-row waves share one K/V stream, run by the ping-pong kernel, 512 queries per
-//           workgroup, one resident per compute unit (head_dim <= 64 only: with head_dim 128 a
-//           64-row wave would need the whole register file of a SIMD);
-//   {8, 1}  the same kernel with 32-row waves, 256 queries per workgroup: the only ping-pong
-//           shape of head_dim 128 (one resident per compute unit); with head_dim <= 64 it serves
-//           the grids that {8, 2} fills badly (without mask two are resident per compute unit;
-//           the causal and the additive-mask variants do not fit 128 registers and run one);
-//   {4, 1}  four 32-row waves, 128 queries per workgroup, three (head_dim <= 64) or two
-//           (head_dim 128) resident per compute unit: more, smaller workgroups for small problems.
+// The tile kernels' shapes (fwd_kernel_pingpong, fwd_kernel_pp16), picked by how the problem's workgroups fill
+// the 256 compute units; pick_variant below then weighs that launch against the key-split and group
+// kernels, which take everything else:
+//   {8, 2}  eight 64-row waves share one K/V stream, 512 queries per workgroup, one resident per
+//           compute unit (head_dim <= 64 only: with head_dim 128 a 64-row wave would need the whole
+//           register file of a SIMD);
+//   {8, 1}  the same with 32-row waves, 256 queries per workgroup: head_dim 128 (with head_dim <= 64 the
+//           group kernel is the faster one of the two on every grid);
+//   {4, 1}  too few workgroups of either: no tile kernel.
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // How well a shape uses the chip, in 1/1024: the share of the (rounds x slots) grid of resident
@@ -102,14 +105,12 @@ CausalPlan plan_causal_walk(int64_t heads, int64_t n, int64_t H) {
     return worst * 100 <= paired.blocks * 92 ? CausalPlan{true, worst} : paired;
 }
 
-// mask_rows_aligned: an additive mask whose rows are 16-byte aligned (L % 8 == 0, aligned pointer).
-Shape pick_shape(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool mask_rows_aligned,
+// mask_chunks: an additive mask whose rows hold a 16-byte chunk at least and stay below 2^24 values (the
+// ping-pong kernel keeps 32-bit byte offsets inside the 64 mask rows of a wave).
+Shape pick_shape(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool mask_chunks,
                  bool causal) {
     const int64_t heads = B * R;
-    // The ping-pong kernel takes an additive mask only through its coalesced, LDS-staged fetch;
-    // any other mask goes to four 32-row waves (the mask staging registers and LDS slabs leave room
-    // for two such workgroups per compute unit, not for 64-row waves).
-    if (has_mask && !mask_rows_aligned) return {4, 1};
+    if (has_mask && !mask_chunks) return {4, 1};
     // The ping-pong kernel is the fastest per compute unit, so it is taken whenever its
     // workgroups fill the chip well enough.  Thresholds measured on MI355X: a lone round may be
     // emptier than the tail of several, because idle units leave the busy ones more of the
@@ -169,21 +170,6 @@ hipError_t allow_large_lds(const void* kernel, int bytes) {
 }
 
 // BF selects the bf16 instantiation (namespace fa::bf16) of the same kernel source.
-template <int H, int NW, int NQB, int WPE, int MODE, bool BF>
-hipError_t launch(const fa::FwdParams& p, hipStream_t stream) {
-    constexpr int lds = MODE == fa::kAdditive ? fa::lds_bytes_masked<H, NW, kKeyTile, NQB>() : fa::lds_bytes<H, NW, kKeyTile>();
-    auto kernel = BF ? fa::bf16::fwd_kernel<H, NW, kKeyTile, NQB, WPE, MODE> : fa::fwd_kernel<H, NW, kKeyTile, NQB, WPE, MODE>;
-    if constexpr (lds > 64 * 1024) {
-        const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), lds);
-        if (e != hipSuccess) return e;
-    }
-    const int grid = p.wgs_per_xcd * fa::kNumXcd;
-    // the launch's own status, not the thread's sticky last error (which may stem from the caller's code)
-    fa::FwdParams params = p;
-    void* args[] = {&params};
-    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(grid), dim3(NW * 64), args, lds, stream);
-}
-
 template <int H, int NW, int NQB, int WPE, int MODE, bool BF>
 hipError_t launch_pingpong(const fa::FwdParams& p, hipStream_t stream) {
     constexpr int lds = MODE == fa::kAdditive ? fa::lds_bytes_pingpong_masked<H, NW, NQB>() : fa::lds_bytes_pingpong<H, NQB>();
@@ -260,22 +246,11 @@ hipError_t dispatch_shape(Shape sh, const fa::FwdParams& p, hipStream_t stream) 
     // (plan_causal never asks for it elsewhere)
     constexpr int BASE = MODE == fa::kCausalDealt ? fa::kCausal : MODE;
     if (MODE == fa::kCausalDealt && (sh.waves != 8 || H < 64)) return hipErrorInvalidValue;
-    // the ping-pong kernel for the eight-wave shapes
-    if (sh.waves == 8) {
-        if constexpr (H > 64)
-            return launch_pingpong<H, 8, 1, 2, MODE, BF>(p, stream);
-        else if (sh.nqb == 2)
-            return launch_pingpong<H, 8, 2, 2, H < 64 ? BASE : MODE, BF>(p, stream);
-        else if constexpr (MODE == fa::kPlain)
-            return launch_pingpong<H, 8, 1, 4, MODE, BF>(p, stream);
-        else
-            return launch_pingpong<H, 8, 1, 2, H < 64 ? BASE : MODE, BF>(p, stream);
-    }
-    // four 32-row waves; three per SIMD where the registers allow it
-    if constexpr (H > 64 || MODE == fa::kAdditive)
-        return launch<H, 4, 1, 2, BASE, BF>(p, stream);
+    // 64-row waves, at head_dim 128 32-row waves
+    if constexpr (H > 64)
+        return sh.waves == 8 ? launch_pingpong<H, 8, 1, 2, MODE, BF>(p, stream) : hipErrorInvalidValue;
     else
-        return launch<H, 4, 1, 3, BASE, BF>(p, stream);
+        return sh.waves == 8 && sh.nqb == 2 ? launch_pingpong<H, 8, 2, 2, H < 64 ? BASE : MODE, BF>(p, stream) : hipErrorInvalidValue;
 }
 
 template <int MODE, bool BF>
@@ -292,6 +267,78 @@ hipError_t dispatch_head_dim(int64_t H, Shape sh, const fa::FwdParams& p, hipStr
 template <int MODE>
 hipError_t dispatch(int64_t H, Shape sh, const fa::FwdParams& p, hipStream_t stream, bool bf16) {
     return bf16 ? dispatch_head_dim<MODE, true>(H, sh, p, stream) : dispatch_head_dim<MODE, false>(H, sh, p, stream);
+}
+
+// Which kernel runs a problem: a tile kernel (the launch of pick_shape), the key-split kernel (`waves` share out
+// the keys of 16 query rows), or the group kernel with 16 NQ rows per wave and GK key groups (kGroup<NQ><GK>).
+enum VariantKind { kTile, kSplit, kGroup11, kGroup12, kGroup21 };
+struct Variant {
+    VariantKind kind;
+    int waves;
+};
+
+// The key-split kernel (16 query rows per workgroup).
+template <int H, int MODE, bool BF>
+hipError_t launch_split(const fa::FwdParams& p, hipStream_t stream) {
+    constexpr int WPE = H <= 64 ? 4 : 2;
+    auto kernel = BF ? fa::bf16::fwd_kernel_split<H, MODE, WPE> : fa::fwd_kernel_split<H, MODE, WPE>;
+    constexpr int most = fa::split_lds_bytes<H, MODE == fa::kAdditive>(fa::kSplitMaxWaves);
+    if constexpr (most > 64 * 1024) {
+        const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), most);
+        if (e != hipSuccess) return e;
+    }
+    fa::FwdParams params = p;
+    void* args[] = {&params};
+    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(p.wgs_per_xcd * fa::kNumXcd), dim3(p.waves * 64), args,
+                           fa::split_lds_bytes<H, MODE == fa::kAdditive>(p.waves), stream);
+}
+
+// The group kernel: 16 NQ query rows per wave, GK key groups.
+template <int H, int NQ, int GK, int MODE, bool BF>
+hipError_t launch_group(const fa::FwdParams& p, hipStream_t stream) {
+    constexpr int lds = fa::group_lds_bytes<H, NQ, GK, MODE == fa::kAdditive>();
+    static_assert(lds <= 160 * 1024, "fits a compute unit");
+    constexpr int WPE = NQ == 1 || H <= 64 ? 4 : 2;
+    auto kernel = BF ? fa::bf16::fwd_kernel_group<H, NQ, GK, MODE, WPE> : fa::fwd_kernel_group<H, NQ, GK, MODE, WPE>;
+    if constexpr (lds > 64 * 1024) {
+        const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), lds);
+        if (e != hipSuccess) return e;
+    }
+    fa::FwdParams params = p;
+    void* args[] = {&params};
+    return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(p.wgs_per_xcd * fa::kNumXcd), dim3(8 * 64), args, lds, stream);
+}
+
+template <int H, int MODE, bool BF>
+hipError_t dispatch_variant(const Variant& v, const fa::FwdParams& p, hipStream_t stream) {
+    switch (v.kind) {
+        case kSplit: return launch_split<H, MODE, BF>(p, stream);
+        case kGroup11: return launch_group<H, 1, 1, MODE, BF>(p, stream);
+        case kGroup12: return launch_group<H, 1, 2, MODE, BF>(p, stream);
+        case kGroup21: return launch_group<H, 2, 1, MODE, BF>(p, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int MODE, bool BF>
+hipError_t dispatch_variant_head_dim(int64_t H, const Variant& v, const fa::FwdParams& p, hipStream_t stream) {
+    switch (H) {
+        case 16: return dispatch_variant<16, MODE, BF>(v, p, stream);
+        case 32: return dispatch_variant<32, MODE, BF>(v, p, stream);
+        case 64: return dispatch_variant<64, MODE, BF>(v, p, stream);
+        case 128: return dispatch_variant<128, MODE, BF>(v, p, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <bool BF>
+hipError_t dispatch_variant_mode(int64_t H, int mode, const Variant& v, const fa::FwdParams& p, hipStream_t stream) {
+    switch (mode) {
+        case fa::kPlain: return dispatch_variant_head_dim<fa::kPlain, BF>(H, v, p, stream);
+        case fa::kCausal: return dispatch_variant_head_dim<fa::kCausal, BF>(H, v, p, stream);
+        case fa::kAdditive: return dispatch_variant_head_dim<fa::kAdditive, BF>(H, v, p, stream);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
@@ -326,9 +373,8 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
     if (L > kMaxInt - 4096 || B > kMaxInt || R > kMaxInt || B * R > kMaxInt) return FA_ERR_TOO_LARGE;
     // the tile loaders keep 32-bit byte offsets inside a 64-key tile
     if (stride_l > ((int64_t)1 << 24)) return FA_ERR_TOO_LARGE;
-    // (the eight-wave kernel keeps 32-bit byte offsets inside the 64 mask rows of a wave)
     *shape = pick_shape(B, R, L, H, mask != nullptr,
-                        (L % 8) == 0 && L <= ((int64_t)1 << 24) && (reinterpret_cast<uintptr_t>(mask) & 15u) == 0, causal);
+                        L >= 8 && L <= ((int64_t)1 << 24), causal);
     const int64_t bq = shape->rows();
     int64_t n_qtiles = (L + bq - 1) / bq;
     int64_t total = 0;
@@ -371,6 +417,159 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
     p->wgs_per_xcd = (int)((total + fa::kNumXcd - 1) / fa::kNumXcd);
     p->scale_log2e = scale * 1.4426950408889634f;
     p->bias = fa_fwd_reference_bias(L);
+    return FA_OK;
+}
+
+// Time of a launch of the key-split or the group kernel, in microseconds: a fit over 1350 random shapes
+// (B 1..32, R 4..40, L 32..16384, every head_dim, plain, causal and masked) on MI355X; half of the
+// shapes are within 5 % of it.  What counts is the order of the estimates: choosing the smallest one
+// loses 1.8 % against the best kernel of each shape.
+//   split:  kLaunch + a ceil(sub-tiles / waves)              the longest wave
+//                   + b sub-tiles of all workgroups / 256    one compute unit's share of the work
+//                   + c workgroups / 256                     start and merge
+//   group:  kLaunch + a (sub-tiles + (rounds - 1) mean) / GK      the longest chain of workgroups
+//                   + b mean w / GK + c k                          w = workgroups per compute unit, taken
+//                                                                  half way between the mean and
+//                                                                  the most (k) of any
+// with sub-tiles of 32 keys, a causal tile's mean being about half of them, and rounds = k over the
+// workgroups resident per compute unit.
+struct Cost {
+    float a, b, c;
+};
+constexpr float kLaunch = 3.2f;
+// [head_dim 16, 32, 64, 128][without, with mask]
+constexpr Cost kCostSplit2[4][2] = {
+    {{0.139f, 0.053f, 0.087f}, {0.114f, 0.071f, 0.095f}},
+    {{0.143f, 0.057f, 0.129f}, {0.291f, 0.076f, 0.065f}},
+    {{0.291f, 0.071f, 0.316f}, {0.356f, 0.087f, 0.301f}},
+    {{0.525f, 0.136f, 1.05f}, {0.733f, 0.153f, 1.05f}},
+};
+constexpr Cost kCostSplit4[4][2] = {
+    {{0.201f, 0.055f, 0.152f}, {0.357f, 0.076f, 0.076f}},
+    {{0.124f, 0.057f, 0.223f}, {0.52f, 0.079f, 0.076f}},
+    {{0.265f, 0.072f, 0.525f}, {0.379f, 0.086f, 0.493f}},
+    {{0.612f, 0.137f, 1.81f}, {0.854f, 0.165f, 1.74f}},
+};
+constexpr Cost kCostGroup11[4][2] = {
+    {{0.242f, 0.102f, 0.452f}, {0.275f, 0.2f, 0.482f}},
+    {{0.162f, 0.14f, 0.353f}, {0.208f, 0.257f, 0.296f}},
+    {{0.215f, 0.22f, 0.449f}, {0.244f, 0.363f, 0.582f}},
+    {{0.422f, 0.327f, 0.944f}, {0.614f, 0.387f, 0.739f}},
+};
+constexpr Cost kCostGroup12[4][2] = {
+    {{0.249f, 0.128f, 0.661f}, {0.278f, 0.264f, 0.49f}},
+    {{0.143f, 0.169f, 0.735f}, {0.231f, 0.31f, 0.512f}},
+    {{0.252f, 0.186f, 1.24f}, {0.372f, 0.339f, 1.17f}},
+    {{0.36f, 0.392f, 2.61f}, {0.672f, 0.419f, 2.32f}},
+};
+constexpr Cost kCostGroup21[4][2] = {
+    {{0.371f, 0.128f, 0.639f}, {0.465f, 0.29f, 1.03f}},
+    {{0.289f, 0.2f, 0.514f}, {0.378f, 0.405f, 1.f}},
+    {{0.399f, 0.307f, 0.837f}, {0.559f, 0.446f, 1.33f}},
+    {{0.865f, 0.136f, 1.97f}, {0.934f, 0.601f, 1.97f}},
+};
+
+struct GroupShape {
+    VariantKind kind;
+    int nq, gk;
+    int resident[4];            // workgroups per compute unit, by head_dim
+    const Cost (*cost)[2];
+};
+constexpr GroupShape kGroups[] = {
+    {kGroup11, 1, 1, {3, 3, 3, 2}, kCostGroup11},
+    {kGroup12, 1, 2, {4, 4, 2, 2}, kCostGroup12},
+    {kGroup21, 2, 1, {2, 2, 2, 1}, kCostGroup21},
+};
+
+// The same for the eight-wave tile kernels that are left beside them: 64-row waves at head_dim 16 to 64,
+// 32-row waves at 128.  One workgroup per compute unit: a per sub-tile of a round, b per sub-tile of the mean
+// compute unit, c per round.
+constexpr Cost kCostTile[4][3] = {       // [head_dim][plain, causal, mask], fwd_kernel_pingpong
+    {{0.51f, 0.094f, 4.06f}, {0.686f, 0.f, 4.38f}, {0.991f, 0.f, 3.04f}},
+    {{0.419f, 0.258f, 3.15f}, {0.38f, 0.34f, 0.f}, {0.345f, 0.89f, 4.08f}},
+    {{0.408f, 0.58f, 4.08f}, {0.894f, 0.f, 0.f}, {1.159f, 0.291f, 4.27f}},
+    {{0.248f, 0.687f, 7.49f}, {0.716f, 0.f, 11.7f}, {0.933f, 0.363f, 6.72f}},
+};
+constexpr Cost kCostTile16[2][2] = {     // [head_dim 64, 128][plain, causal], fwd_kernel_pp16
+    {{0.27f, 0.645f, 7.08f}, {0.302f, 0.68f, 7.69f}},
+    {{0.f, 0.87f, 6.45f}, {0.f, 0.977f, 9.08f}},
+};
+
+float ceil_f(float x) {
+    const float t = (float)(int64_t)x;
+    return t < x ? t + 1.f : t;
+}
+
+// `tile` and `p` hold the launch of the tile kernels (validate).
+Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool causal, const Shape& tile,
+                     const fa::FwdParams& p) {
+#ifdef FA_TUNE
+    const char* env = getenv("FA_SPLIT");
+    if (env != nullptr) {
+        int nq = 0, nw = 0;
+        sscanf(env, "%d,%d", &nq, &nw);
+        if (nq == 0) return tile.waves == 8 && (H > 64 || tile.nqb == 2) ? Variant{kTile, 8} : Variant{kGroup11, 8};
+        return nw < 10 ? Variant{kSplit, nw} : Variant{nq == 2 ? kGroup21 : nw == 11 ? kGroup11 : kGroup12, 8};
+    }
+#endif
+    const int h = H == 16 ? 0 : H == 32 ? 1 : H == 64 ? 2 : 3;
+    const int m = has_mask ? 1 : 0;
+    const float heads = (float)(B * R), nsub = (float)ceil_div(L, 32);
+    Variant best{kGroup11, 8};
+    float least = 3.0e38f;
+    auto offer = [&](VariantKind kind, int waves, float us) {
+        if (us < least) {
+            least = us;
+            best = Variant{kind, waves};
+        }
+    };
+    // short sequences only: the fit ends at 2048, and the vector cache bounds the kernel on long ones
+    if (L <= 2048) {
+        const float wgs = heads * (float)ceil_div(L, 16) / kNumCu;
+        const float mean = causal ? 0.5f * (nsub + 0.5f) : nsub;
+        for (int waves = 2; waves <= (nsub > 2.f ? 4 : 2); waves += 2) {
+            const Cost& t = waves == 2 ? kCostSplit2[h][m] : kCostSplit4[h][m];
+            offer(kSplit, waves, kLaunch + t.a * ceil_f(nsub / (float)waves) + t.b * wgs * mean + t.c * wgs);
+        }
+    }
+    for (const GroupShape& g : kGroups) {
+        const int rows = 16 * g.nq * (8 / g.gk);
+        const float wgs = heads * (float)ceil_div(L, rows) / kNumCu, k = ceil_f(wgs);
+        const float mean = causal ? 0.5f * (nsub + (float)rows / 32.f) : nsub;
+        const float rounds = ceil_f(wgs / (float)g.resident[h]);
+        const Cost& t = g.cost[h][m];
+        offer(g.kind, 8, kLaunch + (t.a * (nsub + (rounds - 1.f) * mean) + t.b * mean * 0.5f * (wgs + k)) / (float)g.gk + t.c * k);
+    }
+    if (tile.waves == 8 && (H > 64 || tile.nqb == 2)) {
+        const float n = (float)ceil_div(L, tile.rows()), rows = (float)tile.rows();
+        float chain = nsub, u = (float)p.total_wgs / kNumCu;
+        if (causal && p.heads_per_xcd > 0) {
+            chain = 0.5f * n * (n + 1.f) * heads * rows / 32.f / kNumCu;
+            u = 1.f;
+        } else if (causal) {
+            chain = (n + 1.f) * rows / 32.f;
+        } else {
+            chain *= ceil_f(n / (float)p.n_qtiles);       // a pair of tiles per workgroup
+        }
+        const Cost& t = !has_mask && use_tiles16(H, tile, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
+                                                                     : kCostTile[h][has_mask ? 2 : causal ? 1 : 0];
+        const float rounds = ceil_f(u);
+        offer(kTile, 8, kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds);
+    }
+    return best;
+}
+
+// The launch of a key-split or group kernel in place of the tile kernels' one.
+int use_variant(const Variant& v, fa::FwdParams* p) {
+    int64_t rows = 16;
+    for (const GroupShape& g : kGroups)
+        if (g.kind == v.kind) rows = 16 * g.nq * (8 / g.gk);
+    const int64_t per_head = ceil_div(p->L, rows), total = (int64_t)p->B * p->R * per_head;
+    if (total > 0x7fffffff - 8) return FA_ERR_TOO_LARGE;
+    p->n_qtiles = (int)per_head;
+    p->total_wgs = (int)total;
+    p->wgs_per_xcd = (int)ceil_div(total, fa::kNumXcd);
+    p->waves = v.waves;
     return FA_OK;
 }
 
@@ -423,7 +622,13 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     if (rc != FA_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;
-    if (mask == nullptr && use_tiles16(H, shape, p, causal))
+    const Variant variant = pick_variant(B, R, L, H, mask != nullptr, causal, shape, p);
+    if (variant.kind != kTile) {
+        const int rcv = use_variant(variant, &p);
+        if (rcv != FA_OK) return rcv;
+        const int mode = causal ? fa::kCausal : mask != nullptr ? fa::kAdditive : fa::kPlain;
+        e = bf16 ? dispatch_variant_mode<true>(H, mode, variant, p, s) : dispatch_variant_mode<false>(H, mode, variant, p, s);
+    } else if (mask == nullptr && use_tiles16(H, shape, p, causal))
         e = launch_tiles16(H, causal ? (p.heads_per_xcd > 0 ? fa::kCausalDealt : fa::kCausal) : fa::kPlain, bf16, p, s);
     else if (causal && p.heads_per_xcd > 0)
         e = dispatch<fa::kCausalDealt>(H, shape, p, s, bf16);
@@ -456,6 +661,42 @@ int fa_fwd_plan(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_m
     plan[4] = p.n_qtiles;
     plan[5] = p.heads_per_xcd;
     plan[6] = (!has_mask && use_tiles16(H, shape, p, causal)) ? 16 : 32;
+    return FA_OK;
+}
+
+int fa_fwd_variant(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_mask, int* variant) {
+    if (variant == nullptr) return FA_ERR_NULL_POINTER;
+    if ((flags & ~(FA_FLAG_CAUSAL | FA_FLAG_BF16)) != 0) return FA_ERR_BAD_FLAGS;
+    const bool causal = (flags & FA_FLAG_CAUSAL) != 0;
+    if (causal && has_mask) return FA_ERR_BAD_FLAGS;
+    void* const fake = reinterpret_cast<void*>(static_cast<uintptr_t>(4096));
+    fa::FwdParams p;
+    Shape shape{4, 1};
+    const Strides dense{L * R * H, H, R * H};
+    int rc = validate(fake, fake, fake, has_mask ? fake : nullptr, fake, B, R, L, H, dense, dense, &p, 1.0f, &shape, causal, nullptr);
+    if (rc != FA_OK) return rc;
+    const Variant v = pick_variant(B, R, L, H, has_mask != 0, causal, shape, p);
+    int rows = shape.rows(), groups = 1;
+    if (v.kind == kSplit) {
+        rows = 16;
+        groups = v.waves;
+    }
+    for (const GroupShape& g : kGroups)
+        if (g.kind == v.kind) {
+            rows = 16 * g.nq * (8 / g.gk);
+            groups = g.gk;
+        }
+    if (v.kind != kTile) {
+        rc = use_variant(v, &p);
+        if (rc != FA_OK) return rc;
+    }
+    variant[0] = v.kind == kTile ? 0 : v.kind == kSplit ? 1 : 2;
+    variant[1] = v.waves;
+    variant[2] = rows;
+    variant[3] = groups;
+    variant[4] = p.wgs_per_xcd * fa::kNumXcd;
+    variant[5] = p.total_wgs;
+    variant[6] = p.n_qtiles;
     return FA_OK;
 }
 

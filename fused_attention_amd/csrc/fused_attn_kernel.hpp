@@ -5,18 +5,20 @@
 // reference's attention_kernel and every threadblock_* helper it calls
 // (reference include/fused_attn.cuh:48-538 and :605-858).
 //
-// Two kernels share the pieces in this file and in fused_attn_kernel_impl.inc:
-//   fwd_kernel           four waves, software pipelined inside each wave (plain and causal); its
-//                        additive-mask variant (plain loop) serves small grids and unaligned masks
-//   fwd_kernel_pingpong  eight waves in two groups that alternate vector and matrix phases;
-//                        plain, causal and additive mask (mask rows 16-byte aligned)
-// Work decomposition
-//   workgroup  = NW wave64s, each wave owns 32 NQB query rows (NQB = 1 or 2 blocks of 32)
-//   K/V        = streamed in 64-key tiles through an LDS ring: global -> registers -> LDS, two slots
-//                (fwd_kernel), or direct-to-LDS loads, three slots (fwd_kernel_pingpong)
-//   per 32 keys: S^T = K_sub * Q^T        v_mfma_f32_32x32x16_{f16,bf16}, Q held in registers
-//                online softmax on S^T     f32, state (m, l) per lane
-//                O^T += V_sub^T * P^T      same MFMA, V^T fetched with ds_read_b64_tr_b16
+// Five kernels share the pieces in this file:
+//   fwd_kernel_split     (fused_attn_split.inc) waves of a workgroup share out the keys of 16 query rows:
+//                        small grids
+//   fwd_kernel_group     (fused_attn_split.inc) eight waves that share key tiles in LDS and run free between
+//                        one barrier per tile: in-between grids, and large ones the next two
+//                        would fill badly
+//   fwd_kernel_pingpong  (fused_attn_kernel_impl.inc) eight waves in two groups that alternate vector and
+//                        matrix phases, 32 x 32 matrix tiles
+//   fwd_kernel_pp16      (fused_attn_kernel_impl.inc) the same phases, 16 x 16 matrix tiles
+//   (qkv_proj_kernel     qkv_proj_kernel.hpp: the projection in front of them)
+// all of them streaming K and V through LDS in tiles and computing, per 32 keys,
+//   S^T = K_sub * Q^T        v_mfma_f32_*_{f16,bf16}, Q held in registers
+//   online softmax on S^T    f32
+//   O^T += V_sub^T * P^T     V^T fetched with ds_read_b64_tr_b16
 //
 // Why the transposed products: in the 32x32 accumulator layout lane l owns column
 // (l % 32) -- one query -- and 16 of the 32 rows (keys); lane l^32 owns the other 16.
@@ -25,7 +27,7 @@
 // a valid B operand of the second product provided the A operand (V^T) enumerates keys
 // in the same order, which the transpose-read from the V tile provides.
 //
-// MFMA operand maps used below (g = lane / 32, ln = lane % 32):
+// MFMA operand maps of fwd_kernel_pingpong (g = lane / 32, ln = lane % 32; fwd_kernel_pp16 gives the 16 x 16 ones):
 //   A (32 x 16): lane holds row ln,   k = 8 g + i          (i = 0..7)
 //   B (16 x 32): lane holds col ln,   k = 8 g + i
 //   C (32 x 32): lane holds col ln,   row = 8 (r / 4) + 4 g + r % 4   (r = 0..15)
@@ -42,6 +44,7 @@ typedef short short4v __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));    // at any 16-bit element
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
@@ -68,47 +71,25 @@ struct FwdParams {
     int heads_per_xcd;     // causal eight-wave launches: 0 = every workgroup takes the pair of query tiles
                            // (t, n - 1 - t) of one head; > 0 = resident grid, the heads of an XCD's
                            // workgroups (B * R / 8 of them) dealt out tile by tile, see the kernel
+    int waves;             // key-split kernel: waves per workgroup
     float scale_log2e;     // scale * log2(e)
     float bias;            // bias of the reference of the exponentials, log2 units (see kBiasMin)
 };
 
 constexpr int kNumXcd = 8;
 
-// Kernel variants of the non-ping-pong kernel.
-constexpr int kPlain = 0;    // no mask: software-pipelined loop
+// Kernel variants.
+constexpr int kPlain = 0;    // no mask
 constexpr int kAdditive = 1; // additive [B, L, L] mask
 constexpr int kCausal = 2;   // key index <= query index, key tiles above the diagonal skipped
-constexpr int kCausalDealt = 3;   // eight-wave kernel only: causal with the query tiles dealt out to a resident grid
+constexpr int kCausalDealt = 3;   // tile kernels only: causal with the query tiles dealt out to a resident grid
 
 template <int H>
 struct Geometry {
     static constexpr int KS = H / 16;                    // k-steps of the QK^T product
     static constexpr int HV = H < 32 ? 32 : H;           // V columns held in LDS (zero padded)
     static constexpr int DB = HV / 32;                   // 32-row blocks of O^T
-    // Row strides (in f16) chosen so that the 16 rows touched by one quarter-wave of a
-    // ds_read_b128 (K) and the 4 rows touched by a 16-lane transpose read (V) fall into
-    // disjoint LDS banks.
-    static constexpr int KSTR = H + 8;
-    static constexpr int VSTR = HV == 32 ? 32 : HV + 32;
 };
-
-template <int H, int NW, int BK>
-constexpr int lds_bytes() {
-    using G = Geometry<H>;
-    return 2 * BK * (G::KSTR + G::VSTR) * (int)sizeof(_Float16);
-}
-
-// Additive-mask variant: behind the K/V buffers every wave has a private slab for the mask values
-// of its 32 NQB queries and the 64 keys of the current tile (row stride kMaskStr halves: 128 bytes
-// of mask plus 16 of padding).
-constexpr int kMaskStr = 72;
-// Not at head_dim 128: there the slabs would cost the second resident workgroup of a compute unit.
-template <int H>
-constexpr bool mask_staging() { return H <= 64; }
-template <int H, int NW, int BK, int NQB>
-constexpr int lds_bytes_masked() {
-    return lds_bytes<H, NW, BK>() + (mask_staging<H>() ? NW * 32 * NQB * kMaskStr * (int)sizeof(_Float16) : 0);
-}
 
 // NaN-propagating maximum: lowers to v_maximum3_f32 without the input canonicalisation that
 // fmaxf needs in IEEE mode.
@@ -136,70 +117,13 @@ __device__ __forceinline__ uint32_t pack_rtz(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
-// Streams K/V tiles from global memory into registers, and from registers into LDS.  K and V are
-// handled separately because the pipelined loop keeps K one tile ahead of V.
-template <int H, int NW, int BK>
-struct TileLoader {
-    using G = Geometry<H>;
-    static constexpr int CPR = H / 8;                       // 16-byte chunks per row
-    static constexpr int NCHUNK = BK * CPR;
-    static constexpr int NT = NW * 64;
-    static constexpr int NP = (NCHUNK + NT - 1) / NT;       // chunks per thread
-    static constexpr bool EXACT = NCHUNK % NT == 0;
-    u32x4 kreg[NP];
-    u32x4 vreg[NP];
-    uint32_t goff[NP];   // byte offset of this thread's chunk i from the first key of a tile
-
-    __device__ __forceinline__ void init(int64_t stride_l, int tid) {
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int idx = EXACT ? tid + i * NT : min(tid + i * NT, NCHUNK - 1);
-            goff[i] = (uint32_t)(((int64_t)(idx / CPR) * stride_l + (idx % CPR) * 8) * 2);
-        }
-    }
-
-    // A full tile is fetched with one uniform base address plus the per-thread byte offsets (no
-    // vector address arithmetic inside the key loop).  In the ragged last tile, rows at or beyond
-    // L are read from row L - 1 instead of being predicated off (a predicated load into a zeroed
-    // register makes every load wait for the one before it).  Such keys are masked to -inf before
-    // the softmax, and a probability of exactly zero times a finite V row contributes nothing.
-    __device__ __forceinline__ void load(u32x4 (&reg)[NP], const _Float16* base, int64_t stride_l,
-                                         int key0, int L, int tid) const {
-        if (key0 >= L) return;
-        if (key0 + BK <= L) {
-            const char* tile = reinterpret_cast<const char*>(base + (int64_t)key0 * stride_l);
-#pragma unroll
-            for (int i = 0; i < NP; ++i) reg[i] = *reinterpret_cast<const u32x4*>(tile + goff[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const int idx = EXACT ? tid + i * NT : min(tid + i * NT, NCHUNK - 1);
-                const int key = min(key0 + idx / CPR, L - 1);
-                reg[i] = *reinterpret_cast<const u32x4*>(base + (int64_t)key * stride_l + (idx % CPR) * 8);
-            }
-        }
-    }
-    template <int STR>
-    static __device__ __forceinline__ void store(const u32x4 (&reg)[NP], _Float16* dst, int tid) {
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int idx = tid + i * NT;
-            if (EXACT || idx < NCHUNK)
-                *reinterpret_cast<u32x4*>(dst + (idx / CPR) * STR + (idx % CPR) * 8) = reg[i];
-        }
-    }
-    __device__ __forceinline__ void load_k(const _Float16* kbase, int64_t sl, int key0, int L, int tid) {
-        load(kreg, kbase, sl, key0, L, tid);
-    }
-    __device__ __forceinline__ void load_v(const _Float16* vbase, int64_t sl, int key0, int L, int tid) {
-        load(vreg, vbase, sl, key0, L, tid);
-    }
-    __device__ __forceinline__ void store_k(_Float16* ks, int tid) const { store<G::KSTR>(kreg, ks, tid); }
-    __device__ __forceinline__ void store_v(_Float16* vs, int tid) const { store<G::VSTR>(vreg, vs, tid); }
-};
-
-// Largest partial row sum (16 terms) the fast path of the online softmax accepts.
-constexpr float kTrip = 16384.f;
+// The eight 16-bit values of `v` moved down by n places (n >= 8: nothing of interest is left).
+__device__ __forceinline__ u32x4 drop_halves(u32x4 v, uint32_t n) {
+    if (n & 4) v = u32x4{v[2], v[3], 0u, 0u};
+    if (n & 2) v = u32x4{v[1], v[2], v[3], 0u};
+    if (n & 1) v = u32x4{(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
+    return v;
+}
 
 // Bias (log2 units) of the reference the exponentials are taken against, in every kernel
 // (FwdParams::bias), and the largest sum of a query's 32 probabilities of one sub-tile that the
@@ -209,9 +133,8 @@ constexpr float kTrip = 16384.f;
 // maximum is lost: a tail of L small weights loses at most L 2^-(24 - bias) of the row.  The
 // launcher picks bias = 11 - ceil(log2 L), between kBiasMin and kBiasMax, which keeps that share
 // at or below 2^-13 = 1.2e-4 whatever the sequence length; what is left of the fp16 range is the
-// leash of the speculative reference, which may lag the true maximum by 15 + bias log2 units (14
-// in the four-wave kernels, whose check works on half rows) before the check sends the wave down
-// the slow path: 14 units at L = 4096, 12 at 16384, 10 at 65536.
+// leash of the speculative reference, which may lag the true maximum by 15 + bias log2 units before
+// the check sends the wave down the slow path: 14 units at L = 4096, 12 at 16384, 10 at 65536.
 constexpr float kBiasMin = -8.0f;
 constexpr float kBiasMax = 6.0f;
 constexpr float kTripSum = 32768.f;
@@ -234,23 +157,6 @@ __device__ __forceinline__ void scale_accumulators(floatx16 (&o)[DB][NQB], int n
     }
 }
 
-// LDS address of this lane's K row for sub-tile `sub` of a tile: A operand of S^T = K_sub * Q^T.
-template <int H>
-__device__ __forceinline__ const _Float16* k_operand_ptr(const _Float16* ks, int sub, int lane) {
-    return ks + (sub * 32 + (lane & 31)) * Geometry<H>::KSTR + 8 * (lane >> 5);
-}
-
-// LDS address this lane hands to the transpose reads of sub-tile `sub`.  Inside each group of 16
-// lanes, lane j receives, for i = 0..3, element (j % 4) of the 8-byte row fetched by lane
-// 4 i + j / 4.  With lane s of a group pointing at V[key0 + s / 4][d0 + 4 (s % 4) ...], lane j ends
-// up with V[key0 + i][d0 + j], i = 0..3: four consecutive keys of one head-dim column.
-template <int H>
-__device__ __forceinline__ const _Float16* v_operand_ptr(const _Float16* vs, int sub, int lane) {
-    const int s16 = lane & 15;
-    return vs + (sub * 32 + 4 * (lane >> 5) + (s16 >> 2)) * Geometry<H>::VSTR + 16 * ((lane >> 4) & 1) +
-           4 * (s16 & 3);
-}
-
 // Ring tiles of the ping-pong kernel are chunk-major: a 64-key tile of H columns is stored as H / 8
 // columns of 64 rows x 16 bytes, column c at c * kColStride halves.  One direct-to-LDS load of a
 // wave (64 lanes x 16 bytes, contiguous in LDS) fills one column, lane = key row.  The 64-byte pad
@@ -266,8 +172,9 @@ __device__ __forceinline__ const _Float16* k_ring_ptr(const _Float16* ks, int su
     return ks + (lane >> 5) * kColStride + (sub * 32 + (lane & 31)) * 8;
 }
 
-// Per-lane part of the transpose-read address in a ring tile (see v_operand_ptr for which element
-// ends up where): lane s of a 16-lane group points at row key0 + s / 4, halves 4 (s % 4) ... of the
+// Per-lane part of the transpose-read address in a ring tile.  Inside each group of 16 lanes, lane j
+// receives, for i = 0..3, element (j % 4) of the 8-byte row fetched by lane 4 i + j / 4: four consecutive
+// keys of one head-dim column.  Lane s of a 16-lane group points at row key0 + s / 4, halves 4 (s % 4) ... of the
 // 32-byte span that starts at column 2 * ((lane / 16) % 2); head-dim block db adds 4 db columns.
 __device__ __forceinline__ const _Float16* v_ring_ptr(const _Float16* vs, int sub, int lane) {
     const int s16 = lane & 15;
@@ -287,6 +194,43 @@ constexpr int kMaskSubStr = 40;
 template <int H, int NW, int NQB>
 constexpr int lds_bytes_pingpong_masked() {
     return lds_bytes_pingpong<H, NQB>() + NW * 32 * NQB * kMaskSubStr * (int)sizeof(_Float16);
+}
+
+// Key-split kernel: LDS of one wave (slabs of the 32 keys it works on and their mask values; at the end
+// its share of 16 rows of O in float32, rows padded by 16 bytes against bank conflicts), and of a
+// workgroup (plus m and l of every row).
+constexpr int kSplitMaxWaves = 4;
+constexpr int kRawBuffer = 0x00027000;     // word 3 of a raw buffer resource: no stride, no swizzle, 32-bit data format
+template <int H>
+constexpr int split_row_floats() { return H + 4; }
+template <int H, bool MASK>
+constexpr int split_wave_bytes() {
+    constexpr int part = 16 * split_row_floats<H>() * 4, slabs = 2 * 32 * H * 2 + (MASK ? 1024 : 0);
+    return part > slabs ? part : slabs;
+}
+template <int H, bool MASK>
+constexpr int split_lds_bytes(int waves) { return waves * (split_wave_bytes<H, MASK>() + 16 * 8); }
+
+// Group kernel: sub-tiles of 32 keys per key group and key tile (two where one group would otherwise pass a
+// barrier per sub-tile: +2 %), and ring slots (two where three would cost a resident workgroup).
+template <int H, int GK>
+constexpr int group_sub() { return GK == 1 && H <= 64 ? 2 : 1; }
+template <int H, int GK>
+constexpr int group_slots() { return H == 128 && GK >= 2 ? 2 : 3; }
+template <int H, int GK>
+constexpr int group_ring_bytes() { return group_slots<H, GK>() * GK * group_sub<H, GK>() * 2 * 32 * H * 2; }
+// LDS: the ring of key tiles and the mask slabs, later the rows of O on their way out or, with several key
+// groups, the waves' shares of O (whichever is larger), and behind them m and l of every row.
+template <int H, int NQ, int GK, bool MASK>
+constexpr int group_stat_offset() {
+    constexpr int ring = group_ring_bytes<H, GK>() + (MASK ? 8 * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 * 16 * NQ * split_row_floats<H>() * 4;
+    return ring > part ? ring : part;
+}
+template <int H, int NQ, int GK, bool MASK>
+constexpr int group_lds_bytes() { return group_stat_offset<H, NQ, GK, MASK>() + (GK == 1 ? 0 : 8 * 16 * NQ * 8); }
+// (written in assembly so that the compiler does not see an LDS write, see RingLoader)
+__device__ __forceinline__ void group_dma16(uint32_t lds_addr, const _Float16* base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
 }
 
 // Barrier between the phases of the ping-pong kernel.  It does not wait for the wave's own LDS
@@ -352,7 +296,9 @@ __device__ __forceinline__ void wait_ring_loads() { asm volatile("s_waitcnt vmcn
 // _Float16 pointers for address arithmetic); only the few operations that interpret them differ.
 #define FA_ELEM_BF16 0
 #include "fused_attn_kernel_impl.inc"
+#include "fused_attn_split.inc"
 #undef FA_ELEM_BF16
 #define FA_ELEM_BF16 1
 #include "fused_attn_kernel_impl.inc"
+#include "fused_attn_split.inc"
 #undef FA_ELEM_BF16

@@ -139,6 +139,33 @@ def test_every_launch_plan_covers_every_query_tile_once():
     assert paired_masks > 10   # ... and masked launches in pairs of tiles
 
 
+def test_every_variant_covers_every_query_row_once():
+    """The kernels that take what the tile kernels do not: rows of a workgroup times workgroups per head
+    reach the end of the sequence and no further than its last workgroup, and the grid holds them all."""
+    import random
+
+    rng = random.Random(11)
+    kinds = set()
+    for _ in range(1500):
+        H, R, L = rng.choice([16, 32, 64, 128]), rng.randint(1, 64), int(2 ** rng.uniform(0, 14))
+        B, mode = rng.randint(1, 32), rng.choice(["plain", "causal", "mask"])
+        v = capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
+        if v["kernel"] == "tile":
+            plan = capi.launch_plan(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
+            assert plan["waves"] == 8 and (v["working"], v["rows"]) == (plan["working"], 8 * plan["rows_per_wave"])
+            assert plan["rows_per_wave"] == (32 if H == 128 else 64)        # the shapes that have a kernel
+        else:
+            assert v["rows"] in ((16,) if v["kernel"] == "split" else (64, 128, 256))
+            assert (v["per_head"] - 1) * v["rows"] < L <= v["per_head"] * v["rows"]
+            assert v["working"] == B * R * v["per_head"] and v["waves"] in ((2, 4) if v["kernel"] == "split" else (8,))
+        assert v["workgroups"] % 8 == 0 and 0 <= v["workgroups"] - v["working"] < 8
+        kinds.add((v["kernel"], v["rows"], v["waves"]))
+    assert {("split", 16, 2), ("split", 16, 4), ("group", 64, 8), ("group", 128, 8), ("group", 256, 8)} <= kinds
+    assert {k for k, _, _ in kinds} == {"split", "group", "tile"}
+    with pytest.raises(capi.FusedAttnError):
+        capi.launch_variant(1, 1, 64, 48)
+
+
 def _tiles_of_projection_plan(plan):
     """Replays how qkv_proj_kernel (qkv_proj_kernel.hpp) turns a workgroup index into output tiles
     (row tile, feature tile)."""

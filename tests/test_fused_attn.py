@@ -1015,6 +1015,63 @@ def test_additive_mask_on_large_grids(gpu, B, R, L, H):
         assert err[keep[b]].max().item() <= TOL, (b, h)
 
 
+@pytest.mark.parametrize("L", [8, 9, 31, 33, 129, 250, 381, 1021, 1026])
+@pytest.mark.parametrize("H", [16, 64, 128])
+def test_mask_rows_at_any_alignment(gpu, L, H):
+    # Rows of 2 L bytes start wherever L puts them; the chunk behind the last row of the tensor is the
+    # one with nothing to read past it, so the last rows of the last batch are compared as well.
+    R = max(2, 64 * 256 // (64 * L) * 8) if L < 200 else 40
+    B = 2
+    q, k, v = (_rand((B, L, R * H), 5100 + L + i) for i in range(3))
+    g = torch.Generator().manual_seed(5105 + L)
+    mask = torch.randn(B, L, L, generator=g).to(torch.float16)
+    mask[:, :, L - L // 3:] = float("-inf")
+    mask[:, L - 1, L - 1] = 2.0                 # the last value of the tensor takes part
+    got = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu))
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        want = attention(q[b:b + 1, :, sl], k[b:b + 1, :, sl], v[b:b + 1, :, sl], H, mask=mask[b:b + 1].float())
+        assert _max_err(got[b, :, sl], want[0]) <= TOL, (b, h)
+
+
+# One shape or two per kernel and head_dim, at the edges of their tiles: 16, 64, 128 and 256 query rows, 32 keys
+# per sub-tile, 64 keys per key tile and three key tiles per turn of the ring.
+SMALL_GRIDS = [(1, 1, 1), (2, 3, 17), (1, 5, 33), (2, 4, 129), (1, 3, 300), (3, 40, 130), (2, 40, 255), (2, 16, 513),
+               (8, 40, 129), (2, 12, 1217), (9, 20, 705)]
+
+
+@pytest.mark.parametrize("H", [16, 32, 64, 128])
+@pytest.mark.parametrize("B,R,L", SMALL_GRIDS)
+@pytest.mark.parametrize("mode", ["plain", "causal", "mask"])
+def test_split_and_group_kernels(gpu, B, R, L, H, mode):
+    variant = capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
+    bf16 = (L + H // 16 + len(mode)) % 2 == 1            # either type at every length
+    dtype = torch.bfloat16 if bf16 else torch.float16
+    for std in (1.0, 3.0):                                # 3: the reference of the exponentials moves often
+        q, k, v = (_rand((B, L, R * H), 6100 + L + i, std if i < 2 else 1.0).to(dtype) for i in range(3))
+        mask = None
+        if mode == "mask":
+            g = torch.Generator().manual_seed(6105 + L)
+            mask = torch.randn(B, L, L, generator=g)
+            mask[:, :, L - L // 3:] = float("-inf")       # whole sub-tiles muted behind a mixed one
+            mask[:, L - 1, L - 1] = 1.0
+            mask = mask.to(dtype)
+        got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu) if mask is not None else None,
+                                causal=mode == "causal", return_lse=True)
+        full = mask.float() if mask is not None else causal_mask(B, L).float() if mode == "causal" else None
+        for b, h in {(0, 0), (B - 1, R - 1), (B // 2, R // 3)}:
+            sl = slice(h * H, (h + 1) * H)
+            args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+            one = full[b:b + 1] if full is not None else None
+            err = _max_err(got[b, :, sl], attention(*args, mask=one)[0])
+            assert err <= (2e-2 if bf16 else TOL), (variant, std, b, h, err)
+            # the log-sum-exp is taken over the rounded probabilities: at worst, all of a row's weight on one
+            # key, their sum is off by one rounding: half of bf16's last place (2^-7) or all of fp16's (2^-10, toward zero)
+            want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
+            off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
+            assert off.max().item() <= (2.0 ** -8 if bf16 else 2.0 ** -10) * 1.01 + 1e-5, (variant, std, b, h)
+
+
 def _block_mask(kind, B, L, seed):
     """Masks under the reference's contract (zero where a pair takes part, -inf where it is muted,
     reference README.md:88-89), made of large all-zero and all-muted blocks: what the kernels'

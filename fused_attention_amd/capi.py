@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(_PKG_DIR, "libfused_attn_gfx950.so")
 
 # every symbol include/fused_attn.h declares
 EXPORTS = ("fa_fwd", "fa_fwd_ex", "fa_fwd_strided", "fa_fwd_plan", "fa_fwd_variant", "fa_fwd_query", "fa_fwd_reference_bias", "fa_strerror",
-           "fa_fwd_timed", "fa_fwd_timed_ex", "fa_qkv_proj", "fa_qkv_proj_plan")
+           "fa_fwd_timed", "fa_fwd_timed_ex", "fa_qkv_proj", "fa_qkv_proj_plan", "fa_qkv_proj_variant")
 FLAG_CAUSAL = 1
 FLAG_BF16 = 2
 
@@ -56,6 +56,8 @@ def load_library():
     lib.fa_qkv_proj.restype = ctypes.c_int
     lib.fa_qkv_proj_plan.argtypes = [i64, i64, i64, i64, i64, ctypes.POINTER(ctypes.c_int)]
     lib.fa_qkv_proj_plan.restype = ctypes.c_int
+    lib.fa_qkv_proj_variant.argtypes = lib.fa_qkv_proj_plan.argtypes
+    lib.fa_qkv_proj_variant.restype = ctypes.c_int
     lib.fa_fwd_plan.argtypes = [i64, i64, i64, i64, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     lib.fa_fwd_plan.restype = ctypes.c_int
     lib.fa_fwd_variant.argtypes = lib.fa_fwd_plan.argtypes
@@ -103,6 +105,13 @@ def projection_plan(B, L, F_in, R, H):
     _check(load_library().fa_qkv_proj_plan(B, L, F_in, R, H, out))
     keys = ("workgroups", "working", "tiles", "tiles_n")
     return dict(zip(keys, out))
+
+
+def projection_variant(B, L, F_in, R, H):
+    """What fa_qkv_proj_variant reports for a problem, as a dict.  Needs no GPU."""
+    out = (ctypes.c_int * 6)()
+    _check(load_library().fa_qkv_proj_variant(B, L, F_in, R, H, out))
+    return dict(zip(("tile_m", "tile_n", "workgroups", "working", "tiles", "tiles_n"), out))
 
 
 def fwd_raw(q_ptr, k_ptr, v_ptr, mask_ptr, out_ptr, B, R, L, H, stride_b, stride_h, stride_l,

@@ -457,5 +457,374 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Small-tile kernel: outputs that 256 x 256 tiles do not spread over the chip.
+//
+// Eight waves as KG contraction groups of WM x WN waves; a wave owns 16 MT rows x 16 NT features, a group the whole
+// (16 MT WM) x (16 NT WN) tile, and with KG = 2 each group takes one 32-wide half of every slice: the
+// wave tiles, and with them the products per byte read from LDS, are then twice as large as with eight waves
+// side by side.  Slices of 64 in a ring of SLOTS slots, one barrier per slice, one tile per workgroup.  The
+// slot layouts, the transposed product and the epilogue are those of the kernel above; w slots of 64
+// features have half as many chunks per row, and the row's lowest bit selects the half of the banks itself.
+//
+// What bounds it: a 256 x 256 tile takes 1.3 to 1.5 us per slice of one compute unit, however many of them have
+// one; a 128 x 256 tile takes 0.65 us, a 128 x 128 one 0.45, 64 x 128 (two per unit) 0.35 and 64 x 64 0.25, a
+// mix of the 32 to 58 bytes per clock the direct loads deliver, the products and the barrier.  Same box,
+// 256 x 256 tiles before, the shape that is picked now: M 512 N 15360 K 5120 113 -> 66 us, M 64 N 7680
+// K 5120 101 -> 23, M 256 N 7680 K 2560 62 -> 18, M 2048 N 3072 K 1024 35 -> 20, M 128 N 1536 K 1024
+// 30 -> 6.1 (geometric mean over 220 random shapes: 1.95x).  Rings of eight and six slots for the two
+// smallest shapes, one workgroup per unit, were up to 1.9 times slower than two workgroups with short rings.
+//
+// The 16-feature blocks of a head are walked in an order that puts the two halves of a rotary pair next to
+// each other (0, HR/32, 1, HR/32 + 1, ...): a wave with any even number of blocks has whole pairs, and a tile
+// of 64 features may be half a head.
+template <int MT, int NT, int WM, int WN, int KG, int SLOTS>
+struct SmallTile {
+    static_assert(WM * WN * KG == kWaves && (KG == 1 || (KG == 2 && MT % 2 == 0)) && NT % 2 == 0);
+    static constexpr int TM = 16 * MT * WM, TN = 16 * NT * WN;
+    static constexpr int XSLOT = TM * kTileK, WSLOT = kTileK * TN;       // halves
+    static constexpr int LX = TM / 64, LW = TN / 64;                     // loads per wave and slice
+    static constexpr int RING = SLOTS * (XSLOT + WSLOT) * 2;             // bytes
+    static constexpr int OWN = MT / KG;                                  // 16-row blocks a wave finishes
+    static constexpr int PART = KG == 1 ? 0 : kWaves * OWN * NT * 1024;  // accumulators handed over
+    static constexpr int STAGE = kWaves * 16 * 16 * NT * 2;
+    static constexpr int LDS = RING > PART + STAGE ? RING : PART + STAGE;
+    static_assert(LDS <= 160 * 1024);
+};
+
+template <class F, int... J>
+__device__ __forceinline__ void for_each_index(F f, std::integer_sequence<int, J...>) { (f(I<J>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void for_each_index(F f) { for_each_index(f, std::make_integer_sequence<int, N>{}); }
+
+// Waits until at most min(left, MOST) slices of LOADS loads each are still under way.
+template <int LOADS, int MOST>
+__device__ __forceinline__ void wait_slices(int left) {
+    if constexpr (MOST > 0) {
+        if (left < MOST) return wait_slices<LOADS, MOST - 1>(left);
+    }
+    wait_loads<LOADS * MOST>();
+}
+
+template <int HR, bool BF, int MT, int NT, int WM, int WN, int KG, int SLOTS>
+__global__ __launch_bounds__(kWaves * 64, MT * NT < 16 ? 4 : 2) void qkv_proj_small_kernel(const Params p) {
+    using T = SmallTile<MT, NT, WM, WN, KG, SLOTS>;
+    constexpr int TM = T::TM, TN = T::TN, LX = T::LX, LW = T::LW;
+    constexpr int CPRX = kTileK / 8, CPRW = TN / 8;       // 16-byte chunks per row of a slot
+    extern __shared__ __attribute__((aligned(16))) _Float16 smem[];
+    typedef short short8v __attribute__((ext_vector_type(8)));
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15;
+    const int g4 = lane >> 4;
+    const int kg = wave / (WM * WN);
+    const int wm = wave % (WM * WN) / WN;
+    const int wn = wave % WN;
+
+    const int wg = blockIdx.x;
+    const int logical = (wg % kNumXcd) * p.wgs_per_xcd + wg / kNumXcd;
+    if (logical >= p.total_wgs) return;
+    // bands of 1024 rows, feature tile by feature tile inside a band, as above
+    constexpr int BAND = kBand * kTileM / TM;
+    const int band = logical / (BAND * p.tiles_n);
+    const int in_band = logical - band * (BAND * p.tiles_n);
+    const int band_rows = min(BAND, p.total_tiles / p.tiles_n - band * BAND);
+    const int m0 = (band * BAND + in_band % band_rows) * TM;
+    const int n0 = (in_band / band_rows) * TN;
+
+    // first feature of the block at place b of the order described above
+    auto feature_of = [](int b) __attribute__((always_inline)) {
+        if constexpr (HR >= 64) {
+            constexpr int HB = HR / 16;
+            return 16 * (b / HB * HB + (b % HB >> 1) + (b & 1) * (HB / 2));
+        }
+        return 16 * b;
+    };
+    // place of chunk c of contraction row k in a w slot, less c
+    auto w_swizzle = [](int k) __attribute__((always_inline)) {
+        return CPRW >= 16 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (k & 2) << 1 | (((k >> 3) & 1) << 1);
+    };
+
+    // What the end of the tile needs from memory, a run's bias and the distinct runs of the tables for every row,
+    // is requested in one go and waits in registers: requested where it is used, one load behind the
+    // other, it made the end of a 128 x 256 tile take 10 us, as long as a dozen slices.
+    constexpr int OWN = T::OWN;
+    constexpr int RUNS = HR == 0 ? 0 : HR <= 32 ? 1 : NT / 2;
+    const int b0 = n0 / 16 + wn * NT;
+    u16x4 bias4[NT];
+    floatx4 cos4[OWN][RUNS > 0 ? RUNS : 1], sin4[OWN][RUNS > 0 ? RUNS : 1];
+    auto request = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int n = feature_of(b0 + nt) + 4 * g4;
+            bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
+        }
+        if constexpr (HR > 0) {
+            const int at = m0 % p.L + 16 * (wm * MT + kg * OWN) + c16;
+#pragma unroll
+            for (int mt = 0; mt < OWN; ++mt) {
+                // (rows beyond M: any row of the tables)
+                int pos = at + 16 * mt;
+                if (p.L < TM)
+                    pos %= p.L;
+                else
+                    pos -= pos >= p.L ? p.L : 0;
+#pragma unroll
+                for (int i = 0; i < RUNS; ++i) {
+                    const int64_t e = (int64_t)pos * (HR / 2) + (feature_of(b0 + 2 * i) + 4 * g4) % (HR / 2);
+                    cos4[mt][i] = *reinterpret_cast<const floatx4*>(p.rope_cos + e);
+                    sin4[mt][i] = *reinterpret_cast<const floatx4*>(p.rope_sin + e);
+                }
+            }
+        }
+    };
+    uint32_t xvo[LX], wvo[LW];
+#pragma unroll
+    for (int i = 0; i < LX; ++i) {
+        const int pos = (wave * LX + i) * 64 + lane;
+        const int row = pos / CPRX;
+        const int c = (pos % CPRX) ^ ((row >> 1) & 7);
+        const int grow = min(m0 + row, p.M - 1) - m0;       // rows beyond M: never stored
+        xvo[i] = ((uint32_t)grow * (uint32_t)p.K + (uint32_t)c * 8u) * 2u;
+    }
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int pos = (wave * LW + i) * 64 + lane;
+        const int krow = pos / CPRW;
+        const int c = (pos % CPRW) ^ w_swizzle(krow);
+        int n = feature_of(n0 / 16 + (c >> 1)) + 8 * (c & 1);
+        if (n >= p.N) n = 0;                                // features beyond N: never stored
+        wvo[i] = ((uint32_t)krow * (uint32_t)p.N + (uint32_t)n) * 2u;
+    }
+    const char* xsrc = reinterpret_cast<const char*>(p.x + (int64_t)m0 * p.K);
+    const char* wsrc = reinterpret_cast<const char*>(p.w);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(FA_LDS void*)smem;
+    const uint32_t xs_lds = lds0 + (uint32_t)(wave * LX) * 1024u;
+    const uint32_t ws_lds = lds0 + (uint32_t)(SLOTS * T::XSLOT * 2 + wave * LW * 1024);
+    constexpr int LOADS = LX + LW;
+    auto issue_one = [&](int slot, auto i_c) __attribute__((always_inline)) {
+        constexpr int J = decltype(i_c)::value;
+        if constexpr (J < LX)
+            dma16(xs_lds + (uint32_t)(slot * T::XSLOT * 2 + J * 1024), xsrc, xvo[J]);
+        else
+            dma16(ws_lds + (uint32_t)(slot * T::WSLOT * 2 + (J - LX) * 1024), wsrc, wvo[J - LX]);
+        if constexpr (J == LOADS - 1) {
+            xsrc += kTileK * 2;
+            wsrc += (int64_t)kTileK * p.N * 2;
+        }
+    };
+    // loads FIRST ... END - 1 of a slice
+    auto issue = [&](int slot, auto first_c, auto end_c) __attribute__((always_inline)) {
+        constexpr int FIRST = decltype(first_c)::value;
+        constexpr int COUNT = decltype(end_c)::value - FIRST;
+        for_each_index<COUNT>([&](auto j_c) __attribute__((always_inline)) { issue_one(slot, I<FIRST + decltype(j_c)::value>{}); });
+    };
+    const int ksteps = p.K / kTileK;
+    constexpr bool PIPE = KG == 1;
+    for (int u = 0; u < min(PIPE ? SLOTS : SLOTS - 1, ksteps); ++u) issue(u, I<0>{}, I<LOADS>{});
+
+    // acc[nt][mt][r]: row 16 (wm MT + mt) + c16 of the tile, feature 4 g4 + r of block wn NT + nt
+    floatx4 acc[NT][MT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    constexpr int NSUB = 2 / KG;       // 32-wide halves of a slice per group
+    int xrd[NSUB];
+#pragma unroll
+    for (int s = 0; s < NSUB; ++s)
+        xrd[s] = ((wm * MT * 16 + c16) * CPRX + ((4 * (s + kg) + g4) ^ ((c16 >> 1) & 7))) * 8;
+    const int krow = 8 * g4 + (c16 >> 2);
+    const int wrd0 = SLOTS * T::XSLOT + (32 * kg + krow) * TN + ((wn * 2 * NT + ((c16 & 3) >> 1)) ^ w_swizzle(krow)) * 8 + 4 * (c16 & 1);
+
+    // Operands of a half slice.  Where a wave multiplies both halves, in two sets: those of the next half are
+    // requested before the matrix instructions of this one.
+    half8 xop[PIPE ? 2 : 1][MT], wop[PIPE ? 2 : 1][NT];
+    auto load = [&](auto set_c, int slot, auto s_c) __attribute__((always_inline)) {
+        constexpr int SET = decltype(set_c)::value;
+        constexpr int S = decltype(s_c)::value;
+        const _Float16* const xb = smem + slot * T::XSLOT;
+        const _Float16* const wb = smem + slot * T::WSLOT;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) xop[SET][mt] = *reinterpret_cast<const half8*>(xb + xrd[S] + mt * 16 * kTileK);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const _Float16* const at = wb + (wrd0 ^ (16 * nt)) + 32 * S * TN;
+            const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FA_LDS short4v*)(at));
+            const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FA_LDS short4v*)(at + 4 * TN));
+            const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            wop[SET][nt] = __builtin_bit_cast(half8, both);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // The loads into a slot go out one by one between the matrix instructions of a whole slice: a wave that
+    // issues them all at once waits at the issue port while the queue drains, its matrix core idle.
+    // HALF: 0 behind a barrier, 1 before the next one (if there is anything between).
+    constexpr int GROUPS = NSUB * NT;
+    auto multiply = [&](auto set_c, auto half_c, bool filling, auto fill_slot) __attribute__((always_inline)) {
+        constexpr int SET = decltype(set_c)::value;
+        constexpr int HALF = decltype(half_c)::value;
+        auto group = [&](auto nt_c) __attribute__((always_inline)) {
+            constexpr int nt = decltype(nt_c)::value;
+            constexpr int GROUP = HALF * NT + nt;
+            constexpr int FIRST = GROUP * LOADS / GROUPS, END = (GROUP + 1) * LOADS / GROUPS;
+            if constexpr (END > FIRST) {
+                if (filling) issue(fill_slot, I<FIRST>{}, I<END>{});
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                if constexpr (BF)
+                    acc[nt][mt] = bf16::mfma16(wop[SET][nt], xop[SET][mt], acc[nt][mt]);
+                else
+                    acc[nt][mt] = mfma16(wop[SET][nt], xop[SET][mt], acc[nt][mt]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for_each_index<NT>(group);
+    };
+
+    // Rounds of the ring in which every load has a slice to fetch, with the slots known at compile time and no
+    // decision in them (a wave issues an instruction every four or five clocks at best, and addresses and
+    // branches took as long as the products), the rest one by one.  No more copies of a slice than
+    // that: a short launch waits for its instructions, too.
+    // step(slots of slices u, u + 1 and u - 1, whether slices u - 1 + AHEAD and u + AHEAD exist, slices behind the
+    // one awaited)
+    auto ring = [&](auto step) __attribute__((always_inline)) {
+        constexpr int AHEAD = PIPE ? SLOTS : SLOTS - 1;        // the loads of slice u + AHEAD follow the barrier of slice u
+        int u = 0;
+        for (; u + SLOTS + AHEAD <= ksteps; u += SLOTS)
+            for_each_index<SLOTS>([&](auto s_c) __attribute__((always_inline)) {
+                constexpr int S = decltype(s_c)::value;
+                step(s_c, I<(S + 1) % SLOTS>{}, I<(S + SLOTS - 1) % SLOTS>{}, S > 0 || u > 0, true, SLOTS);
+            });
+        for (int slot = 0; u < ksteps; ++u) {
+            const int next = slot + 1 == SLOTS ? 0 : slot + 1, before = slot == 0 ? SLOTS - 1 : slot - 1;
+            step(slot, next, before, u > 0 && u - 1 + AHEAD < ksteps, u + AHEAD < ksteps, ksteps - (PIPE ? 2 : 1) - u);
+            slot = next;
+        }
+    };
+    if constexpr (PIPE) {
+        wait_slices<LOADS, SLOTS - 1>(ksteps - 1);
+        ring_barrier();
+        load(I<0>{}, I<0>{}, I<0>{});
+        ring([&](auto slot, auto next, auto before, bool late, bool filling, int left) __attribute__((always_inline)) {
+            load(I<1>{}, slot, I<1>{});
+            multiply(I<0>{}, I<1>{}, late, before);
+            // The operands of the slice's second half are in registers and this wave's loads of the next slice have
+            // landed; behind the barrier that holds for everybody: the next slice may be read, and this
+            // one's slot filled.
+            wait_slices<LOADS, SLOTS - 2>(left);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            ring_barrier();
+            // (behind the last slice: a slot that nobody uses any more, into registers that nobody uses)
+            load(I<0>{}, next, I<0>{});
+            multiply(I<1>{}, I<0>{}, filling, slot);
+        });
+    } else {
+        ring([&](auto slot, auto, auto before, bool, bool filling, int left) __attribute__((always_inline)) {
+            // This wave's loads of the slice have landed; behind the barrier everybody's have, and the slice before
+            // has been read by all: its slot may be filled.
+            wait_slices<LOADS, SLOTS - 2>(left);
+            ring_barrier();
+            load(I<0>{}, slot, I<0>{});
+            multiply(I<0>{}, I<0>{}, filling, before);
+            // (the reads of the slice have all returned: their results went into matrix instructions)
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        });
+    }
+    request();
+    __syncthreads();       // the ring is idle from here on
+
+    // two groups: each finishes half of its rows and hands the sums of the other half over
+    floatx4 own[NT][OWN];
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < OWN; ++mt) own[nt][mt] = acc[nt][mt];
+    } else {
+        float* const part = reinterpret_cast<float*>(smem) + lane * 4;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < OWN; ++mt) {
+                *reinterpret_cast<floatx4*>(part + ((wave * OWN + mt) * NT + nt) * 256) = kg == 0 ? acc[nt][mt + OWN] : acc[nt][mt];
+                own[nt][mt] = kg == 0 ? acc[nt][mt] : acc[nt][mt + OWN];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < OWN; ++mt)
+                own[nt][mt] += *reinterpret_cast<const floatx4*>(part + (((wave ^ (WM * WN)) * OWN + mt) * NT + nt) * 256);
+    }
+
+    // bias, rotation, one rounding; whole rows leave through a private LDS tile of 16 rows (see above)
+    _Float16* const stage = smem + T::PART / 2 + wave * (256 * NT);
+    auto biased = [&](int nt, int mt) __attribute__((always_inline)) {
+        floatx4 v = own[nt][mt];
+        if (p.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
+        }
+        return v;
+    };
+    auto store_run = [&](floatx4 v, int nt) __attribute__((always_inline)) {
+        u16x4 hv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hv[e] = BF ? bf16::float_to_elem(v[e]) : float_to_elem(v[e]);
+        *reinterpret_cast<u32x2*>(stage + c16 * (16 * NT) + ((2 * nt + (g4 >> 1)) ^ (c16 & (2 * NT - 1))) * 8 + 4 * (g4 & 1)) = __builtin_bit_cast(u32x2, hv);
+    };
+#pragma unroll
+    for (int mt = 0; mt < OWN; ++mt) {
+        const int mb = m0 + 16 * (wm * MT + kg * OWN + mt);
+        if constexpr (HR >= 32) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt += 2) {
+                floatx4 a = biased(nt, mt);
+                floatx4 b = biased(nt + 1, mt);
+                if (feature_of(b0 + nt) < 2 * p.F) {
+                    const floatx4 c4 = cos4[mt][nt / 2 % RUNS], s4 = sin4[mt][nt / 2 % RUNS];
+                    const floatx4 ra = a * c4 - b * s4;
+                    const floatx4 rb = b * c4 + a * s4;
+                    a = ra;
+                    b = rb;
+                }
+                store_run(a, nt);
+                store_run(b, nt + 1);
+            }
+        } else {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                floatx4 a = biased(nt, mt);
+                if constexpr (HR == 16) {
+                    // a head is one block and the partner of a run sits 32 lanes away
+                    floatx4 b;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float ae = a[e];
+                        b[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, ae)));
+                    }
+                    if (16 * (b0 + nt) < 2 * p.F) a = g4 < 2 ? a * cos4[mt][0] - b * sin4[mt][0] : a * cos4[mt][0] + b * sin4[mt][0];
+                }
+                store_run(a, nt);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NT / 2; ++i) {
+            const int r = i * (32 / NT) + lane / (2 * NT), ch = lane % (2 * NT);
+            const u32x4 w = *reinterpret_cast<const u32x4*>(stage + r * (16 * NT) + (ch ^ (r & (2 * NT - 1))) * 8);
+            const int n = feature_of(b0 + (ch >> 1)) + 8 * (ch & 1);
+            if (mb + r < p.M && n < p.N)
+                __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p.out + (int64_t)(mb + r) * p.N + n));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+}
+
 }  // namespace qkv
 }  // namespace fa

@@ -204,6 +204,34 @@ def test_every_projection_plan_covers_every_output_tile_once():
         capi.projection_plan(1, 64, 100, 1, 64)          # contraction length not a multiple of 64
 
 
+def test_every_projection_variant_covers_every_output_tile_once():
+    """The grid of the kernel that fa_qkv_proj picks: every tile of its shape exactly once."""
+    seen = set()
+    for B, L, F_in, R, H in [(1, 1, 64, 4, 16), (1, 300, 640, 20, 64), (3, 333, 512, 12, 32), (1, 777, 704, 20, 64),
+                             (3, 1111, 320, 24, 32), (1, 1025, 1024, 16, 128), (1, 7000, 512, 20, 64), (4, 4096, 1024, 16, 64),
+                             (2, 5000, 64, 8, 128), (1, 512, 5120, 40, 128), (1, 64, 5120, 40, 128)]:
+        v = capi.projection_variant(B, L, F_in, R, H)
+        seen.add((v["tile_m"], v["tile_n"]))
+        tiles_m = -(-B * L // v["tile_m"])
+        assert v["tiles_n"] == -(-3 * R * H // v["tile_n"]) and v["tiles"] == tiles_m * v["tiles_n"]
+        assert v["working"] == (min(v["tiles"], 256) if v["tile_m"] == 256 else v["tiles"])
+        per_xcd, band_of = v["workgroups"] // 8, 1024 // v["tile_m"]
+        tiles = []
+        for wg in range(v["workgroups"]):
+            logical = (wg % 8) * per_xcd + wg // 8
+            if logical >= v["working"]:
+                continue
+            for tile in range(logical, v["tiles"], v["working"]):
+                band, in_band = divmod(tile, band_of * v["tiles_n"])
+                band_rows = min(band_of, tiles_m - band * band_of)
+                tiles.append((band * band_of + in_band % band_rows, in_band // band_rows))
+        assert len(tiles) == v["tiles"]
+        assert set(tiles) == {(r, c) for r in range(tiles_m) for c in range(v["tiles_n"])}, (B, L, F_in, R, H, v)
+    assert seen == {(256, 256), (128, 256), (128, 128), (64, 128), (64, 64)}
+    with pytest.raises(capi.FusedAttnError):
+        capi.projection_variant(1, 64, 100, 1, 64)
+
+
 def test_benchmark_workloads_take_the_kernels_the_documentation_names():
     def plan(B, R, L, H, **kw):
         p = capi.launch_plan(B, R, L, H, **kw)

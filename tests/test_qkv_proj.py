@@ -54,6 +54,36 @@ def test_projection_matches_the_oracle(gpu, B, L, Fin, R, H, mode):
     _close(got, want)
 
 
+@pytest.mark.parametrize("B,L,Fin,R,H,tile", [
+    (1, 1, 64, 4, 16, (64, 64)),           # one row, one slice: most of the ring stays empty
+    (5, 13, 256, 12, 16, (64, 64)),        # one row into the second row tile, sequences shorter than a tile
+    (1, 640, 640, 4, 128, (64, 64)),       # tiles of half a head, ten slices: rounds of the ring and a rest
+    (1, 300, 640, 20, 64, (64, 128)),
+    (3, 333, 512, 12, 32, (64, 128)),      # 1152 features, ragged rows
+    (2, 500, 320, 12, 128, (64, 128)),     # five slices: no whole round of the ring
+    (2, 1100, 448, 4, 128, (128, 128)),
+    (1, 777, 704, 20, 64, (128, 128)),
+    (3, 1111, 320, 24, 32, (128, 256)),    # bands of eight row tiles, the last one ragged
+    (1, 1025, 1024, 16, 128, (128, 256)),  # one row into the ninth row tile
+    (1, 2049, 192, 40, 64, (128, 256)),
+    (1, 7000, 512, 20, 64, (256, 256)),    # 420 tiles on 256 workgroups
+])
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("mode", ["plain", "bias+rope"])
+def test_every_tile_shape_matches_the_oracle(gpu, B, L, Fin, R, H, tile, bf16, mode):
+    v = capi.projection_variant(B, L, Fin, R, H)
+    assert (v["tile_m"], v["tile_n"]) == tile
+    F, dtype = R * H, torch.bfloat16 if bf16 else torch.float16
+    x = _rand((B, L, Fin), 7600 + L).to(dtype)
+    w = _rand((Fin, 3 * F), 7601 + L, 1.0 / math.sqrt(Fin)).to(dtype)
+    bias = _rand((3 * F,), 7602 + L).to(dtype) if "bias" in mode else None
+    rope = rope_tables(L, H) if "rope" in mode else None
+    want = qkv_projection(x, w, bias, R, H, *(rope or (None, None)))
+    got = capi.qkv_project(x.to(gpu), w.to(gpu), R, H, bias=bias.to(gpu) if bias is not None else None,
+                           rope=tuple(t.to(gpu) for t in rope) if rope else None)
+    _close(got, want, *((2e-2, 1e-2) if bf16 else (2e-3, 1e-3)))
+
+
 def test_projection_closed_forms_on_the_gpu(gpu):
     # identity weights return the input three times, bit for bit; one-hot columns pick input features
     B, L, R, H = 2, 333, 4, 64

@@ -56,7 +56,7 @@ def load_library():
     lib.fa_qkv_proj.restype = ctypes.c_int
     lib.fa_qkv_proj_plan.argtypes = [i64, i64, i64, i64, i64, ctypes.POINTER(ctypes.c_int)]
     lib.fa_qkv_proj_plan.restype = ctypes.c_int
-    lib.fa_qkv_proj_variant.argtypes = lib.fa_qkv_proj_plan.argtypes
+    lib.fa_qkv_proj_variant.argtypes = [i64, i64, i64, i64, i64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     lib.fa_qkv_proj_variant.restype = ctypes.c_int
     lib.fa_fwd_plan.argtypes = [i64, i64, i64, i64, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     lib.fa_fwd_plan.restype = ctypes.c_int
@@ -107,10 +107,10 @@ def projection_plan(B, L, F_in, R, H):
     return dict(zip(keys, out))
 
 
-def projection_variant(B, L, F_in, R, H):
+def projection_variant(B, L, F_in, R, H, rope=False):
     """What fa_qkv_proj_variant reports for a problem, as a dict.  Needs no GPU."""
     out = (ctypes.c_int * 6)()
-    _check(load_library().fa_qkv_proj_variant(B, L, F_in, R, H, out))
+    _check(load_library().fa_qkv_proj_variant(B, L, F_in, R, H, int(rope), out))
     return dict(zip(("tile_m", "tile_n", "workgroups", "working", "tiles", "tiles_n"), out))
 
 

@@ -839,24 +839,24 @@ hipError_t dispatch_qkv(int64_t rope_head_dim, QkvKind kind, const fa::qkv::Para
     }
 }
 
-// Time of a projection in microseconds, fitted on 220 random shapes (M 64..16384, N 384..15360, K 128..5120) on
-// MI355X: half of them are within 5 % of it, and choosing the smallest estimate loses 0.2 % against the best
-// kernel of each shape (6.6 % at most).  With k workgroups on the busiest of the 256 compute units, w on the
-// mean one and rounds = k over the resident ones:
-//   launch + K / 64 (round rounds + busiest k + mean w) + start rounds + end k
+// Time of a projection in microseconds, fitted on 300 random shapes (M 64..16384, N 384..15360, K 128..5120, both
+// types, with and without tables) on MI355X: half of them are within 5 % of it, and choosing the smallest
+// estimate loses 0.2 % against the best kernel of each shape (9 % at most).  With k workgroups on the busiest
+// of the 256 compute units, w on the mean one and rounds = k over the resident ones:
+//   launch + K / 64 (round rounds + busiest k + mean w) + (start + start_rope) rounds + (end + end_rope) k
 struct QkvCost {
     int resident;
-    float launch, round, busiest, mean, start, end;
+    float launch, round, busiest, mean, start, end, start_rope, end_rope;
 };
 constexpr QkvCost kQkvCost[kQkvKinds] = {
-    {1, 2.594f, 1.081f, 0.f, 0.477f, 10.931f, 0.f},
-    {1, 1.017f, 0.581f, 0.f, 0.239f, 5.956f, 0.f},
-    {1, 1.933f, 0.322f, 0.f, 0.134f, 3.358f, 0.f},
-    {2, 3.226f, 0.058f, 0.147f, 0.139f, 0.272f, 0.787f},
-    {2, 3.577f, 0.021f, 0.069f, 0.134f, 0.f, 0.538f},
+    {1, 0.518f, 1.072f, 0.f, 0.418f, 6.252f, 0.f, 2.267f, 0.f},
+    {1, 1.244f, 0.555f, 0.f, 0.236f, 4.113f, 0.f, 1.791f, 0.f},
+    {1, 2.063f, 0.313f, 0.f, 0.127f, 2.546f, 0.f, 0.84f, 0.f},
+    {2, 3.378f, 0.059f, 0.141f, 0.13f, 0.f, 0.479f, 0.f, 0.556f},
+    {2, 3.471f, 0.026f, 0.071f, 0.114f, 0.f, 0.281f, 0.014f, 0.428f},
 };
 
-QkvKind pick_qkv(int64_t M, int64_t N, int64_t K) {
+QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
 #ifdef FA_TUNE
     const char* env = getenv("FA_QKV");
     if (env != nullptr) return (QkvKind)atoi(env);
@@ -869,7 +869,9 @@ QkvKind pick_qkv(int64_t M, int64_t N, int64_t K) {
         const float mean = (float)ceil_div(M, kQkvTiles[kind].tm) * (float)ceil_div(N, kQkvTiles[kind].tn) / kNumCu;
         if (kind != kQkvWhole && mean > 1e6f) continue;        // (the grid's size in 31 bits)
         const float busiest = ceil_f(mean), rounds = ceil_f(mean / (float)c.resident);
-        const float us = c.launch + slices * (c.round * rounds + c.busiest * busiest + c.mean * mean) + c.start * rounds + c.end * busiest;
+        float us = c.launch + slices * (c.round * rounds + c.busiest * busiest + c.mean * mean) + c.start * rounds + c.end * busiest;
+        if (rope) us += c.start_rope * rounds + c.end_rope * busiest;
+        if (kind == kQkvWhole) us *= 0.96f;        // (between the two the fit is wrong by that much where it matters most)
         if (us < least) {
             least = us;
             best = (QkvKind)kind;
@@ -925,7 +927,7 @@ int fa_qkv_proj(const void* x, const void* w, const void* bias, void* qkv, int64
     p.L = (int)L;
     const int rc = qkv_geometry(B * L, 3 * F, &p);
     if (rc != FA_OK) return rc;
-    const QkvKind kind = pick_qkv(B * L, 3 * F, F_in);
+    const QkvKind kind = pick_qkv(B * L, 3 * F, F_in, rope_cos != nullptr);
     const int rck = use_qkv_kind(kind, &p);
     if (rck != FA_OK) return rck;
     const int64_t hr = rope_cos != nullptr ? H : 0;
@@ -953,7 +955,7 @@ int fa_qkv_proj_plan(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, i
     return FA_OK;
 }
 
-int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, int* variant) {
+int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, int rope, int* variant) {
     int plan[4];
     if (variant == nullptr) return FA_ERR_NULL_POINTER;
     int rc = fa_qkv_proj_plan(B, L, F_in, R, H, plan);
@@ -963,7 +965,7 @@ int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H
     p.N = (int)(3 * R * H);
     rc = qkv_geometry(p.M, p.N, &p);
     if (rc != FA_OK) return rc;
-    const QkvKind kind = pick_qkv(p.M, p.N, F_in);
+    const QkvKind kind = pick_qkv(p.M, p.N, F_in, rope != 0);
     rc = use_qkv_kind(kind, &p);
     if (rc != FA_OK) return rc;
     variant[0] = kQkvTiles[kind].tm;

@@ -229,13 +229,42 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
         int m0, n0;
         tile_origin(done_tile, m0, n0);
         const int nw = n0 + wn * 128;
-        // one run of four features of one row with the bias added
-        auto biased = [&](int nt, int mt, int n) __attribute__((always_inline)) {
-            floatx4 v = acc[nt][mt];
-            if (p.bias != nullptr && n < p.N) {
-                const u16x4 b4 = *reinterpret_cast<const u16x4*>(p.bias + n);
+        // What is read from memory, in one go ahead of its use: the bias of the wave's runs, and per 16-row block
+        // the distinct runs of the tables.  Requested where they are used, one wait behind the other, they took
+        // most of an epilogue's time: M 16384 N 3072 K 1024 with tables 103.9 -> 92.5 us on the same box,
+        // without them 90.3 -> 84.5, M 14400 N 768 K 256 17.5 -> 13.0; at K 5120 it is 1 %.
+        u16x4 bias4[8];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += BF ? bf16::elem_to_float(b4[e]) : elem_to_float(b4[e]);
+        for (int nt = 0; nt < 8; ++nt) {
+            const int n = nw + nt * 16 + 4 * g4;
+            bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
+        }
+        constexpr int RUNS = HR == 0 ? 1 : HR <= 32 ? 1 : HR / 32;
+        floatx4 cos4[RUNS], sin4[RUNS];
+        const int at = HR > 0 ? m0 % p.L + wm * 64 + c16 : 0;
+        auto request = [&](int mt) __attribute__((always_inline)) {
+            if constexpr (HR > 0) {
+                // position of the row in its sequence (rows beyond M: any)
+                int pos = at + mt * 16;
+                if (p.L < kTileM)
+                    pos %= p.L;
+                else
+                    pos -= pos >= p.L ? p.L : 0;
+#pragma unroll
+                for (int i = 0; i < RUNS; ++i) {
+                    const int64_t e = (int64_t)pos * (HR / 2) + (16 * i + 4 * g4) % (HR / 2);
+                    cos4[i] = *reinterpret_cast<const floatx4*>(p.rope_cos + e);
+                    sin4[i] = *reinterpret_cast<const floatx4*>(p.rope_sin + e);
+                }
+            }
+        };
+        request(0);
+        // one run of four features of one row with the bias added
+        auto biased = [&](int nt, int mt) __attribute__((always_inline)) {
+            floatx4 v = acc[nt][mt];
+            if (p.bias != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
             }
             return v;
         };
@@ -255,63 +284,48 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
         };
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            const int m = m0 + wm * 64 + mt * 16 + c16;
-            if constexpr (HR > 0) {
+            if constexpr (HR >= 32) {
                 // rotate-half: within a head, feature i < HR / 2 pairs with feature i + HR / 2:
                 //   out[i] = y[i] cos_i - y[i + HR/2] sin_i,  out[i + HR/2] = y[i + HR/2] cos_i + y[i] sin_i
-                // with cos_i, sin_i taken at the row's position m % L.  Only the q and k slices (n < 2 F).
-                const int pos = (m < p.M ? m : p.M - 1) % p.L;
-                const float* const cs = p.rope_cos + (int64_t)pos * (HR / 2);
-                const float* const sn = p.rope_sin + (int64_t)pos * (HR / 2);
-                if constexpr (HR >= 32) {
-                    // the partner run sits in the same lane, HR / 32 feature blocks on
-                    constexpr int D = HR / 32;
+                // with cos_i, sin_i taken at the row's position.  Only the q and k slices (n < 2 F).  The
+                // partner run sits in the same lane, HR / 32 feature blocks on.
+                constexpr int D = HR / 32;
 #pragma unroll
-                    for (int pr = 0; pr < 4; ++pr) {
-                        const int nt_a = (pr / D) * 2 * D + pr % D, nt_b = nt_a + D;
-                        const int n_a = nw + nt_a * 16 + 4 * g4, n_b = nw + nt_b * 16 + 4 * g4;
-                        floatx4 a = biased(nt_a, mt, n_a);
-                        floatx4 b = biased(nt_b, mt, n_b);
-                        if (n_a < 2 * p.F) {
-                            const int i0 = n_a % (HR / 2);      // index inside the half head
-                            const floatx4 c4 = *reinterpret_cast<const floatx4*>(cs + i0);
-                            const floatx4 s4 = *reinterpret_cast<const floatx4*>(sn + i0);
-                            const floatx4 ra = a * c4 - b * s4;
-                            const floatx4 rb = b * c4 + a * s4;
-                            a = ra;
-                            b = rb;
-                        }
-                        store_run(a, nt_a);
-                        store_run(b, nt_b);
-                        // one pair at a time: all table loads at once would not fit in the registers
-                        __builtin_amdgcn_sched_barrier(0);
+                for (int pr = 0; pr < 4; ++pr) {
+                    const int nt_a = (pr / D) * 2 * D + pr % D, nt_b = nt_a + D;
+                    floatx4 a = biased(nt_a, mt);
+                    floatx4 b = biased(nt_b, mt);
+                    if (nw + nt_a * 16 < 2 * p.F) {
+                        const floatx4 c4 = cos4[pr % D], s4 = sin4[pr % D];
+                        const floatx4 ra = a * c4 - b * s4;
+                        const floatx4 rb = b * c4 + a * s4;
+                        a = ra;
+                        b = rb;
                     }
-                } else {
-                    // head_dim 16: a head is one feature block and the partner of a run sits 32 lanes away
+                    store_run(a, nt_a);
+                    store_run(b, nt_b);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else if constexpr (HR == 16) {
+                // head_dim 16: a head is one feature block and the partner of a run sits 32 lanes away
 #pragma unroll
-                    for (int nt = 0; nt < 8; ++nt) {
-                        const int n = nw + nt * 16 + 4 * g4;
-                        floatx4 a = biased(nt, mt, n);
-                        floatx4 b;
+                for (int nt = 0; nt < 8; ++nt) {
+                    floatx4 a = biased(nt, mt);
+                    floatx4 b;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float ae = a[e];      // (a bit cast taken straight from a vector element reads element 0)
-                            b[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, ae)));
-                        }
-                        if (n < 2 * p.F) {
-                            const int i0 = n % 8;
-                            const floatx4 c4 = *reinterpret_cast<const floatx4*>(cs + i0);
-                            const floatx4 s4 = *reinterpret_cast<const floatx4*>(sn + i0);
-                            a = g4 < 2 ? a * c4 - b * s4 : a * c4 + b * s4;
-                        }
-                        store_run(a, nt);
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int e = 0; e < 4; ++e) {
+                        const float ae = a[e];      // (a bit cast taken straight from a vector element reads element 0)
+                        b[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, ae)));
                     }
+                    if (nw + nt * 16 < 2 * p.F) a = g4 < 2 ? a * cos4[0] - b * sin4[0] : a * cos4[0] + b * sin4[0];
+                    store_run(a, nt);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int nt = 0; nt < 8; ++nt) store_run(biased(nt, mt, nw + nt * 16 + 4 * g4), nt);
+                for (int nt = 0; nt < 8; ++nt) store_run(biased(nt, mt), nt);
             }
+            if (mt < 3) request(mt + 1);
             // LDS operations of one wave complete in order; the waits keep the compiler from moving
             // the reads above the writes (and the next block's writes above these reads)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -204,11 +204,11 @@ int fa_qkv_proj(const void* x, const void* w, const void* bias, void* qkv,
 int fa_qkv_proj_plan(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, int* plan);
 
 /*
- * The kernel fa_qkv_proj picks for a problem, without launching it.  Fills variant[0..5] with: rows and
+ * The kernel fa_qkv_proj picks for a problem (rope != 0: with tables), without launching it.  Fills variant[0..5] with: rows and
  * features of a workgroup's tile (256 x 256: the launch fa_qkv_proj_plan describes; smaller ones: one tile
  * per workgroup); workgroups launched; workgroups that do work; output tiles; feature tiles.
  */
-int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, int* variant);
+int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H, int rope, int* variant);
 
 #ifdef __cplusplus
 }

@@ -60,18 +60,21 @@ def test_projection_matches_the_oracle(gpu, B, L, Fin, R, H, mode):
     (1, 640, 640, 4, 128, (64, 64)),       # tiles of half a head, ten slices: rounds of the ring and a rest
     (1, 300, 640, 20, 64, (64, 128)),
     (3, 333, 512, 12, 32, (64, 128)),      # 1152 features, ragged rows
-    (2, 500, 320, 12, 128, (64, 128)),     # five slices: no whole round of the ring
+    (2, 300, 320, 8, 128, (64, 128)),      # five slices: no whole round of the ring
     (2, 1100, 448, 4, 128, (128, 128)),
     (1, 777, 704, 20, 64, (128, 128)),
     (3, 1111, 320, 24, 32, (128, 256)),    # bands of eight row tiles, the last one ragged
     (1, 1025, 1024, 16, 128, (128, 256)),  # one row into the ninth row tile
     (1, 2049, 192, 40, 64, (128, 256)),
     (1, 7000, 512, 20, 64, (256, 256)),    # 420 tiles on 256 workgroups
+    (70, 100, 512, 10, 128, (256, 256)),   # sequences shorter than a tile
+    (2, 3500, 512, 40, 32, (256, 256)),
+    (20, 350, 512, 80, 16, (256, 256)),
 ])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("mode", ["plain", "bias+rope"])
 def test_every_tile_shape_matches_the_oracle(gpu, B, L, Fin, R, H, tile, bf16, mode):
-    v = capi.projection_variant(B, L, Fin, R, H)
+    v = capi.projection_variant(B, L, Fin, R, H, rope="rope" in mode)
     assert (v["tile_m"], v["tile_n"]) == tile
     F, dtype = R * H, torch.bfloat16 if bf16 else torch.float16
     x = _rand((B, L, Fin), 7600 + L).to(dtype)

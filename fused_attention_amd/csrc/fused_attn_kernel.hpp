@@ -223,7 +223,7 @@ constexpr int group_ring_bytes() { return group_slots<H, GK>() * GK * group_sub<
 // groups, the waves' shares of O (whichever is larger), and behind them m and l of every row.
 template <int H, int NQ, int GK, bool MASK>
 constexpr int group_stat_offset() {
-    constexpr int ring = group_ring_bytes<H, GK>() + (MASK ? 8 * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 * 16 * NQ * split_row_floats<H>() * 4;
+    constexpr int ring = group_ring_bytes<H, GK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 * 16 * NQ * split_row_floats<H>() * 4;
     return ring > part ? ring : part;
 }
 template <int H, int NQ, int GK, bool MASK>

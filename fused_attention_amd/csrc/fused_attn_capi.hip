@@ -495,6 +495,12 @@ constexpr Cost kCostTile16[2][2] = {     // [head_dim 64, 128][plain, causal], f
     {{0.f, 0.87f, 6.45f}, {0.f, 0.977f, 9.08f}},
 };
 
+// ... which is too much for a lone round of plain 64-row waves, whose idle units leave the others a higher clock:
+// where 0.94 of it decides for the tile kernel that is the faster one on 12 of 13 random shapes, by up to
+// 12 % (B2 R40 L1301 52.7 -> 46.9 us, B3 R12 L3200 102.5 -> 92.6, B3 R20 L1408 41.2 -> 41.1, B5 R12 L1408
+// 41.3 -> 42.0).  Over several rounds the same factor loses as often as it gains (0.87 to 1.05).
+constexpr float kLoneRoundTile = 0.94f;
+
 float ceil_f(float x) {
     const float t = (float)(int64_t)x;
     return t < x ? t + 1.f : t;
@@ -554,7 +560,9 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         const Cost& t = !has_mask && use_tiles16(H, tile, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
                                                                      : kCostTile[h][has_mask ? 2 : causal ? 1 : 0];
         const float rounds = ceil_f(u);
-        offer(kTile, 8, kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds);
+        float us = kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds;
+        if (H == 64 && !has_mask && !causal && rounds == 1.f) us *= kLoneRoundTile;
+        offer(kTile, 8, us);
     }
     return best;
 }

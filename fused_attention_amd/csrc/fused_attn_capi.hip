@@ -172,7 +172,7 @@ hipError_t allow_large_lds(const void* kernel, int bytes) {
 // BF selects the bf16 instantiation (namespace fa::bf16) of the same kernel source.
 template <int H, int NW, int NQB, int WPE, int MODE, bool BF>
 hipError_t launch_pingpong(const fa::FwdParams& p, hipStream_t stream) {
-    constexpr int lds = MODE == fa::kAdditive ? fa::lds_bytes_pingpong_masked<H, NW, NQB>() : fa::lds_bytes_pingpong<H, NQB>();
+    constexpr int lds = MODE == fa::kAdditive || MODE == fa::kAdditiveRagged ? fa::lds_bytes_pingpong_masked<H, NW, NQB>() : fa::lds_bytes_pingpong<H, NQB>();
     auto kernel = BF ? fa::bf16::fwd_kernel_pingpong<H, NW, NQB, WPE, MODE> : fa::fwd_kernel_pingpong<H, NW, NQB, WPE, MODE>;
     if constexpr (lds > 64 * 1024) {
         const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), lds);
@@ -642,6 +642,8 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
         e = dispatch<fa::kCausalDealt>(H, shape, p, s, bf16);
     else if (causal)
         e = dispatch<fa::kCausal>(H, shape, p, s, bf16);
+    else if (mask != nullptr && L % 8 != 0)
+        e = dispatch<fa::kAdditiveRagged>(H, shape, p, s, bf16);
     else if (mask != nullptr)
         e = dispatch<fa::kAdditive>(H, shape, p, s, bf16);
     else

@@ -83,6 +83,7 @@ constexpr int kPlain = 0;    // no mask
 constexpr int kAdditive = 1; // additive [B, L, L] mask
 constexpr int kCausal = 2;   // key index <= query index, key tiles above the diagonal skipped
 constexpr int kCausalDealt = 3;   // tile kernels only: causal with the query tiles dealt out to a resident grid
+constexpr int kAdditiveRagged = 4;   // tile kernels only: additive mask, L no multiple of eight
 
 template <int H>
 struct Geometry {

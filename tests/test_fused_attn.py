@@ -1034,6 +1034,41 @@ def test_mask_rows_at_any_alignment(gpu, L, H):
         assert _max_err(got[b, :, sl], want[0]) <= TOL, (b, h)
 
 
+def _shape_on(kernel, H, mode, lengths, rows=None, fits=lambda v: True):
+    """The first (B, R, L) of a small grid of problems, of one of these lengths, that the library runs on this
+    kernel (and, if given, with this many query rows per workgroup and a launch that `fits`)."""
+    for L in lengths:
+        for B, R in [(1, r) for r in range(1, 64)] + [(2, 40), (1, 96), (1, 128), (1, 160), (2, 120), (1, 320)]:
+            v = capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
+            if v["kernel"] == kernel and (rows is None or v["rows"] == rows) and fits(v):
+                return B, R, L
+    raise AssertionError((kernel, H, mode, lengths, rows))
+
+
+@pytest.mark.parametrize("H", [16, 32, 64, 128])
+@pytest.mark.parametrize("residue", [0, 1, 4, 7])
+def test_masked_tile_kernel(gpu, H, residue):
+    # The tile kernel with an additive mask at every head_dim, with rows of any length: where L is no multiple
+    # of eight the last chunk of a row is fetched from where it still fits and shifted into place.  The
+    # last nine keys carry most of the weight, and no two of them the same mask value.
+    B, R, L = _shape_on("tile", H, "mask", [8 * n + residue for n in (127, 191, 255, 320, 447, 511)])
+    dtype = torch.bfloat16 if (H // 16 + residue) % 2 else torch.float16
+    q, k, v = (_rand((B, L, R * H), 5300 + L + i).to(dtype) for i in range(3))
+    mask = _block_mask("blocks", B, L, 5310 + L).float()
+    mask[:, :, L - 9:] = torch.arange(9).float() * 0.75 + 2.0
+    mask[:, ::3, L - 5:] = float("-inf")
+    mask = mask.to(dtype)
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu), return_lse=True)
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        want = attention(*args, mask=mask[b:b + 1].float())
+        assert _max_err(got[b, :, sl], want[0]) <= (TOL if dtype == torch.float16 else BF16_TOL), (b, h)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        off = (lse[b, h].cpu() - attention_lse(args[0], args[1], H, mask=mask[b:b + 1].float())[0, 0]).abs()
+        assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
+
+
 # One shape or two per kernel and head_dim, at the edges of their tiles: 16, 64, 128 and 256 query rows, 32 keys
 # per sub-tile, 64 keys per key tile and three key tiles per turn of the ring.
 SMALL_GRIDS = [(1, 1, 1), (2, 3, 17), (1, 5, 33), (2, 4, 129), (1, 3, 300), (3, 40, 130), (2, 40, 255), (2, 16, 513),

@@ -630,6 +630,7 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     if (rc != FA_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;
+    if (bf16) p.bias = fa::kBiasBf16;
     const Variant variant = pick_variant(B, R, L, H, mask != nullptr, causal, shape, p);
     if (variant.kind != kTile) {
         const int rcv = use_variant(variant, &p);

@@ -136,9 +136,17 @@ __device__ __forceinline__ u32x4 drop_halves(u32x4 v, uint32_t n) {
 // at or below 2^-13 = 1.2e-4 whatever the sequence length; what is left of the fp16 range is the
 // leash of the speculative reference, which may lag the true maximum by 15 + bias log2 units before
 // the check sends the wave down the slow path: 14 units at L = 4096, 12 at 16384, 10 at 65536.
+// bf16 probabilities have the exponents of float32 and lose nothing at the bottom.  What the bias is limited by
+// there is O, which is summed in float32 before it is divided by the row sum: at 2^14 its last bit,
+// 2^-149, is still below a bf16 subnormal's, 2^-133, once divided (2^16 was measured to cost values
+// around 2^-120 precision).  The leash is 29 units, and the sums of a sub-tile stay below kTripSum
+// all the same, so that values up to 2^128 / (kTripSum L / 32) pass whatever the scores do.  (Raising
+// kTripSum to 2^32 instead gives the same leash and infinities from values of 2^91 on, where scores rise
+// that far; without the longer leash scores with a spread of N(0, 3) inputs take 1.03 to 1.3 times as long.)
 constexpr float kBiasMin = -8.0f;
 constexpr float kBiasMax = 6.0f;
 constexpr float kTripSum = 32768.f;
+constexpr float kBiasBf16 = 14.0f;
 
 // O^T[.][nb] *= alpha, in place.  Written as one instruction per register with the register tied
 // as input and output, so that the rarely taken rescale does not make the compiler keep a second

@@ -75,7 +75,8 @@ int fa_fwd(const void* q, const void* k, const void* v, const void* mask, void* 
  *                            are skipped.  Not combinable with `mask`.
  *   flags & FA_FLAG_BF16   : q, k, v, out (and mask) hold bfloat16 instead of fp16 (reference
  *                            README.md:137 lists other input types as not done).  Same kernels,
- *                            bf16 matrix instructions, probabilities rounded to bf16.
+ *                            bf16 matrix instructions, probabilities rounded to bf16 (with the exponents
+ *                            of float32: no key of a row is too small to contribute).
  *   lse (nullable)         : float32 [B, R, L] in device memory, receives
  *                            log(sum_j exp(score_ij)) per query row (-inf for a row whose keys
  *                            are all masked): what a backward pass needs to recompute the
@@ -138,7 +139,7 @@ int fa_fwd_query(int64_t H);
 
 /*
  * The power of two (as a base-2 exponent) the softmax weights of a row of L keys are divided by
- * before they are rounded to 16 bits for the second product: a key at the running maximum of its
+ * before they are rounded to fp16 for the second product (bf16 weights: 2^14 at every length): a key at the running maximum of its
  * row gets the weight 2^-bias.  11 - ceil(log2 L), kept inside [-8, 6]: see "Accuracy" under fa_fwd.
  * Exported so that callers and tests can state the accuracy limit of a launch; no counterpart in the
  * reference, which keeps every intermediate in fp16 (reference include/fused_attn.cuh:174,257,650-653).

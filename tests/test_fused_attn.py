@@ -1228,6 +1228,36 @@ def test_bf16_additive_mask_and_closed_forms(gpu, B, R, L, H):
         capi.forward(q.to(gpu), k.half().to(gpu), v.to(gpu), H)
 
 
+@pytest.mark.parametrize("kernel", ["split", "group", "tile"])
+@pytest.mark.parametrize("H,mode", [(16, "plain"), (32, "mask"), (64, "plain"), (64, "causal"), (64, "mask"),
+                                    (128, "plain"), (128, "causal"), (128, "mask")])
+@pytest.mark.parametrize("power,rise", [(100, 9.0), (100, 25.0), (100, 60.0), (-118, 25.0)])
+def test_bf16_values_at_the_ends_of_the_range(gpu, kernel, H, mode, power, rise):
+    # Scores that rise by so many log2 units behind the first 256 keys leave the reference of the
+    # exponentials behind: O, summed in float32 before the division by the row sum, must stay in range for
+    # values of 2^100, and values of 2^-118 must not sink into its subnormals.
+    B, R, L = _shape_on(kernel, H, mode, (448, 512, 1024, 1536, 2048, 3072, 4096))
+    g = torch.Generator().manual_seed(5400 + L)
+    v = (2.0 ** power * (1.0 + 0.25 * torch.randn(B, L, R * H, generator=g))).to(torch.bfloat16)
+    q = torch.ones(B, L, R * H, dtype=torch.bfloat16)
+    ramp = torch.zeros(L)
+    ramp[256:] = rise * math.log(2.0) / math.sqrt(H)
+    k = ramp.view(1, L, 1).expand(B, L, R * H).to(torch.bfloat16).contiguous()
+    mask = None
+    if mode == "mask":
+        mask = torch.zeros(B, L, L, dtype=torch.bfloat16)
+        mask[:, :, ::7] = -0.5                             # nowhere a block of zeros
+    got = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu) if mask is not None else None, causal=mode == "causal")
+    assert torch.isfinite(got).all()
+    s = k[0, :, 0].double() * math.sqrt(H) + (mask[0, 0].double() if mask is not None else 0.0)
+    p = torch.exp(s - s.max())
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sums = torch.cumsum(p[:, None] * v[b, :, h * H:(h + 1) * H].double(), 0), torch.cumsum(p, 0)[:, None]
+        want = sums[0] / sums[1] if mode == "causal" else (sums[0][-1] / sums[1][-1]).expand(L, H)
+        # two roundings to 8 bits, the weights' (in numerator and denominator alike) and the result's
+        assert ((got[b, :, h * H:(h + 1) * H].double().cpu() - want).abs() / 2.0 ** power).max().item() <= 2.0 ** -6, (b, h)
+
+
 @pytest.mark.parametrize("B,R,L,H", [(2, 3, 200, 64), (4, 16, 2048, 64), (2, 40, 1024, 128)])
 def test_extensions_through_the_compiled_module(gpu, B, R, L, H):
     """fused_attn.attention_forward_ex: causal, mask, log-sum-exp, bf16, the [B, R, L, H] layout and

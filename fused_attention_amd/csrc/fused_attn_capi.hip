@@ -628,13 +628,28 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     const int rc = validate(q, k, v, mask, out, B, R, L, H, Strides{stride_b, stride_h, stride_l},
                             Strides{out_stride_b, out_stride_h, out_stride_l}, &p, scale, &shape, causal, lse);
     if (rc != FA_OK) return rc;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    hipError_t e;
     if (bf16) p.bias = fa::kBiasBf16;
     const Variant variant = pick_variant(B, R, L, H, mask != nullptr, causal, shape, p);
+    const int rcv = variant.kind != kTile ? use_variant(variant, &p) : FA_OK;
+    // A grid of 2^32 threads or more does not fit the dispatch packet (head_dim 16, L = 43: from 11 million heads
+    // on): such a problem runs as two, halves of the batch or of the heads.
+    const int64_t threads = (int64_t)p.wgs_per_xcd * fa::kNumXcd * 64 * (variant.kind == kSplit ? variant.waves : 8);
+    if (rcv != FA_OK && B * R == 1) return rcv;
+    if ((rcv != FA_OK || threads > 0xffffffffll) && B * R > 1) {
+        const int64_t B1 = B > 1 ? B / 2 : 1, R1 = B > 1 ? R : R / 2;
+        const int64_t in = B > 1 ? B1 * stride_b : R1 * stride_h, to = B > 1 ? B1 * out_stride_b : R1 * out_stride_h;
+        auto at = [](const void* ptr, int64_t elements) { return static_cast<const uint16_t*>(ptr) + elements; };
+        const int first = fa_fwd_strided(q, k, v, mask, out, lse, B1, R1, L, H, stride_b, stride_h, stride_l, out_stride_b,
+                                         out_stride_h, out_stride_l, scale, flags, stream);
+        if (first != FA_OK) return first;
+        return fa_fwd_strided(at(q, in), at(k, in), at(v, in), mask != nullptr && B > 1 ? at(mask, B1 * L * L) : mask,
+                              const_cast<uint16_t*>(at(out, to)), lse != nullptr ? static_cast<float*>(lse) + B1 * R1 * L : nullptr,
+                              B > 1 ? B - B1 : 1, B > 1 ? R : R - R1, L, H, stride_b, stride_h, stride_l, out_stride_b,
+                              out_stride_h, out_stride_l, scale, flags, stream);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipError_t e;
     if (variant.kind != kTile) {
-        const int rcv = use_variant(variant, &p);
-        if (rcv != FA_OK) return rcv;
         const int mode = causal ? fa::kCausal : mask != nullptr ? fa::kAdditive : fa::kPlain;
         e = bf16 ? dispatch_variant_mode<true>(H, mode, variant, p, s) : dispatch_variant_mode<false>(H, mode, variant, p, s);
     } else if (mask == nullptr && use_tiles16(H, shape, p, causal))
@@ -878,7 +893,8 @@ QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
     for (int kind = 0; kind < kQkvKinds; ++kind) {
         const QkvCost& c = kQkvCost[kind];
         const float mean = (float)ceil_div(M, kQkvTiles[kind].tm) * (float)ceil_div(N, kQkvTiles[kind].tn) / kNumCu;
-        if (kind != kQkvWhole && mean > 1e6f) continue;        // (the grid's size in 31 bits)
+        // (a grid of less than 2^32 threads: the dispatch packet holds no more)
+        if (kind != kQkvWhole && mean > (float)(0xffffffffu / (64 * fa::qkv::kWaves) / kNumCu - 1)) continue;
         const float busiest = ceil_f(mean), rounds = ceil_f(mean / (float)c.resident);
         float us = c.launch + slices * (c.round * rounds + c.busiest * busiest + c.mean * mean) + c.start * rounds + c.end * busiest;
         if (rope) us += c.start_rope * rounds + c.end_rope * busiest;

@@ -117,6 +117,7 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
  * the matrix instruction's tile, 32, or 16 at head_dim 64 and 128 for plain launches of the eight-wave
  * kernel whose workgroups fill whole rounds of the chip (the last round at least seven eighths full)
  * and for its causal launches from seven eighths of a round on.
+ * (A problem whose grid would have 2^32 threads or more is launched in parts, halves of its batch or heads.)
  * The reference has no counterpart (its grid is fixed at (B, L / chunk_size, R),
  * reference include/fused_attn.cuh:872-883).
  */

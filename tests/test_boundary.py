@@ -232,6 +232,16 @@ def test_every_projection_variant_covers_every_output_tile_once():
         capi.projection_variant(1, 64, 100, 1, 64)
 
 
+def test_projection_grids_stay_below_2_to_the_32_threads():
+    # the dispatch packet counts threads in 32 bits; narrow outputs of very many rows are where the small tiles,
+    # one workgroup of 512 threads each, would pass that
+    for M in (2 ** 24 + 3, 2 ** 27, 2 ** 28, 2 ** 30):
+        for R, H in ((1, 64), (2, 64), (3, 64), (4, 16), (5, 64)):
+            for rope in (False, True):
+                v = capi.projection_variant(1, M, 64, R, H, rope=rope)
+                assert v["workgroups"] * 512 < 2 ** 32, (M, R, H, rope, v)
+
+
 def test_benchmark_workloads_take_the_kernels_the_documentation_names():
     def plan(B, R, L, H, **kw):
         p = capi.launch_plan(B, R, L, H, **kw)

@@ -1228,6 +1228,33 @@ def test_bf16_additive_mask_and_closed_forms(gpu, B, R, L, H):
         capi.forward(q.to(gpu), k.half().to(gpu), v.to(gpu), H)
 
 
+@pytest.mark.parametrize("B,R,mode", [(11_999_999, 1, "plain"), (2_999_999, 4, "causal"), (2_999_999, 4, "mask")])
+def test_more_workgroups_than_one_grid_holds(gpu, B, R, mode):
+    # Grids of 2^32 threads and more, which a dispatch packet does not hold, run in parts.  Every head reads and
+    # writes the same few rows (strides of zero), the log-sum-exps are its own.
+    L, H = 43, 16
+    v = capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
+    assert v["workgroups"] * 64 * v["waves"] >= 2 ** 32
+    q, k, val = (_rand((1, L, H), 5600 + i).to(gpu) for i in range(3))
+    mask, above = None, torch.zeros(B * R, 1, device=gpu)
+    if mode == "mask":                     # 1 more everywhere in the last third of the batch
+        g = torch.Generator().manual_seed(5605)
+        mask = (torch.randint(-32, 32, (1, L, L), generator=g) / 16.0).half().to(gpu).expand(B, L, L).contiguous()
+        mask[2 * B // 3:] += 1.0
+        above[2 * B // 3 * R:] = 1.0
+    want, lse1 = capi.forward(q, k, val, H, mask=None if mask is None else mask[:1], causal=mode == "causal", return_lse=True)
+    out = torch.zeros_like(want)
+    lse = torch.full((B * R, L), float("nan"), device=gpu)
+    status = capi.load_library().fa_fwd_strided(
+        q.data_ptr(), k.data_ptr(), val.data_ptr(), mask.data_ptr() if mask is not None else None, out.data_ptr(),
+        lse.data_ptr(), B, R, L, H, 0, 0, H, 0, 0, H, 0.25, capi.FLAG_CAUSAL if mode == "causal" else 0,
+        torch.cuda.current_stream().cuda_stream or None)
+    assert status == 0, capi.strerror(status)
+    # (another kernel than the small problem's, perhaps: one rounding of a probability apart)
+    assert (out.float() - want.float()).abs().max().item() <= TOL
+    assert (lse - above - lse1[0, 0]).abs().max().item() <= 2.0 ** -10
+
+
 @pytest.mark.parametrize("kernel", ["split", "group", "tile"])
 @pytest.mark.parametrize("H,mode", [(16, "plain"), (32, "mask"), (64, "plain"), (64, "causal"), (64, "mask"),
                                     (128, "plain"), (128, "causal"), (128, "mask")])

@@ -420,60 +420,74 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
     return FA_OK;
 }
 
-// Time of a launch of the key-split or the group kernel, in microseconds: a fit over 1350 random shapes
-// (B 1..32, R 4..40, L 32..16384, every head_dim, plain, causal and masked) on MI355X; half of the
-// shapes are within 5 % of it.  What counts is the order of the estimates: choosing the smallest one
-// loses 1.8 % against the best kernel of each shape.
+// Time of a launch of the key-split or the group kernel, in microseconds: fits over 10700 random shapes
+// (B 1..32, R 4..40, L 32..16384, every head_dim; plain, causal and four kinds of mask, bias, padding, causal
+// pattern and documents, which no estimate can tell apart beforehand) on MI355X, then moved a little, within
+// each head_dim and mode, towards the order of the measured times; half of the estimates of kernels worth
+// choosing are within 4.3 %.  What counts is their order: choosing the smallest one loses 0.9 % against the
+// best kernel of each shape, and more than 5 % for 6 % of them.  (The fit before, without s, one for plain
+// and causal, mostly on smaller shapes: 2.1 and 15 %.  It was wrong where one round of tile kernel workgroups
+// does not fill the chip: 12 % at head_dim 32, 35 % for causal launches, 39 % for padding masks, and a factor
+// for plain launches at head_dim 64 stood in for the rest.)  On 2100 shapes timed afterwards the choice takes
+// 1.3 % less time than that fit's; 50 of them, 146 before, take over 3 % more than the kernel that ran them
+// when there were tile kernels only.  Those are padding and causal-pattern masks for the most part, whose
+// muted blocks the tile kernels skip at less cost: the same shape with a bias or documents is
+// 10 to 40 % faster on the group kernel.
 //   split:  kLaunch + a ceil(sub-tiles / waves)              the longest wave
 //                   + b sub-tiles of all workgroups / 256    one compute unit's share of the work
-//                   + c workgroups / 256                     start and merge
+//                   + c k                                    start and merge
 //   group:  kLaunch + a (sub-tiles + (rounds - 1) mean) / GK      the longest chain of workgroups
-//                   + b mean w / GK + c k                          w = workgroups per compute unit, taken
-//                                                                  half way between the mean and
-//                                                                  the most (k) of any
+//                   + b mean w / GK                               w = workgroups per compute unit, taken
+//                                                                 half way between the mean and
+//                                                                 the most (k) of any
+//                   + s sub-tiles min(k, resident) / GK           the longest one's neighbours
+//                   + c k
 // with sub-tiles of 32 keys, a causal tile's mean being about half of them, and rounds = k over the
 // workgroups resident per compute unit.
 struct Cost {
     float a, b, c;
 };
+struct GroupCost {
+    float a, b, s, c;
+};
 constexpr float kLaunch = 3.2f;
-// [head_dim 16, 32, 64, 128][without, with mask]
-constexpr Cost kCostSplit2[4][2] = {
-    {{0.139f, 0.053f, 0.087f}, {0.114f, 0.071f, 0.095f}},
-    {{0.143f, 0.057f, 0.129f}, {0.291f, 0.076f, 0.065f}},
-    {{0.291f, 0.071f, 0.316f}, {0.356f, 0.087f, 0.301f}},
-    {{0.525f, 0.136f, 1.05f}, {0.733f, 0.153f, 1.05f}},
+// [head_dim 16, 32, 64, 128][plain, causal, mask]
+constexpr Cost kCostSplit2[4][3] = {
+    {{0.0987f, 0.0404f, 0.117f}, {0.182f, 0.0476f, 0.113f}, {0.237f, 0.0567f, 0.124f}},
+    {{0.134f, 0.0506f, 0.157f}, {0.201f, 0.0523f, 0.185f}, {0.291f, 0.0607f, 0.181f}},
+    {{0.312f, 0.0598f, 0.415f}, {0.335f, 0.0473f, 0.505f}, {0.47f, 0.0765f, 0.366f}},
+    {{0.503f, 0.0772f, 1.69f}, {0.696f, 0.0458f, 1.04f}, {0.871f, 0.0688f, 1.06f}},
 };
-constexpr Cost kCostSplit4[4][2] = {
-    {{0.201f, 0.055f, 0.152f}, {0.357f, 0.076f, 0.076f}},
-    {{0.124f, 0.057f, 0.223f}, {0.52f, 0.079f, 0.076f}},
-    {{0.265f, 0.072f, 0.525f}, {0.379f, 0.086f, 0.493f}},
-    {{0.612f, 0.137f, 1.81f}, {0.854f, 0.165f, 1.74f}},
+constexpr Cost kCostSplit4[4][3] = {
+    {{0.105f, 0.0493f, 0.138f}, {0.202f, 0.0465f, 0.219f}, {0.371f, 0.063f, 0.144f}},
+    {{0.16f, 0.0496f, 0.268f}, {0.238f, 0.0537f, 0.309f}, {0.397f, 0.0605f, 0.244f}},
+    {{0.298f, 0.0603f, 0.492f}, {0.18f, 0.0783f, 0.535f}, {0.458f, 0.0685f, 0.579f}},
+    {{0.457f, 0.122f, 1.36f}, {0.374f, 0.137f, 1.33f}, {0.857f, 0.0981f, 1.44f}},
 };
-constexpr Cost kCostGroup11[4][2] = {
-    {{0.242f, 0.102f, 0.452f}, {0.275f, 0.2f, 0.482f}},
-    {{0.162f, 0.14f, 0.353f}, {0.208f, 0.257f, 0.296f}},
-    {{0.215f, 0.22f, 0.449f}, {0.244f, 0.363f, 0.582f}},
-    {{0.422f, 0.327f, 0.944f}, {0.614f, 0.387f, 0.739f}},
+constexpr GroupCost kCostGroup11[4][3] = {
+    {{0.14f, 0.115f, 0.0523f, 0.493f}, {0.196f, 0.109f, 0.0289f, 0.495f}, {0.254f, 0.174f, 0.031f, 0.601f}},
+    {{0.114f, 0.135f, 0.0291f, 0.433f}, {0.188f, 0.113f, 0.0242f, 0.414f}, {0.246f, 0.184f, 0.0129f, 0.569f}},
+    {{0.177f, 0.212f, 0.0291f, 0.588f}, {0.228f, 0.193f, 0.0244f, 0.48f}, {0.18f, 0.294f, 0.0551f, 0.958f}},
+    {{0.361f, 0.332f, 0.00792f, 1.13f}, {0.407f, 0.308f, 0.f, 1.21f}, {0.417f, 0.363f, 0.0182f, 1.47f}},
 };
-constexpr Cost kCostGroup12[4][2] = {
-    {{0.249f, 0.128f, 0.661f}, {0.278f, 0.264f, 0.49f}},
-    {{0.143f, 0.169f, 0.735f}, {0.231f, 0.31f, 0.512f}},
-    {{0.252f, 0.186f, 1.24f}, {0.372f, 0.339f, 1.17f}},
-    {{0.36f, 0.392f, 2.61f}, {0.672f, 0.419f, 2.32f}},
+constexpr GroupCost kCostGroup12[4][3] = {
+    {{0.172f, 0.135f, 0.0295f, 0.523f}, {0.253f, 0.118f, 0.0128f, 0.688f}, {0.295f, 0.263f, 0.f, 0.581f}},
+    {{0.143f, 0.159f, 0.0207f, 0.585f}, {0.226f, 0.136f, 0.00969f, 0.81f}, {0.256f, 0.262f, 0.f, 0.648f}},
+    {{0.198f, 0.195f, 0.0635f, 1.14f}, {0.264f, 0.155f, 0.0333f, 1.25f}, {0.342f, 0.252f, 0.0164f, 1.41f}},
+    {{0.378f, 0.343f, 0.0064f, 2.37f}, {0.378f, 0.334f, 0.f, 2.64f}, {0.473f, 0.399f, 0.0274f, 2.5f}},
 };
-constexpr Cost kCostGroup21[4][2] = {
-    {{0.371f, 0.128f, 0.639f}, {0.465f, 0.29f, 1.03f}},
-    {{0.289f, 0.2f, 0.514f}, {0.378f, 0.405f, 1.f}},
-    {{0.399f, 0.307f, 0.837f}, {0.559f, 0.446f, 1.33f}},
-    {{0.865f, 0.136f, 1.97f}, {0.934f, 0.601f, 1.97f}},
+constexpr GroupCost kCostGroup21[4][3] = {
+    {{0.191f, 0.192f, 0.068f, 0.687f}, {0.243f, 0.209f, 0.0796f, 0.144f}, {0.372f, 0.323f, 0.0533f, 1.22f}},
+    {{0.197f, 0.221f, 0.0518f, 0.616f}, {0.278f, 0.203f, 0.0567f, 0.147f}, {0.388f, 0.332f, 0.0549f, 1.23f}},
+    {{0.27f, 0.35f, 0.044f, 1.25f}, {0.344f, 0.369f, 0.0525f, 0.269f}, {0.515f, 0.42f, 0.0741f, 1.7f}},
+    {{0.56f, 0.492f, 0.00712f, 2.09f}, {0.489f, 0.627f, 0.f, 1.34f}, {0.712f, 0.567f, 0.f, 3.03f}},
 };
 
 struct GroupShape {
     VariantKind kind;
     int nq, gk;
     int resident[4];            // workgroups per compute unit, by head_dim
-    const Cost (*cost)[2];
+    const GroupCost (*cost)[3];
 };
 constexpr GroupShape kGroups[] = {
     {kGroup11, 1, 1, {3, 3, 3, 2}, kCostGroup11},
@@ -483,23 +497,17 @@ constexpr GroupShape kGroups[] = {
 
 // The same for the eight-wave tile kernels that are left beside them: 64-row waves at head_dim 16 to 64,
 // 32-row waves at 128.  One workgroup per compute unit: a per sub-tile of a round, b per sub-tile of the mean
-// compute unit, c per round.
+// compute unit (idle units leave the others a higher clock), c per round.
 constexpr Cost kCostTile[4][3] = {       // [head_dim][plain, causal, mask], fwd_kernel_pingpong
-    {{0.51f, 0.094f, 4.06f}, {0.686f, 0.f, 4.38f}, {0.991f, 0.f, 3.04f}},
-    {{0.419f, 0.258f, 3.15f}, {0.38f, 0.34f, 0.f}, {0.345f, 0.89f, 4.08f}},
-    {{0.408f, 0.58f, 4.08f}, {0.894f, 0.f, 0.f}, {1.159f, 0.291f, 4.27f}},
-    {{0.248f, 0.687f, 7.49f}, {0.716f, 0.f, 11.7f}, {0.933f, 0.363f, 6.72f}},
+    {{0.536f, 0.0518f, 2.81f}, {0.614f, 0.0242f, 7.91f}, {0.825f, 0.136f, 5.06f}},
+    {{0.498f, 0.137f, 2.57f}, {0.599f, 0.0832f, 8.89f}, {0.811f, 0.27f, 3.73f}},
+    {{0.469f, 0.459f, 4.44f}, {0.654f, 0.147f, 11.4f}, {1.07f, 0.294f, 7.86f}},
+    {{0.297f, 0.6f, 5.26f}, {0.505f, 0.287f, 15.2f}, {0.952f, 0.288f, 6.73f}},
 };
 constexpr Cost kCostTile16[2][2] = {     // [head_dim 64, 128][plain, causal], fwd_kernel_pp16
-    {{0.27f, 0.645f, 7.08f}, {0.302f, 0.68f, 7.69f}},
-    {{0.f, 0.87f, 6.45f}, {0.f, 0.977f, 9.08f}},
+    {{0.508f, 0.362f, 7.63f}, {0.0783f, 0.851f, 10.1f}},
+    {{0.184f, 0.662f, 6.51f}, {0.f, 0.913f, 9.56f}},
 };
-
-// ... which is too much for a lone round of plain 64-row waves, whose idle units leave the others a higher clock:
-// where 0.94 of it decides for the tile kernel that is the faster one on 12 of 13 random shapes, by up to
-// 12 % (B2 R40 L1301 52.7 -> 46.9 us, B3 R12 L3200 102.5 -> 92.6, B3 R20 L1408 41.2 -> 41.1, B5 R12 L1408
-// 41.3 -> 42.0).  Over several rounds the same factor loses as often as it gains (0.87 to 1.05).
-constexpr float kLoneRoundTile = 0.94f;
 
 float ceil_f(float x) {
     const float t = (float)(int64_t)x;
@@ -519,7 +527,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
     }
 #endif
     const int h = H == 16 ? 0 : H == 32 ? 1 : H == 64 ? 2 : 3;
-    const int m = has_mask ? 1 : 0;
+    const int m = has_mask ? 2 : causal ? 1 : 0;
     const float heads = (float)(B * R), nsub = (float)ceil_div(L, 32);
     Variant best{kGroup11, 8};
     float least = 3.0e38f;
@@ -535,7 +543,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         const float mean = causal ? 0.5f * (nsub + 0.5f) : nsub;
         for (int waves = 2; waves <= (nsub > 2.f ? 4 : 2); waves += 2) {
             const Cost& t = waves == 2 ? kCostSplit2[h][m] : kCostSplit4[h][m];
-            offer(kSplit, waves, kLaunch + t.a * ceil_f(nsub / (float)waves) + t.b * wgs * mean + t.c * wgs);
+            offer(kSplit, waves, kLaunch + t.a * ceil_f(nsub / (float)waves) + t.b * wgs * mean + t.c * ceil_f(wgs));
         }
     }
     for (const GroupShape& g : kGroups) {
@@ -543,8 +551,9 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         const float wgs = heads * (float)ceil_div(L, rows) / kNumCu, k = ceil_f(wgs);
         const float mean = causal ? 0.5f * (nsub + (float)rows / 32.f) : nsub;
         const float rounds = ceil_f(wgs / (float)g.resident[h]);
-        const Cost& t = g.cost[h][m];
-        offer(g.kind, 8, kLaunch + (t.a * (nsub + (rounds - 1.f) * mean) + t.b * mean * 0.5f * (wgs + k)) / (float)g.gk + t.c * k);
+        const GroupCost& t = g.cost[h][m];
+        const float shared = k < (float)g.resident[h] ? k : (float)g.resident[h];
+        offer(g.kind, 8, kLaunch + t.c * k + (t.a * (nsub + (rounds - 1.f) * mean) + t.b * mean * 0.5f * (wgs + k) + t.s * nsub * shared) / (float)g.gk);
     }
     if (tile.waves == 8 && (H > 64 || tile.nqb == 2)) {
         const float n = (float)ceil_div(L, tile.rows()), rows = (float)tile.rows();
@@ -558,11 +567,9 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
             chain *= ceil_f(n / (float)p.n_qtiles);       // a pair of tiles per workgroup
         }
         const Cost& t = !has_mask && use_tiles16(H, tile, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
-                                                                     : kCostTile[h][has_mask ? 2 : causal ? 1 : 0];
+                                                                     : kCostTile[h][m];
         const float rounds = ceil_f(u);
-        float us = kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds;
-        if (H == 64 && !has_mask && !causal && rounds == 1.f) us *= kLoneRoundTile;
-        offer(kTile, 8, us);
+        offer(kTile, 8, kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds);
     }
     return best;
 }

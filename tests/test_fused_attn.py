@@ -1045,13 +1045,13 @@ def _shape_on(kernel, H, mode, lengths, rows=None, fits=lambda v: True):
     raise AssertionError((kernel, H, mode, lengths, rows))
 
 
-@pytest.mark.parametrize("H", [16, 32, 64, 128])
+@pytest.mark.parametrize("H", [16, 32, 64])
 @pytest.mark.parametrize("residue", [0, 1, 4, 7])
 def test_masked_tile_kernel(gpu, H, residue):
-    # The tile kernel with an additive mask at every head_dim, with rows of any length: where L is no multiple
+    # The tile kernel with an additive mask (at head_dim 128 nothing runs on it), with rows of any length: where L is no multiple
     # of eight the last chunk of a row is fetched from where it still fits and shifted into place.  The
     # last nine keys carry most of the weight, and no two of them the same mask value.
-    B, R, L = _shape_on("tile", H, "mask", [8 * n + residue for n in (127, 191, 255, 320, 447, 511)])
+    B, R, L = _shape_on("tile", H, "mask", [8 * n + residue for n in (127, 191, 255, 320, 384, 447, 511)])
     dtype = torch.bfloat16 if (H // 16 + residue) % 2 else torch.float16
     q, k, v = (_rand((B, L, R * H), 5300 + L + i).to(dtype) for i in range(3))
     mask = _block_mask("blocks", B, L, 5310 + L).float()
@@ -1255,9 +1255,10 @@ def test_more_workgroups_than_one_grid_holds(gpu, B, R, mode):
     assert (lse - above - lse1[0, 0]).abs().max().item() <= 2.0 ** -10
 
 
-@pytest.mark.parametrize("kernel", ["split", "group", "tile"])
-@pytest.mark.parametrize("H,mode", [(16, "plain"), (32, "mask"), (64, "plain"), (64, "causal"), (64, "mask"),
-                                    (128, "plain"), (128, "causal"), (128, "mask")])
+@pytest.mark.parametrize("kernel,H,mode", [
+    (kernel, H, mode) for kernel in ("split", "group", "tile")
+    for H, mode in [(16, "plain"), (32, "mask"), (64, "plain"), (64, "causal"), (64, "mask"), (128, "plain"), (128, "causal"), (128, "mask")]
+    if (kernel, H, mode) != ("tile", 128, "mask")])              # (no masked problem runs there)
 @pytest.mark.parametrize("power,rise", [(100, 9.0), (100, 25.0), (100, 60.0), (-118, 25.0)])
 def test_bf16_values_at_the_ends_of_the_range(gpu, kernel, H, mode, power, rise):
     # Scores that rise by so many log2 units behind the first 256 keys leave the reference of the

@@ -7,10 +7,6 @@
 
 #include "../../include/fused_attn.h"
 
-#ifdef FA_TUNE
-#include <cstdio>
-#include <cstdlib>
-#endif
 #include <mutex>
 #include <utility>
 #include <vector>
@@ -27,15 +23,14 @@ struct Shape {
     int rows() const { return waves * 32 * nqb; }
 };
 
-// The tile kernels' shapes (fwd_kernel_pingpong, fwd_kernel_pp16), picked by how the problem's workgroups fill
-// the 256 compute units; pick_variant below then weighs that launch against the key-split and group
-// kernels, which take everything else:
+// The tile kernels' shapes (fwd_kernel_pingpong, fwd_kernel_pp16); pick_variant below weighs that launch, where
+// the problem fills the chip well enough for one, against the key-split and group kernels, which take
+// everything else:
 //   {8, 2}  eight 64-row waves share one K/V stream, 512 queries per workgroup, one resident per
-//           compute unit (head_dim <= 64 only: with head_dim 128 a 64-row wave would need the whole
+//           compute unit: head_dim <= 64 (with head_dim 128 a 64-row wave would need the whole
 //           register file of a SIMD);
-//   {8, 1}  the same with 32-row waves, 256 queries per workgroup: head_dim 128 (with head_dim <= 64 the
-//           group kernel is the faster one of the two on every grid);
-//   {4, 1}  too few workgroups of either: no tile kernel.
+//   {8, 1}  the same with 32-row waves, 256 queries per workgroup: head_dim 128, without additive mask;
+//   {0, 0}  no tile kernel.
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // How well a shape uses the chip, in 1/1024: the share of the (rounds x slots) grid of resident
@@ -110,47 +105,29 @@ CausalPlan plan_causal_walk(int64_t heads, int64_t n, int64_t H) {
 Shape pick_shape(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool mask_chunks,
                  bool causal) {
     const int64_t heads = B * R;
-    if (has_mask && !mask_chunks) return {4, 1};
-    // The ping-pong kernel is the fastest per compute unit, so it is taken whenever its
-    // workgroups fill the chip well enough.  Thresholds measured on MI355X: a lone round may be
-    // emptier than the tail of several, because idle units leave the busy ones more of the
-    // power budget.  A causal ping-pong workgroup takes two query tiles (see the kernel).
-    const int64_t tile8 = H > 64 ? 256 : 512;
-    const int64_t rows8 = tile8 * (causal ? 2 : 1);
-    const int64_t wgs8 = heads * ceil_div(L, rows8);
-    int64_t usage8 = usage(heads, L, rows8, kNumCu);
+    // head_dim 128 with a mask: the group kernel was the faster one on 843 of 861 random shapes, by up to 33 %,
+    // and at most 7 % slower on the others
+    if (has_mask && (!mask_chunks || H > 64)) return {0, 0};
+    // Taken into account when the workgroups fill the chip well enough: usage of 0.55 in a lone round, 0.7
+    // in a part-filled second round, 0.6 from two rounds on (a lone round may be emptier than the tail of
+    // several, because idle units leave the busy ones more of the power budget).  A causal workgroup
+    // takes two query tiles (see the kernel).
+    const Shape tile = H > 64 ? Shape{8, 1} : Shape{8, 2};
+    const int64_t rows = tile.rows() * (causal ? 2 : 1);
+    const int64_t wgs = heads * ceil_div(L, rows);
     if (causal) {
         // with the dealt schedule: useful key blocks over the blocks the 256 compute units are held for
-        const int64_t n = ceil_div(L, tile8);
+        const int64_t n = ceil_div(L, tile.rows());
         const CausalPlan plan = plan_causal(heads, n, H);
         if (plan.dealt) {
             const double held = (double)plan.blocks * kNumCu;
             const double useful = (double)heads * (double)n * (double)(n + 1) / 2.0;
-            const double rows_used = (double)L / ((double)n * (double)tile8);
-            if (1024.0 * useful / held * rows_used >= 614.0) return H > 64 ? Shape{8, 1} : Shape{8, 2};
+            const double rows_used = (double)L / ((double)n * (double)tile.rows());
+            if (1024.0 * useful / held * rows_used >= 614.0) return tile;
         }
     }
-    // Usage of 0.55 in a lone round, 0.7 in a part-filled second round, 0.6 from two rounds on.
-    const bool pingpong = wgs8 >= 2 * kNumCu ? usage8 >= 614 : usage8 >= (wgs8 <= kNumCu ? 560 : 717);
-    // 256-query workgroups with an additive mask: up to 30 % faster than the four-wave kernel,
-    // whose masked loop is not pipelined, from 160 workgroups on, unless a quarter or more of the
-    // query rows of a head's workgroups do not exist.
-    const int64_t per_head = ceil_div(L, 256);
-    const bool masked81 = has_mask && heads * per_head >= 160 && 4 * L >= 3 * per_head * 256;
-    if (H > 64) return pingpong || masked81 ? Shape{8, 1} : Shape{4, 1};
-    if (pingpong) return {8, 2};
-    // 256-query ping-pong workgroups.  Thresholds from sweeps of mid-size shapes on MI355X.
-    // Causal (a workgroup takes a pair of 256-query tiles, one resident per compute unit): 4 to
-    // 21 % faster than the four-wave kernel when the pairs fill 55 % or more of a single round,
-    // slower on emptier or on several rounds.
-    if (causal)
-        return heads * ceil_div(L, 512) <= kNumCu && usage(heads, L, 512, kNumCu) >= 560 ? Shape{8, 1} : Shape{4, 1};
-    // Additive mask: one resident per compute unit.
-    if (has_mask) return masked81 ? Shape{8, 1} : Shape{4, 1};
-    // Plain, two per compute unit: per compute unit they run at 0.93 of the 512-query ones and
-    // 1.1 to 1.25 times as fast as the four-wave kernel, but they need 160 or more workgroups to
-    // beat the latter's finer grain.
-    return heads * per_head >= 160 ? Shape{8, 1} : Shape{4, 1};
+    const int64_t used = usage(heads, L, rows, kNumCu);
+    return (wgs >= 2 * kNumCu ? used >= 614 : used >= (wgs <= kNumCu ? 560 : 717)) ? tile : Shape{0, 0};
 }
 
 // Dynamic LDS above 64 KiB has to be opted into per kernel function and per device: done on the
@@ -201,8 +178,8 @@ hipError_t launch_pingpong(const fa::FwdParams& p, hipStream_t stream) {
 // (head_dim 64: 144 pairs -4.3 %, 160 -6.2 %, 192 -1.4 and +1.3 %, 200 -0.6 %; 240 +3.6 %, 256
 // +5.5 %, 400 +1.4 %, 960 +4.5 and +7.5 %, 1152 +5.4 %, dealt +3.2 to +4.7 %; head_dim 128: 1024
 // pairs +5.1 and +5.4 %, dealt +4.2 %): taken from seven eighths of a round on.
-bool use_tiles16(int64_t H, Shape sh, const fa::FwdParams& p, bool causal) {
-    if (sh.waves != 8 || !((H == 64 && sh.nqb == 2) || H == 128)) return false;
+bool use_tiles16(int64_t H, const fa::FwdParams& p, bool causal) {
+    if (H < 64) return false;
     if (8 * (int64_t)p.total_wgs < 7 * kNumCu) return false;
     if (causal) return true;            // (a dealt launch is a whole resident grid)
     if (H == 64 && p.total_wgs < kNumCu) return false;     // (224 and 240 workgroups: +1.6 and +2.5 % at L = 4096, -1.4 % at L = 1024)
@@ -241,32 +218,30 @@ hipError_t launch_tiles16(int64_t H, int mode, bool bf16, const fa::FwdParams& p
 }
 
 template <int H, int MODE, bool BF>
-hipError_t dispatch_shape(Shape sh, const fa::FwdParams& p, hipStream_t stream) {
-    // the dealt causal schedule exists for the eight-wave kernel at head_dim 64 and 128 only
-    // (plan_causal never asks for it elsewhere)
-    constexpr int BASE = MODE == fa::kCausalDealt ? fa::kCausal : MODE;
-    if (MODE == fa::kCausalDealt && (sh.waves != 8 || H < 64)) return hipErrorInvalidValue;
-    // 64-row waves, at head_dim 128 32-row waves
-    if constexpr (H > 64)
-        return sh.waves == 8 ? launch_pingpong<H, 8, 1, 2, MODE, BF>(p, stream) : hipErrorInvalidValue;
+hipError_t dispatch_shape(const fa::FwdParams& p, hipStream_t stream) {
+    constexpr bool MASK = MODE == fa::kAdditive || MODE == fa::kAdditiveRagged;
+    // the dealt causal schedule exists at head_dim 64 and 128 only (plan_causal never asks for it elsewhere),
+    // and no masked launch at head_dim 128 (pick_shape)
+    if constexpr ((MODE == fa::kCausalDealt && H < 64) || (MASK && H > 64))
+        return hipErrorInvalidValue;
     else
-        return sh.waves == 8 && sh.nqb == 2 ? launch_pingpong<H, 8, 2, 2, H < 64 ? BASE : MODE, BF>(p, stream) : hipErrorInvalidValue;
+        return launch_pingpong<H, 8, (H > 64 ? 1 : 2), 2, MODE, BF>(p, stream);
 }
 
 template <int MODE, bool BF>
-hipError_t dispatch_head_dim(int64_t H, Shape sh, const fa::FwdParams& p, hipStream_t stream) {
+hipError_t dispatch_head_dim(int64_t H, const fa::FwdParams& p, hipStream_t stream) {
     switch (H) {
-        case 16: return dispatch_shape<16, MODE, BF>(sh, p, stream);
-        case 32: return dispatch_shape<32, MODE, BF>(sh, p, stream);
-        case 64: return dispatch_shape<64, MODE, BF>(sh, p, stream);
-        case 128: return dispatch_shape<128, MODE, BF>(sh, p, stream);
+        case 16: return dispatch_shape<16, MODE, BF>(p, stream);
+        case 32: return dispatch_shape<32, MODE, BF>(p, stream);
+        case 64: return dispatch_shape<64, MODE, BF>(p, stream);
+        case 128: return dispatch_shape<128, MODE, BF>(p, stream);
         default: return hipErrorInvalidValue;
     }
 }
 
 template <int MODE>
-hipError_t dispatch(int64_t H, Shape sh, const fa::FwdParams& p, hipStream_t stream, bool bf16) {
-    return bf16 ? dispatch_head_dim<MODE, true>(H, sh, p, stream) : dispatch_head_dim<MODE, false>(H, sh, p, stream);
+hipError_t dispatch(int64_t H, const fa::FwdParams& p, hipStream_t stream, bool bf16) {
+    return bf16 ? dispatch_head_dim<MODE, true>(H, p, stream) : dispatch_head_dim<MODE, false>(H, p, stream);
 }
 
 // Which kernel runs a problem: a tile kernel (the launch of pick_shape), the key-split kernel (`waves` share out
@@ -309,13 +284,20 @@ hipError_t launch_group(const fa::FwdParams& p, hipStream_t stream) {
     return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(p.wgs_per_xcd * fa::kNumXcd), dim3(8 * 64), args, lds, stream);
 }
 
+// 32 rows per wave at head_dim 128: without mask and causal flag only (with one of them it was the fastest kernel
+// on none of 2100 random shapes)
+template <int H, int MODE>
+constexpr bool group21_offered() { return H <= 64 || MODE == fa::kPlain; }
+
 template <int H, int MODE, bool BF>
 hipError_t dispatch_variant(const Variant& v, const fa::FwdParams& p, hipStream_t stream) {
     switch (v.kind) {
         case kSplit: return launch_split<H, MODE, BF>(p, stream);
         case kGroup11: return launch_group<H, 1, 1, MODE, BF>(p, stream);
         case kGroup12: return launch_group<H, 1, 2, MODE, BF>(p, stream);
-        case kGroup21: return launch_group<H, 2, 1, MODE, BF>(p, stream);
+        case kGroup21:
+            if constexpr (group21_offered<H, MODE>()) return launch_group<H, 2, 1, MODE, BF>(p, stream);
+            return hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }
@@ -375,26 +357,26 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
     if (stride_l > ((int64_t)1 << 24)) return FA_ERR_TOO_LARGE;
     *shape = pick_shape(B, R, L, H, mask != nullptr,
                         L >= 8 && L <= ((int64_t)1 << 24), causal);
-    const int64_t bq = shape->rows();
-    int64_t n_qtiles = (L + bq - 1) / bq;
-    int64_t total = 0;
+    int64_t n_qtiles = 0, total = 0;       // (no tile kernel: use_variant fills in the launch)
     p->heads_per_xcd = 0;
-    if (causal && shape->waves == 8) {
-        const CausalPlan plan = plan_causal(B * R, n_qtiles, H);
-        n_qtiles = (n_qtiles + 1) / 2;                                // pairs of query tiles
-        if (plan.dealt) {
-            p->heads_per_xcd = (int)(B * R / fa::kNumXcd);
-            total = kNumCu;                                           // a resident grid
+    if (shape->waves != 0) {
+        n_qtiles = ceil_div(L, shape->rows());
+        // Pairs of query tiles for causal launches, and for masked ones (see the kernel) when the pairs, two tiles
+        // long, need no more time on the chip than the tiles in rounds of their own
+        const int64_t pairs = ceil_div(n_qtiles, 2);
+        if (causal) {
+            const CausalPlan plan = plan_causal(B * R, n_qtiles, H);
+            n_qtiles = pairs;
+            if (plan.dealt) {
+                p->heads_per_xcd = (int)(B * R / fa::kNumXcd);
+                total = kNumCu;                                       // a resident grid
+            }
+        } else if (mask != nullptr && 2 * ceil_div(B * R * pairs, kNumCu) <= ceil_div(B * R * n_qtiles, kNumCu)) {
+            n_qtiles = pairs;
         }
+        if (total == 0) total = B * R * n_qtiles;
+        if (total > kMaxInt - 8) return FA_ERR_TOO_LARGE;
     }
-    if (mask != nullptr && shape->waves == 8 && n_qtiles > 1) {
-        // Pairs of query tiles for a masked launch of the eight-wave kernel (see the kernel) when the
-        // pairs, two tiles long, need no more time on the chip than the tiles in rounds of their own
-        const int64_t pairs = (n_qtiles + 1) / 2;
-        if (2 * ceil_div(B * R * pairs, kNumCu) <= ceil_div(B * R * n_qtiles, kNumCu)) n_qtiles = pairs;
-    }
-    if (total == 0) total = B * R * n_qtiles;
-    if (total > kMaxInt - 8 || B * R > kMaxInt) return FA_ERR_TOO_LARGE;
     if (!extent_ok(in, B, R, L) || !extent_ok(os, B, R, L)) return FA_ERR_TOO_LARGE;
 
     p->q = static_cast<const _Float16*>(q);
@@ -480,7 +462,7 @@ constexpr GroupCost kCostGroup21[4][3] = {
     {{0.191f, 0.192f, 0.068f, 0.687f}, {0.243f, 0.209f, 0.0796f, 0.144f}, {0.372f, 0.323f, 0.0533f, 1.22f}},
     {{0.197f, 0.221f, 0.0518f, 0.616f}, {0.278f, 0.203f, 0.0567f, 0.147f}, {0.388f, 0.332f, 0.0549f, 1.23f}},
     {{0.27f, 0.35f, 0.044f, 1.25f}, {0.344f, 0.369f, 0.0525f, 0.269f}, {0.515f, 0.42f, 0.0741f, 1.7f}},
-    {{0.56f, 0.492f, 0.00712f, 2.09f}, {0.489f, 0.627f, 0.f, 1.34f}, {0.712f, 0.567f, 0.f, 3.03f}},
+    {{0.56f, 0.492f, 0.00712f, 2.09f}, {}, {}},
 };
 
 struct GroupShape {
@@ -502,7 +484,7 @@ constexpr Cost kCostTile[4][3] = {       // [head_dim][plain, causal, mask], fwd
     {{0.536f, 0.0518f, 2.81f}, {0.614f, 0.0242f, 7.91f}, {0.825f, 0.136f, 5.06f}},
     {{0.498f, 0.137f, 2.57f}, {0.599f, 0.0832f, 8.89f}, {0.811f, 0.27f, 3.73f}},
     {{0.469f, 0.459f, 4.44f}, {0.654f, 0.147f, 11.4f}, {1.07f, 0.294f, 7.86f}},
-    {{0.297f, 0.6f, 5.26f}, {0.505f, 0.287f, 15.2f}, {0.952f, 0.288f, 6.73f}},
+    {{0.297f, 0.6f, 5.26f}, {0.505f, 0.287f, 15.2f}, {}},
 };
 constexpr Cost kCostTile16[2][2] = {     // [head_dim 64, 128][plain, causal], fwd_kernel_pp16
     {{0.508f, 0.362f, 7.63f}, {0.0783f, 0.851f, 10.1f}},
@@ -517,15 +499,6 @@ float ceil_f(float x) {
 // `tile` and `p` hold the launch of the tile kernels (validate).
 Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool causal, const Shape& tile,
                      const fa::FwdParams& p) {
-#ifdef FA_TUNE
-    const char* env = getenv("FA_SPLIT");
-    if (env != nullptr) {
-        int nq = 0, nw = 0;
-        sscanf(env, "%d,%d", &nq, &nw);
-        if (nq == 0) return tile.waves == 8 && (H > 64 || tile.nqb == 2) ? Variant{kTile, 8} : Variant{kGroup11, 8};
-        return nw < 10 ? Variant{kSplit, nw} : Variant{nq == 2 ? kGroup21 : nw == 11 ? kGroup11 : kGroup12, 8};
-    }
-#endif
     const int h = H == 16 ? 0 : H == 32 ? 1 : H == 64 ? 2 : 3;
     const int m = has_mask ? 2 : causal ? 1 : 0;
     const float heads = (float)(B * R), nsub = (float)ceil_div(L, 32);
@@ -547,6 +520,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         }
     }
     for (const GroupShape& g : kGroups) {
+        if (g.nq == 2 && H == 128 && m != 0) continue;         // (group21_offered)
         const int rows = 16 * g.nq * (8 / g.gk);
         const float wgs = heads * (float)ceil_div(L, rows) / kNumCu, k = ceil_f(wgs);
         const float mean = causal ? 0.5f * (nsub + (float)rows / 32.f) : nsub;
@@ -555,7 +529,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         const float shared = k < (float)g.resident[h] ? k : (float)g.resident[h];
         offer(g.kind, 8, kLaunch + t.c * k + (t.a * (nsub + (rounds - 1.f) * mean) + t.b * mean * 0.5f * (wgs + k) + t.s * nsub * shared) / (float)g.gk);
     }
-    if (tile.waves == 8 && (H > 64 || tile.nqb == 2)) {
+    if (tile.waves != 0) {
         const float n = (float)ceil_div(L, tile.rows()), rows = (float)tile.rows();
         float chain = nsub, u = (float)p.total_wgs / kNumCu;
         if (causal && p.heads_per_xcd > 0) {
@@ -566,7 +540,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         } else {
             chain *= ceil_f(n / (float)p.n_qtiles);       // a pair of tiles per workgroup
         }
-        const Cost& t = !has_mask && use_tiles16(H, tile, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
+        const Cost& t = !has_mask && use_tiles16(H, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
                                                                      : kCostTile[h][m];
         const float rounds = ceil_f(u);
         offer(kTile, 8, kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds);
@@ -584,8 +558,23 @@ int use_variant(const Variant& v, fa::FwdParams* p) {
     p->n_qtiles = (int)per_head;
     p->total_wgs = (int)total;
     p->wgs_per_xcd = (int)ceil_div(total, fa::kNumXcd);
+    p->heads_per_xcd = 0;
     p->waves = v.waves;
     return FA_OK;
+}
+
+// The launch fa_fwd makes for a problem on dense tensors, without making it.
+int describe_launch(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_mask, Shape* shape, Variant* v, fa::FwdParams* p) {
+    if ((flags & ~(FA_FLAG_CAUSAL | FA_FLAG_BF16)) != 0) return FA_ERR_BAD_FLAGS;
+    const bool causal = (flags & FA_FLAG_CAUSAL) != 0;
+    if (causal && has_mask) return FA_ERR_BAD_FLAGS;
+    // validate() only looks at the pointers' alignment
+    void* const fake = reinterpret_cast<void*>(static_cast<uintptr_t>(4096));
+    const Strides dense{L * R * H, H, R * H};
+    const int rc = validate(fake, fake, fake, has_mask ? fake : nullptr, fake, B, R, L, H, dense, dense, p, 1.0f, shape, causal, nullptr);
+    if (rc != FA_OK) return rc;
+    *v = pick_variant(B, R, L, H, has_mask != 0, causal, *shape, *p);
+    return v->kind != kTile ? use_variant(*v, p) : FA_OK;
 }
 
 }  // namespace
@@ -631,7 +620,7 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     if (causal && mask != nullptr) return FA_ERR_BAD_FLAGS;
     if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return FA_ERR_MISALIGNED;
     fa::FwdParams p;
-    Shape shape{4, 2};
+    Shape shape{0, 0};
     const int rc = validate(q, k, v, mask, out, B, R, L, H, Strides{stride_b, stride_h, stride_l},
                             Strides{out_stride_b, out_stride_h, out_stride_l}, &p, scale, &shape, causal, lse);
     if (rc != FA_OK) return rc;
@@ -659,70 +648,52 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     if (variant.kind != kTile) {
         const int mode = causal ? fa::kCausal : mask != nullptr ? fa::kAdditive : fa::kPlain;
         e = bf16 ? dispatch_variant_mode<true>(H, mode, variant, p, s) : dispatch_variant_mode<false>(H, mode, variant, p, s);
-    } else if (mask == nullptr && use_tiles16(H, shape, p, causal))
+    } else if (mask == nullptr && use_tiles16(H, p, causal))
         e = launch_tiles16(H, causal ? (p.heads_per_xcd > 0 ? fa::kCausalDealt : fa::kCausal) : fa::kPlain, bf16, p, s);
     else if (causal && p.heads_per_xcd > 0)
-        e = dispatch<fa::kCausalDealt>(H, shape, p, s, bf16);
+        e = dispatch<fa::kCausalDealt>(H, p, s, bf16);
     else if (causal)
-        e = dispatch<fa::kCausal>(H, shape, p, s, bf16);
+        e = dispatch<fa::kCausal>(H, p, s, bf16);
     else if (mask != nullptr && L % 8 != 0)
-        e = dispatch<fa::kAdditiveRagged>(H, shape, p, s, bf16);
+        e = dispatch<fa::kAdditiveRagged>(H, p, s, bf16);
     else if (mask != nullptr)
-        e = dispatch<fa::kAdditive>(H, shape, p, s, bf16);
+        e = dispatch<fa::kAdditive>(H, p, s, bf16);
     else
-        e = dispatch<fa::kPlain>(H, shape, p, s, bf16);
+        e = dispatch<fa::kPlain>(H, p, s, bf16);
     return static_cast<int>(e);
 }
 
 int fa_fwd_plan(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_mask, int* plan) {
     if (plan == nullptr) return FA_ERR_NULL_POINTER;
-    if ((flags & ~(FA_FLAG_CAUSAL | FA_FLAG_BF16)) != 0) return FA_ERR_BAD_FLAGS;
-    const bool causal = (flags & FA_FLAG_CAUSAL) != 0;
-    if (causal && has_mask) return FA_ERR_BAD_FLAGS;
-    // validate() only looks at the pointers' alignment
-    void* const fake = reinterpret_cast<void*>(static_cast<uintptr_t>(4096));
     fa::FwdParams p;
-    Shape shape{4, 1};
-    const Strides dense{L * R * H, H, R * H};
-    const int rc = validate(fake, fake, fake, has_mask ? fake : nullptr, fake, B, R, L, H, dense, dense, &p, 1.0f,
-                            &shape, causal, nullptr);
+    Shape shape{0, 0};
+    Variant v{kTile, 0};
+    const int rc = describe_launch(B, R, L, H, flags, has_mask, &shape, &v, &p);
     if (rc != FA_OK) return rc;
-    plan[0] = shape.waves;
-    plan[1] = 32 * shape.nqb;
+    const bool tile = v.kind == kTile;
+    plan[0] = v.waves;
+    plan[1] = tile ? 32 * shape.nqb : v.kind == kGroup21 ? 32 : 16;
     plan[2] = p.wgs_per_xcd * fa::kNumXcd;
     plan[3] = p.total_wgs;
     plan[4] = p.n_qtiles;
     plan[5] = p.heads_per_xcd;
-    plan[6] = (!has_mask && use_tiles16(H, shape, p, causal)) ? 16 : 32;
+    plan[6] = !tile || (!has_mask && use_tiles16(H, p, (flags & FA_FLAG_CAUSAL) != 0)) ? 16 : 32;
     return FA_OK;
 }
 
 int fa_fwd_variant(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_mask, int* variant) {
     if (variant == nullptr) return FA_ERR_NULL_POINTER;
-    if ((flags & ~(FA_FLAG_CAUSAL | FA_FLAG_BF16)) != 0) return FA_ERR_BAD_FLAGS;
-    const bool causal = (flags & FA_FLAG_CAUSAL) != 0;
-    if (causal && has_mask) return FA_ERR_BAD_FLAGS;
-    void* const fake = reinterpret_cast<void*>(static_cast<uintptr_t>(4096));
     fa::FwdParams p;
-    Shape shape{4, 1};
-    const Strides dense{L * R * H, H, R * H};
-    int rc = validate(fake, fake, fake, has_mask ? fake : nullptr, fake, B, R, L, H, dense, dense, &p, 1.0f, &shape, causal, nullptr);
+    Shape shape{0, 0};
+    Variant v{kTile, 0};
+    const int rc = describe_launch(B, R, L, H, flags, has_mask, &shape, &v, &p);
     if (rc != FA_OK) return rc;
-    const Variant v = pick_variant(B, R, L, H, has_mask != 0, causal, shape, p);
-    int rows = shape.rows(), groups = 1;
-    if (v.kind == kSplit) {
-        rows = 16;
-        groups = v.waves;
-    }
+    int rows = v.kind == kTile ? shape.rows() : 16, groups = v.kind == kSplit ? v.waves : 1;
     for (const GroupShape& g : kGroups)
         if (g.kind == v.kind) {
             rows = 16 * g.nq * (8 / g.gk);
             groups = g.gk;
         }
-    if (v.kind != kTile) {
-        rc = use_variant(v, &p);
-        if (rc != FA_OK) return rc;
-    }
     variant[0] = v.kind == kTile ? 0 : v.kind == kSplit ? 1 : 2;
     variant[1] = v.waves;
     variant[2] = rows;
@@ -890,10 +861,6 @@ constexpr QkvCost kQkvCost[kQkvKinds] = {
 };
 
 QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
-#ifdef FA_TUNE
-    const char* env = getenv("FA_QKV");
-    if (env != nullptr) return (QkvKind)atoi(env);
-#endif
     QkvKind best = kQkvWhole;
     float least = 3.0e38f;
     const float slices = (float)(K / fa::qkv::kTileK);

@@ -106,17 +106,16 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
                    float scale, int flags, void* stream);
 
 /*
- * The launch of the eight-wave tile kernels for a problem, without making it (no GPU is touched): for
- * tests of the launcher and for tuning.  fa_fwd_variant says whether they or another kernel run it.
- * has_mask != 0 stands for an additive mask.  Fills plan[0..6] with: wave64s per workgroup (4: the problem
- * has too few workgroups for a tile kernel, and another one runs it); query rows per wave; workgroups
- * launched; workgroups that do work (the rest exit at once); workgroups per (batch, head), or
- * pairs of query tiles per head for a causal launch of the eight-wave kernel and for those masked
- * launches of it that pairs cost no round of the chip; 0, or, when the
- * query tiles of a causal launch are dealt out to a resident grid, the heads per XCD; the edge of
- * the matrix instruction's tile, 32, or 16 at head_dim 64 and 128 for plain launches of the eight-wave
- * kernel whose workgroups fill whole rounds of the chip (the last round at least seven eighths full)
- * and for its causal launches from seven eighths of a round on.
+ * The launch the library would make for a problem, without making it (no GPU is touched): for
+ * tests of the launcher and for tuning.  has_mask != 0 stands for an additive mask.  Fills plan[0..6]
+ * with: wave64s per workgroup; query rows per wave (waves may share them, see fa_fwd_variant);
+ * workgroups launched; workgroups that do work (the rest exit at once); workgroups per (batch, head),
+ * or pairs of query tiles per head for a causal launch of a tile kernel and for those masked
+ * launches of one that pairs cost no round of the chip; 0, or, when the query tiles of a causal launch
+ * are dealt out to a resident grid, the heads per XCD; the edge of the matrix instruction's tile: 16,
+ * or, in a tile kernel, 32 except at head_dim 64 and 128 for plain launches whose workgroups fill whole
+ * rounds of the chip (the last round at least seven eighths full) and for causal launches from seven
+ * eighths of a round on.
  * (A problem whose grid would have 2^32 threads or more is launched in parts, halves of its batch or heads.)
  * The reference has no counterpart (its grid is fixed at (B, L / chunk_size, R),
  * reference include/fused_attn.cuh:872-883).
@@ -125,8 +124,7 @@ int fa_fwd_plan(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_m
 
 /*
  * Which kernel fa_fwd runs a problem on, without running it (no GPU is touched), has_mask as in fa_fwd_plan.
- * Fills variant[0..6] with: 0 = a tile kernel (fa_fwd_plan has its launch), 1 = the key-split kernel, 2 = the
- * group kernel; waves per workgroup; query rows per workgroup; waves that share a row's keys between
+ * Fills variant[0..6] with: 0 = a tile kernel, 1 = the key-split kernel, 2 = the group kernel; waves per workgroup; query rows per workgroup; waves that share a row's keys between
  * them; workgroups launched; workgroups that do work; workgroups per (batch, head) (pairs of query
  * tiles where fa_fwd_plan says so).  No counterpart in the reference (see fa_fwd_plan).
  */

@@ -73,11 +73,10 @@ def test_status_codes_for_rejected_arguments():
     assert capi.strerror(0) == "success"
 
 
-def _items_of_plan(plan, heads, L, causal):
+def _items_of_plan(plan, variant, heads, L, causal):
     """Replays how the kernels turn a workgroup index into (head, query tile) items
-    (fwd_kernel and fwd_kernel_pingpong in fused_attn_kernel_impl.inc) for a launch plan."""
-    rows = plan["waves"] * plan["rows_per_wave"]
-    tiles = -(-L // rows)
+    (fused_attn_kernel_impl.inc, fused_attn_split.inc) for a launch plan."""
+    tiles = -(-L // variant["rows"])
     per_xcd = plan["workgroups"] // 8
     items = []
     for wg in range(plan["workgroups"]):
@@ -92,7 +91,7 @@ def _items_of_plan(plan, heads, L, causal):
                     break
                 items.append((wg % 8 + 8 * (j % plan["heads_per_xcd"]), tiles - 1 - j // plan["heads_per_xcd"]))
                 rnd += 1
-        elif plan["waves"] == 8 and (causal or plan["per_head"] < tiles):   # a pair of tiles per workgroup (causal; some masked launches)
+        elif variant["kernel"] == "tile" and (causal or plan["per_head"] < tiles):   # a pair of tiles per workgroup (causal; some masked launches)
             head, slot = divmod(logical, plan["per_head"])
             items.append((head, tiles - 1 - slot))
             if 2 * slot != tiles - 1:
@@ -120,19 +119,26 @@ def test_every_launch_plan_covers_every_query_tile_once():
         heads = rng.choice([1, 3, 8, 12, 16, 20, 24, 40, 48, 64, 80, 96, 120, 160, 256, 320, 640])
         B = rng.choice([b for b in (1, 2, 4, 8) if heads % b == 0])
         shapes.append((B, heads // B, L, H))
+    for _ in range(60):                     # where the masked tile kernel runs, in pairs of tiles
+        shapes.append((1, rng.randint(230, 256), 8 * rng.randint(108, 128), rng.choice([16, 32, 64])))
     dealt = paired_masks = 0
     for B, R, L, H in shapes:
         for causal, has_mask in ((False, False), (True, False), (False, True)):
             if has_mask and L % 8:
                 continue
             plan = capi.launch_plan(B, R, L, H, causal=causal, has_mask=has_mask)
-            assert plan["waves"] in (4, 8) and plan["rows_per_wave"] in (32, 64) and plan["workgroups"] % 8 == 0
-            assert plan["heads_per_xcd"] == 0 or (causal and plan["waves"] == 8 and H >= 64 and (B * R) % 8 == 0)
-            items, tiles = _items_of_plan(plan, B * R, L, causal)
+            variant = capi.launch_variant(B, R, L, H, causal=causal, has_mask=has_mask)
+            tile = variant["kernel"] == "tile"
+            assert all(plan[key] == variant[key] for key in ("waves", "workgroups", "working", "per_head"))
+            assert plan["waves"] * plan["rows_per_wave"] == variant["rows"] * variant["key_groups"] and plan["workgroups"] % 8 == 0
+            assert (plan["waves"], plan["rows_per_wave"]) in ([(8, 32 if H == 128 else 64)] if tile else [(2, 16), (4, 16), (8, 16), (8, 32)])
+            assert plan["matrix_tile"] == 16 or (tile and plan["matrix_tile"] == 32)
+            assert plan["heads_per_xcd"] == 0 or (causal and tile and H >= 64 and (B * R) % 8 == 0)
+            items, tiles = _items_of_plan(plan, variant, B * R, L, causal)
             assert len(items) == B * R * tiles, (B, R, L, H, causal, has_mask, plan)
             assert set(items) == {(h, t) for h in range(B * R) for t in range(tiles)}, (B, R, L, H, causal, has_mask, plan)
             dealt += plan["heads_per_xcd"] > 0
-            paired_masks += has_mask and plan["waves"] == 8 and plan["per_head"] < tiles
+            paired_masks += has_mask and tile and plan["per_head"] < tiles
             if not causal and not has_mask:
                 assert plan["per_head"] == tiles
     assert dealt > 10          # the dealt schedule was among the plans
@@ -244,56 +250,60 @@ def test_projection_grids_stay_below_2_to_the_32_threads():
 
 def test_benchmark_workloads_take_the_kernels_the_documentation_names():
     def plan(B, R, L, H, **kw):
-        p = capi.launch_plan(B, R, L, H, **kw)
-        return p["waves"], p["rows_per_wave"], p["heads_per_xcd"] > 0
+        p, v = capi.launch_plan(B, R, L, H, **kw), capi.launch_variant(B, R, L, H, **kw)
+        return v["kernel"], p["waves"], p["rows_per_wave"], v["key_groups"], p["heads_per_xcd"] > 0
 
-    assert plan(4, 16, 4096, 64) == (8, 64, False)                       # c3: 512 workgroups of 512 queries
-    assert plan(1, 32, 16384, 128) == (8, 32, False)                     # c4
-    assert plan(4, 40, 2048, 128) == (8, 32, False)                      # README shape
-    assert plan(8, 12, 1024, 64) == (8, 64, False)                       # c2
-    assert plan(2, 8, 3073, 64) == (8, 32, False)                        # c5b: 256-query workgroups
-    assert plan(1, 4, 256, 64) == (4, 32, False)                         # c1
-    assert plan(2, 8, 1000, 64) == (4, 32, False)                        # c5a
-    assert plan(4, 16, 4096, 64, causal=True) == (8, 64, False)          # one whole round of pairs
-    assert plan(1, 32, 16384, 128, causal=True) == (8, 32, False)        # four whole rounds of pairs
-    assert plan(4, 40, 2048, 128, causal=True) == (8, 32, True)          # 2.5 rounds of pairs: dealt
-    assert plan(2, 40, 4096, 64, causal=True) == (8, 64, True)
-    assert plan(2, 48, 5000, 32, causal=True) == (8, 64, False)          # never dealt below head_dim 64
-    assert plan(8, 12, 1024, 64, causal=True)[:2] == (8, 32)             # pairs of 256-query tiles
-    assert plan(2, 12, 2048, 64, causal=True) == (4, 32, False)
-    assert plan(4, 16, 4096, 64, has_mask=True) == (8, 64, False)
-    assert plan(1, 40, 2048, 128, has_mask=True) == (8, 32, False)
-    assert plan(2, 12, 2048, 64, has_mask=True) == (8, 32, False)
-    assert plan(64, 12, 128, 64, has_mask=True) == (4, 32, False)
+    assert plan(4, 16, 4096, 64) == ("tile", 8, 64, 1, False)                    # c3: 512 workgroups of 512 queries
+    assert plan(1, 32, 16384, 128) == ("tile", 8, 32, 1, False)                  # c4
+    assert plan(4, 40, 2048, 128) == ("tile", 8, 32, 1, False)                   # README shape
+    assert plan(8, 12, 1024, 64) == ("tile", 8, 64, 1, False)                    # c2
+    assert plan(2, 8, 3073, 64) == ("group", 8, 16, 1, False)                    # c5b: 400 workgroups of 128 queries
+    assert plan(1, 4, 256, 64) == ("split", 4, 16, 4, False)                     # c1
+    assert plan(2, 8, 1000, 64) == ("group", 8, 16, 2, False)                    # c5a: 256 workgroups of 64 queries
+    assert plan(4, 16, 4096, 64, causal=True) == ("tile", 8, 64, 1, False)       # one whole round of pairs
+    assert plan(1, 32, 16384, 128, causal=True) == ("tile", 8, 32, 1, False)     # four whole rounds of pairs
+    assert plan(4, 40, 2048, 128, causal=True) == ("tile", 8, 32, 1, True)       # 2.5 rounds of pairs: dealt
+    assert plan(2, 40, 4096, 64, causal=True) == ("tile", 8, 64, 1, True)
+    assert plan(2, 48, 5000, 32, causal=True)[4] is False                        # never dealt below head_dim 64
+    assert plan(8, 12, 1024, 64, causal=True) == ("group", 8, 16, 1, False)
+    assert plan(2, 12, 2048, 64, causal=True) == ("group", 8, 16, 2, False)
+    assert plan(4, 16, 4096, 64, has_mask=True) == ("tile", 8, 64, 1, False)
+    assert plan(1, 40, 2048, 128, has_mask=True)[0] == "group"                   # head_dim 128 with a mask: never a tile kernel
+    assert plan(2, 12, 2048, 64, has_mask=True) == ("group", 8, 16, 2, False)
+    assert plan(64, 12, 128, 64, has_mask=True) == ("group", 8, 16, 1, False)
 
 
 def test_the_16_row_matrix_tile_is_taken_on_whole_rounds_only():
-    tile = lambda B, R, L, H, **kw: capi.launch_plan(B, R, L, H, **kw)["matrix_tile"]
+    def tile(B, R, L, H, **kw):
+        if H != 128 or not kw.get("has_mask"):            # (the group kernel, whose matrix tile is 16 everywhere)
+            assert capi.launch_variant(B, R, L, H, **kw)["kernel"] == "tile"
+        return capi.launch_plan(B, R, L, H, **kw)["matrix_tile"]
+
     wgs = lambda B, R, L, H: capi.launch_plan(B, R, L, H)["working"]
     assert (wgs(4, 16, 4096, 64), tile(4, 16, 4096, 64)) == (512, 16)     # c3: two whole rounds
     assert (wgs(4, 16, 2048, 64), tile(4, 16, 2048, 64)) == (256, 16)     # one whole round
-    assert (wgs(8, 32, 1000, 64), tile(8, 32, 1000, 64)) == (512, 16)     # ragged tiles make no difference
+    assert (wgs(8, 16, 2011, 64), tile(8, 16, 2011, 64)) == (512, 16)     # ragged tiles make no difference
     assert (wgs(2, 60, 2048, 64), tile(2, 60, 2048, 64)) == (480, 16)     # last round seven eighths full
     assert (wgs(2, 56, 2048, 64), tile(2, 56, 2048, 64)) == (448, 32)     # ... three quarters full
-    assert (wgs(6, 16, 2048, 64), tile(6, 16, 2048, 64)) == (384, 32)     # one and a half rounds
+    assert (wgs(3, 16, 4096, 64), tile(3, 16, 4096, 64)) == (384, 32)     # one and a half rounds
     assert (wgs(9, 16, 4096, 64), tile(9, 16, 4096, 64)) == (1152, 32)    # four and a half
     assert (wgs(8, 12, 1024, 64), tile(8, 12, 1024, 64)) == (192, 32)     # c2: less than one round
     assert tile(4, 16, 4096, 64, causal=True) == 16                       # causal: whole rounds of pairs of tiles
-    assert tile(2, 85, 2500, 64, causal=True) == 16                       # ... 510 pairs and lone middle tiles
-    assert tile(2, 64, 1300, 64, causal=True) == 16                       # ... and where the tiles are dealt out to a resident grid
-    assert tile(3, 12, 4096, 64, causal=True) == 32                       # 144 pairs: little more than half a round
+    assert tile(2, 51, 4500, 64, causal=True) == 16                       # ... 510 pairs and lone middle tiles
+    assert tile(2, 64, 2500, 64, causal=True) == 16                       # ... and where the tiles are dealt out to a resident grid
+    assert tile(1, 12, 12288, 64, causal=True) == 32                      # 144 pairs: little more than half a round
     assert tile(3, 20, 4096, 64, causal=True) == 16                       # 240 pairs: causal launches from 7/8 of a round on,
     assert tile(5, 20, 4096, 64, causal=True) == 16                       # ... whatever the last round holds (400 pairs)
     assert tile(5, 20, 2048, 64, causal=True) == 32                       # 200 pairs
     assert tile(4, 16, 4096, 64, has_mask=True) == 32                     # never with a mask
-    assert tile(4, 32, 4096, 32) == 32 and tile(16, 16, 4096, 16) == 32   # head_dim 64 and 128 only
+    assert tile(4, 32, 4096, 32) == 32 and tile(4, 32, 4096, 16) == 32    # head_dim 64 and 128 only
     assert (wgs(1, 32, 16384, 128), tile(1, 32, 16384, 128)) == (2048, 16)    # c4: eight rounds of 256-query workgroups
     assert (wgs(4, 40, 2048, 128), tile(4, 40, 2048, 128)) == (1280, 16)      # the reference's benchmark shape: five rounds
     assert (wgs(1, 28, 2048, 128), tile(1, 28, 2048, 128)) == (224, 16)       # seven eighths of a round
     assert (wgs(1, 48, 2048, 128), tile(1, 48, 2048, 128)) == (384, 32)       # one and a half rounds
     assert (wgs(1, 24, 2048, 128), tile(1, 24, 2048, 128)) == (192, 32)
     assert tile(1, 32, 16384, 128, causal=True) == 16 and tile(4, 40, 2048, 128, causal=True) == 16   # pairs; dealt
-    assert tile(4, 40, 2048, 128, has_mask=True) == 32
+    assert tile(4, 40, 2048, 128, has_mask=True) == 16                        # with a mask the group kernel
 
 
 def test_missing_library_fails_loudly(monkeypatch):

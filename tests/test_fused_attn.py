@@ -1069,8 +1069,8 @@ def test_masked_tile_kernel(gpu, H, residue):
         assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
 
 
-# One shape or two per kernel and head_dim, at the edges of their tiles: 16, 64, 128 and 256 query rows, 32 keys
-# per sub-tile, 64 keys per key tile and three key tiles per turn of the ring.
+# One shape or two per kernel and head_dim, at the edges of their tiles: 16, 64 and 128 query rows (256: LAUNCHES
+# below), 32 keys per sub-tile, 64 keys per key tile and three key tiles per turn of the ring.
 SMALL_GRIDS = [(1, 1, 1), (2, 3, 17), (1, 5, 33), (2, 4, 129), (1, 3, 300), (3, 40, 130), (2, 40, 255), (2, 16, 513),
                (8, 40, 129), (2, 12, 1217), (9, 20, 705)]
 
@@ -1226,6 +1226,51 @@ def test_bf16_additive_mask_and_closed_forms(gpu, B, R, L, H):
     assert _max_err(zq, want) <= 2e-3
     with pytest.raises(TypeError):
         capi.forward(q.to(gpu), k.half().to(gpu), v.to(gpu), H)
+
+
+# One problem, nearly always of a ragged length, for every launch the other tests do not reach: kernel, query rows per
+# workgroup, edge of the matrix tile, and whether the tiles of a causal launch are dealt out.
+LAUNCHES = [
+    ("group", 256, 16, False, 16, "causal", 2, 117, 180), ("group", 256, 16, False, 16, "mask", 1, 454, 151),
+    ("group", 256, 16, False, 16, "plain", 2, 118, 129), ("group", 256, 16, False, 32, "causal", 2, 193, 135),
+    ("group", 256, 16, False, 32, "mask", 1, 437, 131), ("group", 256, 16, False, 32, "plain", 1, 176, 129),
+    ("group", 256, 16, False, 64, "causal", 1, 408, 132), ("group", 256, 16, False, 64, "mask", 1, 390, 129),
+    ("group", 256, 16, False, 64, "plain", 2, 206, 130), ("group", 256, 16, False, 128, "plain", 2, 108, 131),
+    ("group", 64, 16, False, 16, "mask", 1, 220, 50), ("group", 64, 16, False, 32, "mask", 1, 238, 33),
+    ("tile", 512, 32, False, 16, "plain", 1, 235, 390), ("tile", 512, 32, False, 32, "plain", 2, 125, 387),
+    ("tile", 512, 32, False, 64, "plain", 1, 204, 391), ("tile", 512, 16, False, 64, "plain", 2, 32, 1671),
+    ("tile", 256, 32, False, 128, "plain", 2, 42, 434), ("tile", 256, 16, False, 128, "plain", 1, 77, 655),
+    ("tile", 512, 32, False, 16, "causal", 1, 114, 1991), ("tile", 512, 32, False, 32, "causal", 1, 70, 3026),
+    ("tile", 512, 32, False, 64, "causal", 2, 54, 1799), ("tile", 512, 16, False, 64, "causal", 1, 112, 1882),
+    ("tile", 512, 16, True, 64, "causal", 1, 64, 2041), ("tile", 512, 16, False, 64, "causal", 2, 51, 4500),
+    ("tile", 256, 32, False, 128, "causal", 1, 105, 993), ("tile", 256, 16, True, 128, "causal", 2, 68, 507),
+    ("tile", 512, 32, False, 16, "mask", 2, 56, 785), ("tile", 512, 32, False, 32, "mask", 1, 253, 499),
+    ("tile", 512, 32, False, 64, "mask", 2, 38, 1293),
+]
+
+
+@pytest.mark.parametrize("kernel,rows,edge,dealt,H,mode,B,R,L", LAUNCHES)
+def test_every_launch(gpu, kernel, rows, edge, dealt, H, mode, B, R, L):
+    kw = dict(causal=mode == "causal", has_mask=mode == "mask")
+    variant, plan = capi.launch_variant(B, R, L, H, **kw), capi.launch_plan(B, R, L, H, **kw)
+    assert (variant["kernel"], variant["rows"], plan["matrix_tile"], plan["heads_per_xcd"] > 0) == (kernel, rows, edge, dealt)
+    dtype = torch.bfloat16 if (L + H // 16) % 2 else torch.float16
+    q, k, v = (_rand((B, L, R * H), 5700 + L + i).to(dtype) for i in range(3))
+    mask = causal_mask(1, L).expand(B, L, L) if mode == "causal" else None
+    if mode == "mask":
+        mask = torch.randn(B, L, L, generator=torch.Generator().manual_seed(5705)).to(dtype)
+        mask[:, :, L - L // 3:] = float("-inf")
+        mask[:, L - 1, L - 1] = 1.0
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu) if mode == "mask" else None,
+                            causal=mode == "causal", return_lse=True)
+    for b, h in [(0, 0), (B - 1, R // 2), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        one = None if mask is None else mask[b:b + 1].float()
+        assert _max_err(got[b, :, sl], attention(*args, mask=one)[0]) <= (TOL if dtype == torch.float16 else BF16_TOL), (b, h)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        off = (lse[b, h].cpu() - attention_lse(args[0], args[1], H, mask=one)[0, 0]).abs()
+        assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
 
 
 @pytest.mark.parametrize("B,R,mode", [(11_999_999, 1, "plain"), (2_999_999, 4, "causal"), (2_999_999, 4, "mask")])

@@ -843,21 +843,23 @@ hipError_t dispatch_qkv(int64_t rope_head_dim, QkvKind kind, const fa::qkv::Para
     }
 }
 
-// Time of a projection in microseconds, fitted on 300 random shapes (M 64..16384, N 384..15360, K 128..5120, both
-// types, with and without tables) on MI355X: half of them are within 5 % of it, and choosing the smallest
-// estimate loses 0.2 % against the best kernel of each shape (9 % at most).  With k workgroups on the busiest
-// of the 256 compute units, w on the mean one and rounds = k over the resident ones:
+// Time of a projection in microseconds, fitted on 2853 random shapes (M 32..16384, N 192..15360, K 64..5120, both
+// types, with and without tables) on MI355X: half of the estimates are within 3.6 %, and choosing the smallest
+// one loses 0.12 % against the best kernel of each shape (over 3 % for 41 of them, 18 % at most).  (A fit over
+// 300 of them that favoured the 256 x 256 kernel by 4 %: 0.25 %, 72 shapes, 51 %; of 59 shapes that those 4 %
+// decided, 31 went to the slower kernel.)  With k workgroups on the busiest of the 256 compute units, w on the mean
+// one and rounds = k over the resident ones:
 //   launch + K / 64 (round rounds + busiest k + mean w) + (start + start_rope) rounds + (end + end_rope) k
 struct QkvCost {
     int resident;
     float launch, round, busiest, mean, start, end, start_rope, end_rope;
 };
 constexpr QkvCost kQkvCost[kQkvKinds] = {
-    {1, 0.518f, 1.072f, 0.f, 0.418f, 6.252f, 0.f, 2.267f, 0.f},
-    {1, 1.244f, 0.555f, 0.f, 0.236f, 4.113f, 0.f, 1.791f, 0.f},
-    {1, 2.063f, 0.313f, 0.f, 0.127f, 2.546f, 0.f, 0.84f, 0.f},
-    {2, 3.378f, 0.059f, 0.141f, 0.13f, 0.f, 0.479f, 0.f, 0.556f},
-    {2, 3.471f, 0.026f, 0.071f, 0.114f, 0.f, 0.281f, 0.014f, 0.428f},
+    {1, 0.84f, 1.04f, 0.f, 0.542f, 5.85f, 0.f, 2.84f, 0.f},
+    {1, 0.43f, 0.514f, 0.f, 0.308f, 4.61f, 0.f, 2.14f, 0.f},
+    {1, 1.29f, 0.303f, 0.f, 0.143f, 3.04f, 0.f, 0.961f, 0.f},
+    {2, 2.54f, 0.0987f, 0.11f, 0.134f, 0.f, 0.919f, 0.0769f, 0.5f},
+    {2, 2.74f, 0.0456f, 0.0856f, 0.0836f, 0.f, 0.536f, 0.0806f, 0.381f},
 };
 
 QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
@@ -872,7 +874,6 @@ QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
         const float busiest = ceil_f(mean), rounds = ceil_f(mean / (float)c.resident);
         float us = c.launch + slices * (c.round * rounds + c.busiest * busiest + c.mean * mean) + c.start * rounds + c.end * busiest;
         if (rope) us += c.start_rope * rounds + c.end_rope * busiest;
-        if (kind == kQkvWhole) us *= 0.96f;        // (between the two the fit is wrong by that much where it matters most)
         if (us < least) {
             least = us;
             best = (QkvKind)kind;

@@ -275,11 +275,11 @@ def test_views_in_the_bhld_layout_and_mismatched_strides(gpu):
         capi.forward(q.transpose(2, 3).contiguous().transpose(2, 3), k, v, H, layout="bhld")
 
 
-@pytest.mark.parametrize("R,L,H", [(2, 70, 64), (160, 600, 64), (80, 600, 128)])
+@pytest.mark.parametrize("R,L,H", [(2, 70, 64), (160, 600, 64), (80, 600, 128), (204, 391, 64), (88, 448, 128)])
 def test_row_pitch_at_the_limit(gpu, R, L, H):
     """stride_l = 2^24 elements, the largest the library accepts (32 MiB between sequence
     positions): q, k, v are column ranges of one [L, 2^24] buffer.  Bitwise the result of the
-    same call on contiguous copies, through the four-wave and the eight-wave kernel."""
+    same call on contiguous copies, through the key-split, the group and the tile kernels."""
     F = R * H
     pitch = 1 << 24
     buf = torch.empty((L, pitch), dtype=torch.float16, device=gpu)      # 2.3 GB / 20 GB, mostly untouched
@@ -401,11 +401,13 @@ def test_heads_and_batches_are_independent_bitwise(gpu):
 
 
 @pytest.mark.parametrize("B,R,L,H,causal", [
-    (2, 16, 1024, 64, False),       # the four-wave kernel
+    (2, 16, 1024, 64, False),       # the group kernel
+    (1, 4, 256, 64, False),         # the key-split kernel
     (4, 16, 2048, 64, False),       # the 16 x 16 kernel, one whole round
     (2, 64, 1024, 128, False),      # ... at head_dim 128
-    (16, 16, 1024, 64, True),       # ... causal, a pair of tiles per workgroup
-    (2, 40, 2048, 128, True),       # ... causal, tiles dealt out to a resident grid
+    (8, 16, 2048, 64, True),        # ... causal, a pair of tiles per workgroup
+    (16, 16, 1024, 64, True),       # the group kernel, causal
+    (2, 40, 2048, 128, True),       # the 16 x 16 kernel, causal, tiles dealt out to a resident grid
 ])
 def test_launch_can_be_captured_in_a_graph_and_replayed(gpu, B, R, L, H, causal):
     # The library allocates nothing and clears nothing at launch time, so a launch on a capturing
@@ -452,7 +454,7 @@ def _random_cases(n, seed):
 
 
 def _random_big_cases(n, seed):
-    # grids of several hundred workgroups and more: the eight-wave kernel in all its variants
+    # grids of several hundred workgroups and more: tile and group kernels
     import random
 
     rng = random.Random(seed)
@@ -598,7 +600,7 @@ def test_row_logsumexp(gpu, name, causal):
 
 
 def test_lse_of_the_pingpong_kernel(gpu):
-    # enough workgroups to select the eight-wave kernel; zero queries give lse = log(L) exactly
+    # enough workgroups to select a tile kernel; zero queries give lse = log(L) exactly
     B, R, L, H = 4, 16, 2048, 64
     k, v = _rand((B, L, R * H), 3800), _rand((B, L, R * H), 3801)
     out, lse = capi.forward(torch.zeros_like(k).to(gpu), k.to(gpu), v.to(gpu), H, return_lse=True)
@@ -707,15 +709,15 @@ def _check_pairs(got, q, k, v, H, pairs, mask=None):
 
 @pytest.mark.parametrize("B,R,L,H", [
     (1, 20, 4096, 64),      # eight-wave workgroups filling part of one round of the chip
-    (1, 40, 4096, 64),      # a poorly filled second round: eight 32-row waves, two workgroups per CU
+    (1, 40, 4096, 64),      # a poorly filled second round: the group kernel
     (1, 500, 256, 64),      # ... on short sequences
     (2, 8, 3073, 64),       # ... with ragged tiles, less than one workgroup per CU
     (1, 40, 2100, 32), (3, 20, 1111, 16),   # ... at the smaller head dims
     (1, 400, 40, 64), (2, 200, 7, 32),      # ... with sequences far shorter than a workgroup's 256 rows
-    (1, 32, 1024, 64),      # too few of those: four-wave workgroups
+    (1, 32, 1024, 64),      # ... two key groups
     (4, 16, 2112, 64),      # many workgroups, ragged last key tile and last query tile
     (1, 20, 2048, 128),     # head_dim 128, eight-wave workgroups in a part-filled round
-    (1, 40, 2048, 128),     # head_dim 128, four-wave workgroups
+    (1, 40, 2048, 128),     # head_dim 128, two key groups of the group kernel
     (2, 160, 1088, 128),    # head_dim 128, many workgroups, ragged tiles
 ])
 def test_launch_shapes_plain(gpu, B, R, L, H):
@@ -727,15 +729,16 @@ def test_launch_shapes_plain(gpu, B, R, L, H):
 
 @pytest.mark.parametrize("B,R,L", [
     (4, 16, 2048),      # one whole round of 512-query workgroups
-    (8, 32, 1000),      # two rounds, ragged last key tile and second query tile
+    (8, 16, 2011),      # two rounds, ragged last key tile and fourth query tile
+    (8, 32, 1000),      # (the group kernel, like any shape without a whole 512-query tile to spare)
     (4, 64, 1500),      # three rounds, three tiles per head, the last a quarter full
     (2, 60, 2048),      # a last round seven eighths full
     (1, 16, 16384),     # long rows: 256 key tiles per workgroup
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_kernel_with_16_row_matrix_tiles(gpu, B, R, L, dtype):
-    # Plain launches at head_dim 64 whose workgroups fill whole rounds of the chip take the kernel
-    # written on 16 x 16 x 32 products; here with row log-sum-exps, in both layouts.
+    # Plain launches at head_dim 64 whose workgroups fill whole rounds of the chip take the tile kernel
+    # written on 16 x 16 x 32 products, but for the one marked; here with row log-sum-exps, in both layouts.
     H = 64
     assert capi.launch_plan(B, R, L, H)["matrix_tile"] == 16
     q, k, v = (_rand((B, L, R * H), 4000 + L + i).to(dtype) for i in range(3))
@@ -790,12 +793,15 @@ def test_kernel_with_16_row_matrix_tiles_at_head_dim_128(gpu, B, R, L, causal, d
 
 @pytest.mark.parametrize("B,R,L", [
     (4, 16, 4096),      # 256 pairs of 512-query tiles
-    (16, 16, 1024),     # one pair per head: both tiles are diagonal tiles
-    (16, 16, 1000),     # ... with a ragged second tile
-    (2, 85, 2500),      # five tiles per head: two pairs and the middle tile alone, ragged end
+    (16, 16, 1024),     # (the group kernel)
+    (16, 16, 1000),     # (the group kernel)
+    (2, 85, 2500),      # (the group kernel)
+    (8, 16, 2000),      # two pairs per head, ragged end
+    (2, 51, 4500),      # nine tiles per head: four pairs and the middle tile alone, ragged end
     (1, 16, 16384),     # 16 pairs per head, up to 32 key tiles below the diagonal
     (2, 40, 4096),      # 320 pairs would be 1.25 rounds: tiles dealt out to a resident grid
-    (2, 64, 1300),      # ... three tiles per head, ragged end
+    (2, 64, 2500),      # ... five tiles per head, ragged end
+    (2, 64, 1300),      # (the group kernel)
     (3, 20, 4096),      # 240 pairs: a single round, not quite full
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -826,7 +832,7 @@ def test_causal_kernel_with_16_row_matrix_tiles(gpu, B, R, L, dtype):
 @pytest.mark.parametrize("B,R,L,H", [(4, 16, 2048, 64), (2, 64, 1024, 128)])
 @pytest.mark.parametrize("kind", ["std3", "rising", "falling"])
 def test_eight_wave_kernel_on_adversarial_scores(gpu, B, R, L, H, kind):
-    # Grids large enough for the eight-wave kernel, with scores that stress its running reference
+    # Grids large enough for the tile kernels, with scores that stress its running reference
     # maximum: |score| > 20 all over (std3), or a score that climbs (falls) by about 100 along the
     # key axis, so that the reference is overtaken again and again (never after the first key).
     q, k, v = (_rand((B, L, R * H), 4100 + L + i) for i in range(3))
@@ -847,12 +853,13 @@ def test_eight_wave_kernel_on_adversarial_scores(gpu, B, R, L, H, kind):
     assert scores.abs().max() > 20
 
 
-@pytest.mark.parametrize("B,R,L", [(4, 16, 4096), (16, 16, 1024), (2, 40, 4096)])
+@pytest.mark.parametrize("B,R,L", [(4, 16, 4096), (16, 16, 1024), (8, 16, 2000), (2, 40, 4096)])
 @pytest.mark.parametrize("kind", ["std3", "rising", "falling"])
 def test_causal_16_row_kernel_on_adversarial_scores(gpu, B, R, L, kind):
     # The same stress as above under the causal flag, where the 16 x 16 kernel leaves the blocks of a
     # wave one after the other: the reference is overtaken inside the sub-tiles in which only some
-    # of a wave's blocks still take part (pairs of tiles, one pair per head, tiles dealt out).
+    # of a wave's blocks still take part (pairs of tiles, two pairs per head, tiles dealt out; 16 x 16 heads of
+    # 1024 run on the group kernel).
     H = 64
     assert capi.launch_plan(B, R, L, H, causal=True)["matrix_tile"] == 16
     q, k, v = (_rand((B, L, R * H), 4200 + L + i) for i in range(3))
@@ -900,7 +907,7 @@ def test_heavy_tail_of_small_weights(gpu, B, R, L, H, gap_log2):
     # 2^-gap, together (L - 1) 2^-gap: 6 % of the row at gap 18 and L = 16384.  The probabilities
     # are rounded to fp16 before the second product, so a kernel whose reference pushes such
     # weights into the fp16 subnormals (or below 2^-24, to zero) loses that share of the row; the
-    # float32 oracle keeps it.  Both kernel families, through eight-wave and four-wave grids.
+    # float32 oracle keeps it.  Through the group, the tile and the key-split kernel.
     t = gap_log2 / math.log2(math.e) / math.sqrt(H)      # key 0 = t * ones: scaled score H t / sqrt(H)
     q = torch.ones(B, L, R * H).half()
     k = torch.zeros(B, L, R * H)
@@ -960,14 +967,16 @@ def test_long_sequences_where_the_reference_bias_is_most_negative(gpu, R, L, H):
 
 @pytest.mark.parametrize("B,R,L,H", [
     (4, 16, 4096, 64),      # eight-wave workgroups, each taking a pair of query tiles (8 tiles per head)
-    (2, 64, 1300, 64),      # ... with an odd number of tiles (the middle one runs alone) and a ragged end
+    (2, 51, 4500, 64),      # ... with an odd number of tiles (the middle one runs alone) and a ragged end
+    (2, 64, 1300, 64),      # the group kernel
     (2, 64, 1024, 128),     # head_dim 128, four tiles of 256 queries
     (4, 64, 1250, 128),     # head_dim 128, five tiles, ragged end
-    (8, 64, 512, 64), (3, 100, 300, 32),     # four-wave workgroups
-    (8, 12, 1024, 64), (1, 20, 4096, 64),    # eight 32-row waves: pairs of 256-query tiles filling most of one round
+    (8, 64, 512, 64), (3, 100, 300, 32),     # ... on several rounds
+    (8, 12, 1024, 64), (1, 20, 4096, 64),    # ... on part-filled ones
     (3, 16, 2000, 32), (16, 16, 500, 16),    # ... at the smaller head dims, with ragged ends
+    (2, 48, 5000, 32),
     (2, 40, 2048, 128), (2, 40, 4096, 64),   # 320 pairs would leave a second round three quarters empty: tiles dealt out to a resident grid
-    (2, 40, 2300, 128), (2, 48, 5000, 32),   # ... with an odd number of tiles and ragged ends
+    (2, 40, 2300, 128),                      # ... with an odd number of tiles and ragged ends
     (1, 40, 2048, 128), (1, 40, 4000, 64),   # ... fewer pairs than compute units: single tiles spread over all of them
 ])
 def test_causal_on_large_grids(gpu, B, R, L, H):
@@ -985,13 +994,13 @@ def test_causal_on_large_grids(gpu, B, R, L, H):
 
 
 @pytest.mark.parametrize("B,R,L,H", [
-    (8, 64, 512, 64), (16, 40, 384, 16), (2, 64, 1024, 32),     # eight-wave kernel, mask staged through LDS
-    (4, 40, 704, 128),                                           # ... head_dim 128, ragged end
-    (2, 64, 1023, 64),                                           # element-wise mask loads (L % 4 != 0)
-    (4, 40, 700, 128),                                           # 8-byte mask loads (L % 8 != 0)
-    (2, 12, 2048, 64), (1, 500, 256, 64), (2, 12, 2040, 16), (1, 40, 2104, 32),   # eight 32-row waves, 256-query workgroups
-    (1, 40, 2048, 128), (4, 40, 512, 128),   # head_dim 128: 256-query workgroups on a part-filled second round
-    (4, 12, 1536, 64),                       # 64-row waves on a lone round filled to 56 %
+    (8, 64, 512, 64), (16, 40, 384, 16),     # the group kernel
+    (2, 64, 1024, 32),                       # the tile kernel (test_masked_tile_kernel has more of them)
+    (4, 40, 704, 128),                       # the group kernel at head_dim 128, ragged end
+    (2, 64, 1023, 64),                       # ... with mask rows at any 2-byte address
+    (4, 40, 700, 128),                       # ... at 8-byte addresses
+    (2, 12, 2048, 64), (1, 500, 256, 64), (2, 12, 2040, 16), (1, 40, 2104, 32),   # ... on part-filled and ragged grids
+    (1, 40, 2048, 128), (4, 40, 512, 128), (4, 12, 1536, 64),
 ])
 def test_additive_mask_on_large_grids(gpu, B, R, L, H):
     q, k, v = (_rand((B, L, R * H), 3970 + L + i) for i in range(3))
@@ -1140,12 +1149,13 @@ def _block_mask(kind, B, L, seed):
 
 
 @pytest.mark.parametrize("B,R,L,H", [
-    (4, 16, 2048, 64),       # eight 64-row waves
-    (2, 40, 1024, 128),      # eight 32-row waves, head_dim 128
-    (2, 12, 2048, 64),       # eight 32-row waves, 256-query workgroups
-    (2, 64, 1000, 32),       # ... ragged end
-    (2, 2, 200, 64),         # four waves
-    (1, 4, 1023, 64),        # four waves, element-wise mask loads
+    (4, 16, 2048, 64),       # the tile kernel
+    (2, 40, 1024, 128),      # the group kernel, head_dim 128
+    (2, 12, 2048, 64),       # ... two key groups
+    (2, 64, 1000, 32),       # the tile kernel, ragged end
+    (2, 64, 1003, 16),       # ... rows of an odd length
+    (2, 2, 200, 64),         # the key-split kernel
+    (1, 4, 1023, 64),        # ... mask rows at any address
 ])
 @pytest.mark.parametrize("kind", ["causal", "padding", "documents", "blocks", "finite_min"])
 def test_block_structured_masks(gpu, B, R, L, H, kind):
@@ -1187,11 +1197,11 @@ BF16_TOL = 2e-2   # bf16 keeps 8 significant bits: the output rounding alone is 
 
 @pytest.mark.parametrize("B,R,L,H,causal", [
     (1, 2, 64, 64, False), (2, 3, 200, 32, False), (1, 2, 333, 16, True), (2, 2, 300, 128, False),
-    (4, 16, 2048, 64, False), (4, 16, 2048, 64, True),       # eight-wave kernel
+    (4, 16, 2048, 64, False), (4, 16, 2048, 64, True),       # the tile kernels
     (2, 64, 1024, 128, False), (2, 64, 1024, 128, True),
     (2, 8, 1000, 64, False),
-    (2, 8, 3073, 64, False),                                  # eight 32-row waves, two workgroups per CU
-    (8, 12, 1024, 64, True), (3, 16, 2000, 32, True),         # ... causal, one workgroup per CU
+    (2, 8, 3073, 64, False),                                  # the group kernel
+    (8, 12, 1024, 64, True), (3, 16, 2000, 32, True),         # ... causal
     (2, 40, 2048, 128, True), (1, 40, 4000, 64, True),        # causal, query tiles dealt out to a resident grid
 ])
 def test_bf16_inputs(gpu, B, R, L, H, causal):

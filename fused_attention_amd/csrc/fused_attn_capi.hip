@@ -29,7 +29,8 @@ struct Shape {
 //   {8, 2}  eight 64-row waves share one K/V stream, 512 queries per workgroup, one resident per
 //           compute unit: head_dim <= 64 (with head_dim 128 a 64-row wave would need the whole
 //           register file of a SIMD);
-//   {8, 1}  the same with 32-row waves, 256 queries per workgroup: head_dim 128, without additive mask;
+//   {8, 1}  the same with 32-row waves, 256 queries per workgroup: head_dim 128, without additive mask, and
+//           causal launches at head_dim 64 that fill one round of pairs of such tiles, not of larger ones;
 //   {0, 0}  no tile kernel.
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -127,7 +128,13 @@ Shape pick_shape(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, bool
         }
     }
     const int64_t used = usage(heads, L, rows, kNumCu);
-    return (wgs >= 2 * kNumCu ? used >= 614 : used >= (wgs <= kNumCu ? 560 : 717)) ? tile : Shape{0, 0};
+    if (wgs >= 2 * kNumCu ? used >= 614 : used >= (wgs <= kNumCu ? 560 : 717)) return tile;
+    // One round of pairs of 256-query tiles: of 500 random causal shapes at head_dim 64 it is the fastest on a
+    // quarter, by up to 26 % (B1 R32 L4096 103 -> 91 us, B3 R12 L3394 93.8 -> 77.8, B2 R40 L999 29.1 -> 24.1), and
+    // the choice with it loses 1.3 % against the best kernel of each, without it 4.8 %.  (At head_dim 16 and 32
+    // the group kernel is never more than 3 % behind it; plain launches, 214 shapes: 7 % at most, on 9 of them.)
+    if (causal && H == 64 && heads * ceil_div(L, 512) <= kNumCu && usage(heads, L, 512, kNumCu) >= 560) return {8, 1};
+    return {0, 0};
 }
 
 // Dynamic LDS above 64 KiB has to be opted into per kernel function and per device: done on the
@@ -178,8 +185,8 @@ hipError_t launch_pingpong(const fa::FwdParams& p, hipStream_t stream) {
 // (head_dim 64: 144 pairs -4.3 %, 160 -6.2 %, 192 -1.4 and +1.3 %, 200 -0.6 %; 240 +3.6 %, 256
 // +5.5 %, 400 +1.4 %, 960 +4.5 and +7.5 %, 1152 +5.4 %, dealt +3.2 to +4.7 %; head_dim 128: 1024
 // pairs +5.1 and +5.4 %, dealt +4.2 %): taken from seven eighths of a round on.
-bool use_tiles16(int64_t H, const fa::FwdParams& p, bool causal) {
-    if (H < 64) return false;
+bool use_tiles16(int64_t H, Shape sh, const fa::FwdParams& p, bool causal) {
+    if (H < 64 || (H == 64 && sh.nqb != 2)) return false;
     if (8 * (int64_t)p.total_wgs < 7 * kNumCu) return false;
     if (causal) return true;            // (a dealt launch is a whole resident grid)
     if (H == 64 && p.total_wgs < kNumCu) return false;     // (224 and 240 workgroups: +1.6 and +2.5 % at L = 4096, -1.4 % at L = 1024)
@@ -218,30 +225,32 @@ hipError_t launch_tiles16(int64_t H, int mode, bool bf16, const fa::FwdParams& p
 }
 
 template <int H, int MODE, bool BF>
-hipError_t dispatch_shape(const fa::FwdParams& p, hipStream_t stream) {
+hipError_t dispatch_shape(Shape sh, const fa::FwdParams& p, hipStream_t stream) {
     constexpr bool MASK = MODE == fa::kAdditive || MODE == fa::kAdditiveRagged;
     // the dealt causal schedule exists at head_dim 64 and 128 only (plan_causal never asks for it elsewhere),
     // and no masked launch at head_dim 128 (pick_shape)
     if constexpr ((MODE == fa::kCausalDealt && H < 64) || (MASK && H > 64))
         return hipErrorInvalidValue;
+    else if constexpr (H == 64 && (MODE == fa::kCausal || MODE == fa::kCausalDealt))
+        return sh.nqb == 1 ? launch_pingpong<H, 8, 1, 2, MODE, BF>(p, stream) : launch_pingpong<H, 8, 2, 2, MODE, BF>(p, stream);
     else
         return launch_pingpong<H, 8, (H > 64 ? 1 : 2), 2, MODE, BF>(p, stream);
 }
 
 template <int MODE, bool BF>
-hipError_t dispatch_head_dim(int64_t H, const fa::FwdParams& p, hipStream_t stream) {
+hipError_t dispatch_head_dim(int64_t H, Shape sh, const fa::FwdParams& p, hipStream_t stream) {
     switch (H) {
-        case 16: return dispatch_shape<16, MODE, BF>(p, stream);
-        case 32: return dispatch_shape<32, MODE, BF>(p, stream);
-        case 64: return dispatch_shape<64, MODE, BF>(p, stream);
-        case 128: return dispatch_shape<128, MODE, BF>(p, stream);
+        case 16: return dispatch_shape<16, MODE, BF>(sh, p, stream);
+        case 32: return dispatch_shape<32, MODE, BF>(sh, p, stream);
+        case 64: return dispatch_shape<64, MODE, BF>(sh, p, stream);
+        case 128: return dispatch_shape<128, MODE, BF>(sh, p, stream);
         default: return hipErrorInvalidValue;
     }
 }
 
 template <int MODE>
-hipError_t dispatch(int64_t H, const fa::FwdParams& p, hipStream_t stream, bool bf16) {
-    return bf16 ? dispatch_head_dim<MODE, true>(H, p, stream) : dispatch_head_dim<MODE, false>(H, p, stream);
+hipError_t dispatch(int64_t H, Shape sh, const fa::FwdParams& p, hipStream_t stream, bool bf16) {
+    return bf16 ? dispatch_head_dim<MODE, true>(H, sh, p, stream) : dispatch_head_dim<MODE, false>(H, sh, p, stream);
 }
 
 // Which kernel runs a problem: a tile kernel (the launch of pick_shape), the key-split kernel (`waves` share out
@@ -425,7 +434,7 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
 //                   + s sub-tiles min(k, resident) / GK           the longest one's neighbours
 //                   + c k
 // with sub-tiles of 32 keys, a causal tile's mean being about half of them, and rounds = k over the
-// workgroups resident per compute unit.
+// workgroups resident per compute unit (a zero: the times do not tell that term from the others).
 struct Cost {
     float a, b, c;
 };
@@ -437,31 +446,31 @@ constexpr float kLaunch = 3.2f;
 constexpr Cost kCostSplit2[4][3] = {
     {{0.0987f, 0.0404f, 0.117f}, {0.182f, 0.0476f, 0.113f}, {0.237f, 0.0567f, 0.124f}},
     {{0.134f, 0.0506f, 0.157f}, {0.201f, 0.0523f, 0.185f}, {0.291f, 0.0607f, 0.181f}},
-    {{0.312f, 0.0598f, 0.415f}, {0.335f, 0.0473f, 0.505f}, {0.47f, 0.0765f, 0.366f}},
-    {{0.503f, 0.0772f, 1.69f}, {0.696f, 0.0458f, 1.04f}, {0.871f, 0.0688f, 1.06f}},
+    {{0.312f, 0.0598f, 0.415f}, {0.342f, 0.0415f, 0.548f}, {0.47f, 0.0765f, 0.366f}},
+    {{0.503f, 0.0772f, 1.69f}, {0.587f, 0.0857f, 1.15f}, {0.871f, 0.0688f, 1.06f}},
 };
 constexpr Cost kCostSplit4[4][3] = {
     {{0.105f, 0.0493f, 0.138f}, {0.202f, 0.0465f, 0.219f}, {0.371f, 0.063f, 0.144f}},
     {{0.16f, 0.0496f, 0.268f}, {0.238f, 0.0537f, 0.309f}, {0.397f, 0.0605f, 0.244f}},
-    {{0.298f, 0.0603f, 0.492f}, {0.18f, 0.0783f, 0.535f}, {0.458f, 0.0685f, 0.579f}},
-    {{0.457f, 0.122f, 1.36f}, {0.374f, 0.137f, 1.33f}, {0.857f, 0.0981f, 1.44f}},
+    {{0.298f, 0.0603f, 0.492f}, {0.209f, 0.0655f, 0.517f}, {0.458f, 0.0685f, 0.579f}},
+    {{0.457f, 0.122f, 1.36f}, {0.411f, 0.0846f, 1.56f}, {0.857f, 0.0981f, 1.44f}},
 };
 constexpr GroupCost kCostGroup11[4][3] = {
     {{0.14f, 0.115f, 0.0523f, 0.493f}, {0.196f, 0.109f, 0.0289f, 0.495f}, {0.254f, 0.174f, 0.031f, 0.601f}},
     {{0.114f, 0.135f, 0.0291f, 0.433f}, {0.188f, 0.113f, 0.0242f, 0.414f}, {0.246f, 0.184f, 0.0129f, 0.569f}},
-    {{0.177f, 0.212f, 0.0291f, 0.588f}, {0.228f, 0.193f, 0.0244f, 0.48f}, {0.18f, 0.294f, 0.0551f, 0.958f}},
-    {{0.361f, 0.332f, 0.00792f, 1.13f}, {0.407f, 0.308f, 0.f, 1.21f}, {0.417f, 0.363f, 0.0182f, 1.47f}},
+    {{0.177f, 0.212f, 0.0291f, 0.588f}, {0.169f, 0.203f, 0.034f, 0.652f}, {0.18f, 0.294f, 0.0551f, 0.958f}},
+    {{0.361f, 0.332f, 0.00792f, 1.13f}, {0.441f, 0.319f, 0.f, 1.19f}, {0.417f, 0.363f, 0.0182f, 1.47f}},
 };
 constexpr GroupCost kCostGroup12[4][3] = {
     {{0.172f, 0.135f, 0.0295f, 0.523f}, {0.253f, 0.118f, 0.0128f, 0.688f}, {0.295f, 0.263f, 0.f, 0.581f}},
     {{0.143f, 0.159f, 0.0207f, 0.585f}, {0.226f, 0.136f, 0.00969f, 0.81f}, {0.256f, 0.262f, 0.f, 0.648f}},
-    {{0.198f, 0.195f, 0.0635f, 1.14f}, {0.264f, 0.155f, 0.0333f, 1.25f}, {0.342f, 0.252f, 0.0164f, 1.41f}},
-    {{0.378f, 0.343f, 0.0064f, 2.37f}, {0.378f, 0.334f, 0.f, 2.64f}, {0.473f, 0.399f, 0.0274f, 2.5f}},
+    {{0.198f, 0.195f, 0.0635f, 1.14f}, {0.196f, 0.18f, 0.0528f, 1.36f}, {0.342f, 0.252f, 0.0164f, 1.41f}},
+    {{0.378f, 0.343f, 0.0064f, 2.37f}, {0.386f, 0.337f, 0.f, 2.66f}, {0.473f, 0.399f, 0.0274f, 2.5f}},
 };
 constexpr GroupCost kCostGroup21[4][3] = {
     {{0.191f, 0.192f, 0.068f, 0.687f}, {0.243f, 0.209f, 0.0796f, 0.144f}, {0.372f, 0.323f, 0.0533f, 1.22f}},
     {{0.197f, 0.221f, 0.0518f, 0.616f}, {0.278f, 0.203f, 0.0567f, 0.147f}, {0.388f, 0.332f, 0.0549f, 1.23f}},
-    {{0.27f, 0.35f, 0.044f, 1.25f}, {0.344f, 0.369f, 0.0525f, 0.269f}, {0.515f, 0.42f, 0.0741f, 1.7f}},
+    {{0.27f, 0.35f, 0.044f, 1.25f}, {0.292f, 0.385f, 0.068f, 0.312f}, {0.515f, 0.42f, 0.0741f, 1.7f}},
     {{0.56f, 0.492f, 0.00712f, 2.09f}, {}, {}},
 };
 
@@ -483,13 +492,21 @@ constexpr GroupShape kGroups[] = {
 constexpr Cost kCostTile[4][3] = {       // [head_dim][plain, causal, mask], fwd_kernel_pingpong
     {{0.536f, 0.0518f, 2.81f}, {0.614f, 0.0242f, 7.91f}, {0.825f, 0.136f, 5.06f}},
     {{0.498f, 0.137f, 2.57f}, {0.599f, 0.0832f, 8.89f}, {0.811f, 0.27f, 3.73f}},
-    {{0.469f, 0.459f, 4.44f}, {0.654f, 0.147f, 11.4f}, {1.07f, 0.294f, 7.86f}},
-    {{0.297f, 0.6f, 5.26f}, {0.505f, 0.287f, 15.2f}, {}},
+    {{0.469f, 0.459f, 4.44f}, {0.612f, 0.169f, 14.9f}, {1.07f, 0.294f, 7.86f}},
+    {{0.297f, 0.6f, 5.26f}, {0.417f, 0.405f, 15.8f}, {}},
 };
 constexpr Cost kCostTile16[2][2] = {     // [head_dim 64, 128][plain, causal], fwd_kernel_pp16
-    {{0.508f, 0.362f, 7.63f}, {0.0783f, 0.851f, 10.1f}},
-    {{0.184f, 0.662f, 6.51f}, {0.f, 0.913f, 9.56f}},
+    {{0.508f, 0.362f, 7.63f}, {0.626f, 0.233f, 8.55f}},
+    {{0.184f, 0.662f, 6.51f}, {0.4f, 0.406f, 14.8f}},
 };
+
+// ... and for causal launches of 32-row waves at head_dim 64 (500 random shapes that fit one round of them)
+constexpr Cost kCostTile256 = {0.445f, 0.099f, 6.95f};
+// Causal launches with their tiles dealt out: a per sub-tile of the busiest workgroup, b per sub-tile of the mean
+// one, s per sub-tile of the mean one and head of its XCD, up to the 32 that its workgroups can be on at a
+// time (each head's K and V then serve one workgroup instead of many: half as long again at B17 R40 L1635 H128),
+// c per tile of a workgroup.  64-row and 32-row waves at head_dim 64, 32-row waves at 128.
+constexpr GroupCost kCostDealt[3] = {{0.387f, 0.394f, 0.00282f, 5.89f}, {0.199f, 0.295f, 0.013f, 0.804f}, {0.126f, 0.686f, 0.00439f, 6.54f}};
 
 float ceil_f(float x) {
     const float t = (float)(int64_t)x;
@@ -530,18 +547,19 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
         offer(g.kind, 8, kLaunch + t.c * k + (t.a * (nsub + (rounds - 1.f) * mean) + t.b * mean * 0.5f * (wgs + k) + t.s * nsub * shared) / (float)g.gk);
     }
     if (tile.waves != 0) {
-        const float n = (float)ceil_div(L, tile.rows()), rows = (float)tile.rows();
-        float chain = nsub, u = (float)p.total_wgs / kNumCu;
+        const float n = (float)ceil_div(L, tile.rows()), steps = (float)tile.rows() / 32.f;     // sub-tiles per block
         if (causal && p.heads_per_xcd > 0) {
-            chain = 0.5f * n * (n + 1.f) * heads * rows / 32.f / kNumCu;
-            u = 1.f;
-        } else if (causal) {
-            chain = (n + 1.f) * rows / 32.f;
-        } else {
-            chain *= ceil_f(n / (float)p.n_qtiles);       // a pair of tiles per workgroup
+            const float hx = (float)p.heads_per_xcd, worst = (float)plan_causal(B * R, (int64_t)n, H).blocks * steps;
+            const float mean = 0.5f * n * (n + 1.f) * heads * steps / kNumCu;
+            const GroupCost& t = kCostDealt[H == 128 ? 2 : tile.nqb == 1 ? 1 : 0];
+            offer(kTile, 8, kLaunch + t.a * worst + mean * (t.b + t.s * (hx < 32.f ? hx : 32.f)) +
+                                t.c * ceil_f(hx * n * fa::kNumXcd / kNumCu));
+            return best;
         }
-        const Cost& t = !has_mask && use_tiles16(H, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0]
-                                                                     : kCostTile[h][m];
+        // a pair of tiles per workgroup: causal ones, and masked ones where the grid says so
+        const float u = (float)p.total_wgs / kNumCu, chain = causal ? (n + 1.f) * steps : nsub * ceil_f(n / (float)p.n_qtiles);
+        const Cost& t = H == 64 && tile.nqb == 1 ? kCostTile256
+                        : !has_mask && use_tiles16(H, tile, p, causal) ? kCostTile16[h - 2][causal ? 1 : 0] : kCostTile[h][m];
         const float rounds = ceil_f(u);
         offer(kTile, 8, kLaunch + chain * (t.a * rounds + t.b * u) + t.c * rounds);
     }
@@ -648,18 +666,18 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
     if (variant.kind != kTile) {
         const int mode = causal ? fa::kCausal : mask != nullptr ? fa::kAdditive : fa::kPlain;
         e = bf16 ? dispatch_variant_mode<true>(H, mode, variant, p, s) : dispatch_variant_mode<false>(H, mode, variant, p, s);
-    } else if (mask == nullptr && use_tiles16(H, p, causal))
+    } else if (mask == nullptr && use_tiles16(H, shape, p, causal))
         e = launch_tiles16(H, causal ? (p.heads_per_xcd > 0 ? fa::kCausalDealt : fa::kCausal) : fa::kPlain, bf16, p, s);
     else if (causal && p.heads_per_xcd > 0)
-        e = dispatch<fa::kCausalDealt>(H, p, s, bf16);
+        e = dispatch<fa::kCausalDealt>(H, shape, p, s, bf16);
     else if (causal)
-        e = dispatch<fa::kCausal>(H, p, s, bf16);
+        e = dispatch<fa::kCausal>(H, shape, p, s, bf16);
     else if (mask != nullptr && L % 8 != 0)
-        e = dispatch<fa::kAdditiveRagged>(H, p, s, bf16);
+        e = dispatch<fa::kAdditiveRagged>(H, shape, p, s, bf16);
     else if (mask != nullptr)
-        e = dispatch<fa::kAdditive>(H, p, s, bf16);
+        e = dispatch<fa::kAdditive>(H, shape, p, s, bf16);
     else
-        e = dispatch<fa::kPlain>(H, p, s, bf16);
+        e = dispatch<fa::kPlain>(H, shape, p, s, bf16);
     return static_cast<int>(e);
 }
 
@@ -677,7 +695,7 @@ int fa_fwd_plan(int64_t B, int64_t R, int64_t L, int64_t H, int flags, int has_m
     plan[3] = p.total_wgs;
     plan[4] = p.n_qtiles;
     plan[5] = p.heads_per_xcd;
-    plan[6] = !tile || (!has_mask && use_tiles16(H, p, (flags & FA_FLAG_CAUSAL) != 0)) ? 16 : 32;
+    plan[6] = !tile || (!has_mask && use_tiles16(H, shape, p, (flags & FA_FLAG_CAUSAL) != 0)) ? 16 : 32;
     return FA_OK;
 }
 

@@ -228,15 +228,16 @@ template <int H, int GK>
 constexpr int group_slots() { return H == 128 && GK >= 2 ? 2 : 3; }
 template <int H, int GK>
 constexpr int group_ring_bytes() { return group_slots<H, GK>() * GK * group_sub<H, GK>() * 2 * 32 * H * 2; }
-// LDS: the ring of key tiles and the mask slabs, later the rows of O on their way out or, with several key
-// groups, the waves' shares of O (whichever is larger), and behind them m and l of every row.
+// What the second key group's wave of a row group hands to the first one's: O as the lanes hold it, m and l.
+template <int H, int NQ>
+constexpr int group_part_bytes() { return NQ * (H / 16 * 1024 + 512); }
+// LDS: the ring of key tiles and the mask slabs, later the rows of O on their way out or, with two key groups,
+// the second one's shares (whichever is larger).
 template <int H, int NQ, int GK, bool MASK>
-constexpr int group_stat_offset() {
-    constexpr int ring = group_ring_bytes<H, GK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 * 16 * NQ * split_row_floats<H>() * 4;
+constexpr int group_lds_bytes() {
+    constexpr int ring = group_ring_bytes<H, GK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
     return ring > part ? ring : part;
 }
-template <int H, int NQ, int GK, bool MASK>
-constexpr int group_lds_bytes() { return group_stat_offset<H, NQ, GK, MASK>() + (GK == 1 ? 0 : 8 * 16 * NQ * 8); }
 // (written in assembly so that the compiler does not see an LDS write, see RingLoader)
 __device__ __forceinline__ void group_dma16(uint32_t lds_addr, const _Float16* base, uint32_t voff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");

@@ -50,6 +50,15 @@ typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 #define FA_LDS __attribute__((address_space(3)))
 
+// Division of numbers below 2^31 by d: the high half of n * mul, shifted (mul = 0: d is 1).  mul is
+// floor(2^(31 + s) / d) + 1 with s = ceil(log2 d), which exceeds 2^(31 + s) / d by less than 2^s / d <= 2, so that the
+// quotient is exact for n < 2^31.
+struct Divisor {
+    uint32_t mul;
+    uint32_t shift;
+    __device__ __forceinline__ int of(int n) const { return mul == 0 ? n : (int)(__umulhi((uint32_t)n, mul) >> shift); }
+};
+
 struct FwdParams {
     const _Float16* q;
     const _Float16* k;
@@ -72,7 +81,12 @@ struct FwdParams {
                            // (t, n - 1 - t) of one head; > 0 = resident grid, the heads of an XCD's
                            // workgroups (B * R / 8 of them) dealt out tile by tile, see the kernel
     int waves;             // key-split kernel: waves per workgroup
+    Divisor by_qtiles;     // split and group kernels: division by n_qtiles and by R
+    Divisor by_heads;
     float scale_log2e;     // scale * log2(e)
+    // split and group kernels: what a score may be above the reference, in raw scores (the limit of one probability in
+    // fp16, and in bf16 what keeps the sum of 32 of them below kTripSum), and log2(e) / scale_log2e
+    float leash, mask_scale;
     float bias;            // bias of the reference of the exponentials, log2 units (see kBiasMin)
 };
 
@@ -103,6 +117,14 @@ __device__ __forceinline__ float fmax2(float a, float b) { return __builtin_elem
 __device__ __forceinline__ float pair_max(float x) {
     const uint32_t xb = __builtin_bit_cast(uint32_t, x);
     const u32x2 r = __builtin_amdgcn_permlane32_swap(xb, xb, false, false);
+    const uint32_t r0 = r[0], r1 = r[1];
+    return fmax2(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+}
+
+// ... and the same with lanes l and l^16.
+__device__ __forceinline__ float quad_max(float x) {
+    const uint32_t xb = __builtin_bit_cast(uint32_t, x);
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(xb, xb, false, false);
     const uint32_t r0 = r[0], r1 = r[1];
     return fmax2(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
 }
@@ -205,6 +227,18 @@ constexpr int lds_bytes_pingpong_masked() {
     return lds_bytes_pingpong<H, NQB>() + NW * 32 * NQB * kMaskSubStr * (int)sizeof(_Float16);
 }
 
+// Split and group kernels.  The launch's parameters in one go: left to itself the compiler loads them in three rounds, each behind a branch.
+__device__ __forceinline__ void load_args(const FwdParams& p) {
+    asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.stride_b), "s"(p.stride_h), "s"(p.stride_l), "s"(p.R), "s"(p.L), "s"(p.n_qtiles),
+                 "s"(p.total_wgs), "s"(p.wgs_per_xcd), "s"(p.by_qtiles.mul), "s"(p.by_qtiles.shift), "s"(p.by_heads.mul), "s"(p.by_heads.shift));
+}
+
+// What the launcher has worked out for the softmax (see FwdParams).
+struct SplitConstants {
+    float c, bias, leash, mask_scale;
+    __device__ __forceinline__ explicit SplitConstants(const FwdParams& p) : c(p.scale_log2e), bias(p.bias), leash(p.leash), mask_scale(p.mask_scale) {}
+};
+
 // Key-split kernel: LDS of one wave (slabs of the 32 keys it works on and their mask values; at the end
 // its share of 16 rows of O in float32, rows padded by 16 bytes against bank conflicts), and of a
 // workgroup (plus m and l of every row).
@@ -224,12 +258,12 @@ constexpr int split_lds_bytes(int waves) { return waves * (split_wave_bytes<H, M
 // barrier per sub-tile: +2 %), and ring slots (two where three would cost a resident workgroup: with the mask slabs
 // behind them a compute unit would hold two workgroups instead of three at head_dim 64, and the wait for a tile's
 // mask values is one for everything under way in any case).
-template <int H, int GK>
+template <int H, int NQ, int GK>
 constexpr int group_sub() { return GK == 1 && H <= 64 ? 2 : 1; }
-template <int H, int GK, bool MASK>
-constexpr int group_slots() { return (H == 128 && GK == 2) || MASK ? 2 : 3; }
-template <int H, int GK, bool MASK>
-constexpr int group_ring_bytes() { return group_slots<H, GK, MASK>() * GK * group_sub<H, GK>() * 2 * 32 * H * 2; }
+template <int H, int NQ, int GK, bool MASK>
+constexpr int group_slots() { return (GK == 2 && H == 128) || MASK ? 2 : 3; }
+template <int H, int NQ, int GK, bool MASK>
+constexpr int group_ring_bytes() { return group_slots<H, NQ, GK, MASK>() * GK * group_sub<H, NQ, GK>() * 2 * 32 * H * 2; }
 // What the second key group's wave of a row group hands to the first one's: O as the lanes hold it, m and l.
 template <int H, int NQ>
 constexpr int group_part_bytes() { return NQ * (H / 16 * 1024 + 512); }
@@ -237,7 +271,7 @@ constexpr int group_part_bytes() { return NQ * (H / 16 * 1024 + 512); }
 // the second one's shares (whichever is larger).
 template <int H, int NQ, int GK, bool MASK>
 constexpr int group_lds_bytes() {
-    constexpr int ring = group_ring_bytes<H, GK, MASK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
+    constexpr int ring = group_ring_bytes<H, NQ, GK, MASK>() + (MASK ? 8 * group_sub<H, NQ, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
     return ring > part ? ring : part;
 }
 // (written in assembly so that the compiler does not see an LDS write, see RingLoader)

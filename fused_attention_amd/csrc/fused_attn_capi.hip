@@ -571,7 +571,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
 
 // (two divisions by run-time numbers are 0.05 to 0.1 us at the start of a workgroup)
 fa::Divisor divisor(int64_t d) {
-    if (d == 1) return {0, 0};
+    if (d <= 1) return {0, 0};
     uint32_t s = 0;
     while (((int64_t)1 << s) < d) ++s;
     return {(uint32_t)(((uint64_t)1 << (31 + s)) / (uint64_t)d + 1), s - 1};
@@ -919,8 +919,13 @@ QkvKind pick_qkv(int64_t M, int64_t N, int64_t K, bool rope) {
 int use_qkv_kind(QkvKind kind, fa::qkv::Params* p) {
     if (kind == kQkvWhole) return FA_OK;
     const QkvTile t = kQkvTiles[kind];
-    const int64_t tiles_n = ceil_div(p->N, t.tn), tiles = ceil_div(p->M, t.tm) * tiles_n;
+    const int64_t tiles_n = ceil_div(p->N, t.tn), tiles_m = ceil_div(p->M, t.tm), tiles = tiles_m * tiles_n;
     if (tiles > 0x7fffffff - 8) return FA_ERR_TOO_LARGE;
+    const int64_t band = (int64_t)fa::qkv::kBand * fa::qkv::kTileM / t.tm;
+    p->tiles_m = (int)tiles_m;
+    p->by_band = divisor(band * tiles_n);
+    p->by_last = divisor(tiles_m % band != 0 ? tiles_m % band : band);
+    p->by_len = divisor(p->L);
     p->tiles_n = (int)tiles_n;
     p->total_tiles = (int)tiles;
     p->total_wgs = (int)tiles;
@@ -998,6 +1003,7 @@ int fa_qkv_proj_variant(int64_t B, int64_t L, int64_t F_in, int64_t R, int64_t H
     fa::qkv::Params p;
     p.M = (int)(B * L);
     p.N = (int)(3 * R * H);
+    p.L = (int)L;
     rc = qkv_geometry(p.M, p.N, &p);
     if (rc != FA_OK) return rc;
     const QkvKind kind = pick_qkv(p.M, p.N, F_in, rope != 0);

@@ -63,6 +63,9 @@ struct Params {
     int total_tiles;         // tiles_m * tiles_n
     int total_wgs;           // workgroups that take tiles: min(total_tiles, one per compute unit)
     int wgs_per_xcd;         // ceil(total_wgs / 8): the grid is 8 times this
+    // small tiles: row tiles, and division by the tiles of a band, by the row tiles of the last band and by L
+    int tiles_m;
+    Divisor by_band, by_last, by_len;
 };
 
 __device__ __forceinline__ void dma16(uint32_t lds_addr, const void* base, uint32_t voff) {
@@ -542,11 +545,12 @@ __global__ __launch_bounds__(kWaves * 64, MT * NT < 16 ? 4 : 2) void qkv_proj_sm
     if (logical >= p.total_wgs) return;
     // bands of 1024 rows, feature tile by feature tile inside a band, as above
     constexpr int BAND = kBand * kTileM / TM;
-    const int band = logical / (BAND * p.tiles_n);
+    const int band = p.by_band.of(logical);
     const int in_band = logical - band * (BAND * p.tiles_n);
-    const int band_rows = min(BAND, p.total_tiles / p.tiles_n - band * BAND);
-    const int m0 = (band * BAND + in_band % band_rows) * TM;
-    const int n0 = (in_band / band_rows) * TN;
+    const int left = p.tiles_m - band * BAND, band_rows = min(BAND, left);
+    const int col = left < BAND ? p.by_last.of(in_band) : in_band / BAND;
+    const int m0 = (band * BAND + in_band - col * band_rows) * TM;
+    const int n0 = col * TN;
 
     // first feature of the block at place b of the order described above
     auto feature_of = [](int b) __attribute__((always_inline)) {
@@ -576,13 +580,13 @@ __global__ __launch_bounds__(kWaves * 64, MT * NT < 16 ? 4 : 2) void qkv_proj_sm
             bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
         }
         if constexpr (HR > 0) {
-            const int at = m0 % p.L + 16 * (wm * MT + kg * OWN) + c16;
+            const int at = m0 - p.by_len.of(m0) * p.L + 16 * (wm * MT + kg * OWN) + c16;
 #pragma unroll
             for (int mt = 0; mt < OWN; ++mt) {
                 // (rows beyond M: any row of the tables)
                 int pos = at + 16 * mt;
                 if (p.L < TM)
-                    pos %= p.L;
+                    pos -= p.by_len.of(pos) * p.L;
                 else
                     pos -= pos >= p.L ? p.L : 0;
 #pragma unroll

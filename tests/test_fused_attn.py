@@ -1117,6 +1117,37 @@ def test_split_and_group_kernels(gpu, B, R, L, H, mode):
             assert off.max().item() <= (2.0 ** -8 if bf16 else 2.0 ** -10) * 1.01 + 1e-5, (variant, std, b, h)
 
 
+# Lengths with whole key tiles before a ragged one, an odd and an even number of them, by query rows per workgroup.
+@pytest.mark.parametrize("H,mode,rows", [(16, "plain", 128), (64, "plain", 64), (64, "plain", 128), (64, "causal", 128), (64, "plain", 256),
+                                         (64, "causal", 64), (128, "causal", 64), (128, "plain", 128)])
+@pytest.mark.parametrize("kind", ["climb", "leap"])
+def test_whole_key_tiles_of_the_group_kernel(gpu, H, mode, rows, kind):
+    # Whole key tiles have a loop of their own, which a wave leaves for good when the exponentials' reference
+    # has failed too often ("climb": in every third of the first half's sub-tiles) and stays in when it fails
+    # once ("leap": in the last whole tile but two, for every second row).
+    B, R, L = _shape_on("group", H, mode, [705, 833, 1217, 513, 391, 300, 261, 1473], rows)
+    dtype = torch.bfloat16 if (H // 16 + rows // 64) % 2 else torch.float16
+    q, k, v = (_rand((B, L, R, H), 6200 + L + i) for i in range(3))
+    up = torch.arange(L) // 32
+    up = torch.minimum(up, up.max() // 2 + 1) * 6.0 if kind == "climb" else (up >= up.max() - 5) * 40.0
+    q[..., 0] = 4.0
+    if kind == "leap":
+        q[:, 1::2, :, 0] = 0.0
+    k[..., 0] = (up * 0.6931 * H ** 0.5 / 4.0)[None, :, None]        # powers of two that the score rises by
+    q, k, v = (t.reshape(B, L, R * H).to(dtype) for t in (q, k, v))
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, causal=mode == "causal", return_lse=True)
+    one = causal_mask(1, L).float() if mode == "causal" else None
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        err = _max_err(got[b, :, sl], attention(*args, mask=one)[0])
+        assert err <= (2e-2 if dtype == torch.bfloat16 else TOL), (b, h, err)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
+        off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
+        assert off.max().item() <= 2.0 ** (-8 if dtype == torch.bfloat16 else -10) * 1.01 + 1e-5, (b, h)
+
+
 def _block_mask(kind, B, L, seed):
     """Masks under the reference's contract (zero where a pair takes part, -inf where it is muted,
     reference README.md:88-89), made of large all-zero and all-muted blocks: what the kernels'

@@ -1375,6 +1375,30 @@ def test_bf16_values_at_the_ends_of_the_range(gpu, kernel, H, mode, power, rise)
         assert ((got[b, :, h * H:(h + 1) * H].double().cpu() - want).abs() / 2.0 ** power).max().item() <= 2.0 ** -6, (b, h)
 
 
+@pytest.mark.parametrize("H,rows", [(16, 256), (64, 256), (128, 128), (64, 128), (128, 64)])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_scores_below_the_range_of_float32_in_some_rows(gpu, H, rows, odd):
+    # The first keys' scores are -inf in float32 for one of a wave's two blocks of 16 rows and ordinary for the other:
+    # the rows without a score so far have no reference yet, which their own sums tell and the other block's do not.
+    B, R, L = _shape_on("group", H, "plain", [512, 705, 833, 1217, 1473, 2048], rows)
+    q, k, v = (_rand((B, L, R, H), 6400 + L + i).float() for i in range(3))
+    low = (torch.arange(L) // 16) % 2 == odd
+    q[..., 0] = torch.where(low, 2.0 ** 100, 2.0 ** -100)[None, :, None]
+    k[..., 0] = 0.0
+    k[:, :200, :, 0] = -2.0 ** 100
+    q, k, v = (t.reshape(B, L, R * H).to(torch.bfloat16) for t in (q, k, v))
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, return_lse=True)
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        want = attention(*args)[0]
+        assert torch.isfinite(want).all()
+        err = _max_err(got[b, :, sl], want)
+        assert err <= 2e-2, (b, h, err)
+        off = (lse[b, h].cpu() - attention_lse(args[0], args[1], H)[0, 0]).abs()
+        assert off.max().item() <= 2.0 ** -8 * 1.01 + 1e-4, (b, h)
+
+
 @pytest.mark.parametrize("B,R,L,H", [(2, 3, 200, 64), (4, 16, 2048, 64), (2, 40, 1024, 128)])
 def test_extensions_through_the_compiled_module(gpu, B, R, L, H):
     """fused_attn.attention_forward_ex: causal, mask, log-sum-exp, bf16, the [B, R, L, H] layout and

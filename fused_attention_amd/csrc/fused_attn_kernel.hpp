@@ -81,13 +81,15 @@ struct FwdParams {
                            // (t, n - 1 - t) of one head; > 0 = resident grid, the heads of an XCD's
                            // workgroups (B * R / 8 of them) dealt out tile by tile, see the kernel
     int waves;             // key-split kernel: waves per workgroup
-    Divisor by_qtiles;     // split and group kernels: division by n_qtiles and by R
-    Divisor by_heads;
     float scale_log2e;     // scale * log2(e)
-    // split and group kernels: what a score may be above the reference, in raw scores (the limit of one probability in
-    // fp16, and in bf16 what keeps the sum of 32 of them below kTripSum), and log2(e) / scale_log2e
-    float leash, mask_scale;
     float bias;            // bias of the reference of the exponentials, log2 units (see kBiasMin)
+    // For the split and group kernels, behind what the tile kernels read: in between it moved their parameters, and
+    // the compiler's order of their instructions with them.
+    // Division by n_qtiles and by R; what a score may be above the reference, in raw scores (the limit of one probability
+    // in fp16, and in bf16 what keeps the sum of 32 of them below kTripSum); log2(e) / scale_log2e.
+    Divisor by_qtiles;
+    Divisor by_heads;
+    float leash, mask_scale;
 };
 
 constexpr int kNumXcd = 8;

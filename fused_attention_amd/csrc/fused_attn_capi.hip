@@ -261,6 +261,21 @@ struct Variant {
     int waves;
 };
 
+// (two divisions by run-time numbers are 0.05 to 0.1 us at the start of a workgroup)
+fa::Divisor divisor(int64_t d) {
+    if (d <= 1) return {0, 0};
+    uint32_t s = 0;
+    while (((int64_t)1 << s) < d) ++s;
+    return {(uint32_t)(((uint64_t)1 << (31 + s)) / (uint64_t)d + 1), s - 1};
+}
+
+fa::SplitParams split_params(const fa::FwdParams& p, bool bf16) {
+    fa::SplitParams params{p, divisor(p.n_qtiles), divisor(p.R), 0.f, 0.f};
+    params.leash = ((bf16 ? 10.f : 15.f) + p.bias) / p.scale_log2e;
+    params.mask_scale = 1.4426950408889634f / p.scale_log2e;
+    return params;
+}
+
 // The key-split kernel (16 query rows per workgroup).
 template <int H, int MODE, bool BF>
 hipError_t launch_split(const fa::FwdParams& p, hipStream_t stream) {
@@ -271,7 +286,7 @@ hipError_t launch_split(const fa::FwdParams& p, hipStream_t stream) {
         const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), most);
         if (e != hipSuccess) return e;
     }
-    fa::FwdParams params = p;
+    fa::SplitParams params = split_params(p, BF);
     void* args[] = {&params};
     return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(p.wgs_per_xcd * fa::kNumXcd), dim3(p.waves * 64), args,
                            fa::split_lds_bytes<H, MODE == fa::kAdditive>(p.waves), stream);
@@ -291,7 +306,7 @@ hipError_t launch_group(const fa::FwdParams& p, hipStream_t stream) {
         const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), lds);
         if (e != hipSuccess) return e;
     }
-    fa::FwdParams params = p;
+    fa::SplitParams params = split_params(p, BF);
     void* args[] = {&params};
     return hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(p.wgs_per_xcd * fa::kNumXcd), dim3(8 * 64), args, lds, stream);
 }
@@ -569,14 +584,6 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
     return best;
 }
 
-// (two divisions by run-time numbers are 0.05 to 0.1 us at the start of a workgroup)
-fa::Divisor divisor(int64_t d) {
-    if (d <= 1) return {0, 0};
-    uint32_t s = 0;
-    while (((int64_t)1 << s) < d) ++s;
-    return {(uint32_t)(((uint64_t)1 << (31 + s)) / (uint64_t)d + 1), s - 1};
-}
-
 // The launch of a key-split or group kernel in place of the tile kernels' one.
 int use_variant(const Variant& v, fa::FwdParams* p) {
     int64_t rows = 16;
@@ -589,8 +596,6 @@ int use_variant(const Variant& v, fa::FwdParams* p) {
     p->wgs_per_xcd = (int)ceil_div(total, fa::kNumXcd);
     p->heads_per_xcd = 0;
     p->waves = v.waves;
-    p->by_qtiles = divisor(per_head);
-    p->by_heads = divisor(p->R);
     return FA_OK;
 }
 
@@ -656,8 +661,6 @@ int fa_fwd_strided(const void* q, const void* k, const void* v, const void* mask
                             Strides{out_stride_b, out_stride_h, out_stride_l}, &p, scale, &shape, causal, lse);
     if (rc != FA_OK) return rc;
     if (bf16) p.bias = fa::kBiasBf16;
-    p.leash = ((bf16 ? 10.f : 15.f) + p.bias) / p.scale_log2e;
-    p.mask_scale = 1.4426950408889634f / p.scale_log2e;
     const Variant variant = pick_variant(B, R, L, H, mask != nullptr, causal, shape, p);
     const int rcv = variant.kind != kTile ? use_variant(variant, &p) : FA_OK;
     // A grid of 2^32 threads or more does not fit the dispatch packet (head_dim 16, L = 43: from 11 million heads

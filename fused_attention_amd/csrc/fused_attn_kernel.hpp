@@ -83,12 +83,16 @@ struct FwdParams {
     int waves;             // key-split kernel: waves per workgroup
     float scale_log2e;     // scale * log2(e)
     float bias;            // bias of the reference of the exponentials, log2 units (see kBiasMin)
-    // For the split and group kernels, behind what the tile kernels read: in between it moved their parameters, and
-    // the compiler's order of their instructions with them.
-    // Division by n_qtiles and by R; what a score may be above the reference, in raw scores (the limit of one probability
-    // in fp16, and in bf16 what keeps the sum of 32 of them below kTripSum); log2(e) / scale_log2e.
-    Divisor by_qtiles;
+};
+
+// The split and group kernels', apart from the tile kernels': fields added to those changed the compiler's order of the tile
+// kernels' instructions, B1 R32 L16384 H128 +1.1 % and B4 R16 L4096 H64 +1.6 % of the time; behind what they read, with
+// the same instructions, the second of these stayed (256.9 -> 261.0 us); apart, 253.9 and 254.3.
+struct SplitParams : FwdParams {
+    Divisor by_qtiles;     // division by n_qtiles and by R
     Divisor by_heads;
+    // what a score may be above the reference, in raw scores (the limit of one probability in fp16, and in bf16 what
+    // keeps the sum of 32 of them below kTripSum), and log2(e) / scale_log2e
     float leash, mask_scale;
 };
 
@@ -230,15 +234,15 @@ constexpr int lds_bytes_pingpong_masked() {
 }
 
 // Split and group kernels.  The launch's parameters in one go: left to itself the compiler loads them in three rounds, each behind a branch.
-__device__ __forceinline__ void load_args(const FwdParams& p) {
+__device__ __forceinline__ void load_args(const SplitParams& p) {
     asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.stride_b), "s"(p.stride_h), "s"(p.stride_l), "s"(p.R), "s"(p.L), "s"(p.n_qtiles),
                  "s"(p.total_wgs), "s"(p.wgs_per_xcd), "s"(p.by_qtiles.mul), "s"(p.by_qtiles.shift), "s"(p.by_heads.mul), "s"(p.by_heads.shift));
 }
 
-// What the launcher has worked out for the softmax (see FwdParams).
+// What the launcher has worked out for the softmax (see SplitParams).
 struct SplitConstants {
     float c, bias, leash, mask_scale;
-    __device__ __forceinline__ explicit SplitConstants(const FwdParams& p) : c(p.scale_log2e), bias(p.bias), leash(p.leash), mask_scale(p.mask_scale) {}
+    __device__ __forceinline__ explicit SplitConstants(const SplitParams& p) : c(p.scale_log2e), bias(p.bias), leash(p.leash), mask_scale(p.mask_scale) {}
 };
 
 // Key-split kernel: LDS of one wave (slabs of the 32 keys it works on and their mask values; at the end

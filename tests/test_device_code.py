@@ -1,0 +1,59 @@
+"""What the compiler made of the kernels, read in the assembly it prints for them (no GPU needed)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from fused_attention_amd import build
+
+HIPCC = os.path.join(build.ROCM, "bin", "hipcc")
+
+# (head_dim, blocks of 16 rows per wave, key groups, waves per SIMD): two and three ring slots, one and two key groups
+GROUP_KERNELS = [(16, 1, 2, 6), (32, 2, 1, 4), (64, 1, 1, 6), (128, 1, 1, 4), (128, 1, 2, 4)]
+
+
+@pytest.fixture(scope="module")
+def group_kernels(tmp_path_factory):
+    """{(head_dim, NQ, GK, mode): [lines of the kernel's assembly]}, unmasked (mode 0) and causal (2), fp16."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    where = tmp_path_factory.mktemp("asm")
+    source = ['#include "%s"' % os.path.join(build.CSRC, "fused_attn_kernel.hpp")]
+    source += ["template __global__ void fa::fwd_kernel_group<%d, %d, %d, fa::%s, %d>(const fa::SplitParams);" % (h, nq, gk, mode, wpe)
+               for h, nq, gk, wpe in GROUP_KERNELS for mode in ("kPlain", "kCausal")]
+    (where / "one.hip").write_text("\n".join(source) + "\n")
+    subprocess.run([HIPCC] + build.HIPCC_FLAGS + ["--cuda-device-only", "-S", str(where / "one.hip"), "-o", str(where / "one.s")],
+                   check=True, capture_output=True)
+    kernels, lines = {}, None
+    for line in (where / "one.s").read_text().splitlines():
+        found = re.match(r"_ZN2fa16fwd_kernel_groupILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E\w+:", line)
+        if found:
+            lines = kernels[tuple(int(n) for n in found.groups())] = []
+        elif line.startswith(".Lfunc_end"):
+            lines = None
+        elif lines is not None:
+            lines.append(line.strip())
+    return kernels
+
+
+def _loop_lines(lines):
+    """The instructions of the blocks that the compiler marks as part of a loop, without those written by hand."""
+    in_loop = by_hand = False
+    for line in lines:
+        if re.match(r"(\.LBB\d+_\d+:|; %bb\.)", line):
+            in_loop = False
+        in_loop = in_loop or (line.startswith((";", ".LBB")) and "Loop" in line)
+        by_hand = "#ASMSTART" in line or (by_hand and "#ASMEND" not in line)
+        if in_loop and not by_hand and line[:1] not in (";", ".", ""):
+            yield line
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("H,NQ,GK,wpe", GROUP_KERNELS)
+def test_the_group_kernel_waits_for_its_queries_once(group_kernels, H, NQ, GK, wpe, mode):
+    # The key tiles come by loads written in assembly, with exact waits of their own, so that the only loads the compiler
+    # knows of are the queries'.  A wait of its making inside a loop would be one for the key tiles on their way, in every pass.
+    lines = group_kernels[H, NQ, GK, mode]
+    assert any("s_barrier" in line for line in _loop_lines(lines))
+    assert [line for line in _loop_lines(lines) if line.startswith("s_waitcnt") and "vmcnt" in line] == []

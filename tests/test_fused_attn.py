@@ -1117,35 +1117,102 @@ def test_split_and_group_kernels(gpu, B, R, L, H, mode):
             assert off.max().item() <= (2.0 ** -8 if bf16 else 2.0 ** -10) * 1.01 + 1e-5, (variant, std, b, h)
 
 
-# Lengths with whole key tiles before a ragged one, an odd and an even number of them, by query rows per workgroup.
-@pytest.mark.parametrize("H,mode,rows", [(16, "plain", 128), (64, "plain", 64), (64, "plain", 128), (64, "causal", 128), (64, "plain", 256),
-                                         (64, "causal", 64), (128, "causal", 64), (128, "plain", 128)])
-@pytest.mark.parametrize("kind", ["climb", "leap"])
-def test_whole_key_tiles_of_the_group_kernel(gpu, H, mode, rows, kind):
-    # Whole key tiles have a loop of their own, which a wave leaves for good when the exponentials' reference
-    # has failed too often ("climb": in every third of the first half's sub-tiles) and stays in when it fails
-    # once ("leap": in the last whole tile but two, for every second row).
-    B, R, L = _shape_on("group", H, mode, [705, 833, 1217, 513, 391, 300, 261, 1473], rows)
-    dtype = torch.bfloat16 if (H // 16 + rows // 64) % 2 else torch.float16
+def _whole_tile_steps(q, k, H, mode, bf16, variant, waves):
+    """How the group kernel's waves take the sub-tiles of their whole key tiles behind the first (split_subtile), for one
+    head's q and k [L, H]: per wave a string of 't' (reference trusted, and it held), 'f' (it failed and the sub-tile is
+    done again) and 'l' (looked at first).  `waves`: (first row, key group) of those asked for."""
+    L, GK = q.shape[0], variant["key_groups"]
+    QW, SUB = variant["rows"] * GK // 8, 2 if GK == 1 and H <= 64 else 1
+    c = 1.4426950408889634 / H ** 0.5
+    bias = capi.load_library().fa_fwd_reference_bias(L)
+    leash, keys = ((10.0 if bf16 else 15.0) + bias) / c, 32 * GK * SUB
+    res = []
+    for row, kg in waves:
+        s = q[row:row + QW].float() @ k.float().t()
+        sub = lambda t, u: s[:, 32 * ((t * SUB + u) * GK + kg):][:, :32]
+        m = torch.cat([sub(0, u) for u in range(SUB)], 1).max(1).values
+        wary, steps = 0, ""
+        whole = min(L, row + 1 if mode == "causal" else L) // keys
+        for t, u in ((t, u) for t in range(1, whole) for u in range(SUB)):
+            trusted = wary == 0
+            if trusted:
+                sums = torch.exp2((sub(t, u) - m[:, None]) * c - bias).sum(1)
+                if sums.reshape(-1, 16).sum(0).max() < 32768.0:
+                    steps += "t"
+                    continue
+            wary = 2 if trusted else wary - 1
+            steps += "f" if trusted else "l"
+            new = sub(t, u).max(1).values
+            if (new >= m + leash).any():
+                m = torch.maximum(m, new)
+                if not trusted:
+                    wary = min(wary + 8, 32)
+        res.append(steps)
+    return res
+
+
+# By query rows per workgroup: one and two key groups, ring slots two (head_dim 128 and 64 rows) and three.  The lengths leave a
+# ragged end behind whole key tiles, an odd and an even number of them.
+@pytest.mark.parametrize("H,mode,rows", [(16, "plain", 128), (32, "plain", 256), (64, "plain", 64), (64, "plain", 128), (64, "plain", 256),
+                                         (64, "causal", 64), (64, "causal", 128), (128, "plain", 64), (128, "causal", 64), (128, "plain", 128)])
+@pytest.mark.parametrize("kind", ["climb", "stairs", "leap"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_whole_key_tiles_of_the_group_kernel(gpu, H, mode, rows, kind, dtype):
+    # Whole key tiles have a loop of their own, in which a wave looks at a sub-tile's scores first for a while after its
+    # reference has failed: all the time while every sub-tile's scores exceed the one before by more than the
+    # reference allows ("climb", three quarters of the sequence), again and again where they do at every twelfth
+    # ("stairs"), once in the last whole tile but two, for every second row ("leap").
+    B, R, L = _shape_on("group", H, mode, [1473, 1217, 1089, 833, 1537, 2049, 705], rows)
+    bf16 = dtype == torch.bfloat16
     q, k, v = (_rand((B, L, R, H), 6200 + L + i) for i in range(3))
     up = torch.arange(L) // 32
-    up = torch.minimum(up, up.max() // 2 + 1) * 6.0 if kind == "climb" else (up >= up.max() - 5) * 40.0
+    if kind == "climb":
+        up = torch.minimum(up, up.max() * 3 // 4) * 32.0
+    elif kind == "stairs":
+        up = up // 12 * 40.0
+    else:
+        up = (up >= up.max() - 5) * 40.0
     q[..., 0] = 4.0
     if kind == "leap":
         q[:, 1::2, :, 0] = 0.0
     k[..., 0] = (up * 0.6931 * H ** 0.5 / 4.0)[None, :, None]        # powers of two that the score rises by
     q, k, v = (t.reshape(B, L, R * H).to(dtype) for t in (q, k, v))
+    variant = capi.launch_variant(B, R, L, H, causal=mode == "causal")
+    group_rows = rows * variant["key_groups"] // 8
     got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, causal=mode == "causal", return_lse=True)
     one = causal_mask(1, L).float() if mode == "causal" else None
     for b, h in [(0, 0), (B - 1, R - 1)]:
         sl = slice(h * H, (h + 1) * H)
+        # the inputs do to the waves what is said above
+        last = (L - group_rows) // group_rows * group_rows
+        for steps in _whole_tile_steps(q[b, :, sl], k[b, :, sl], H, mode, bf16, variant, [(last, g) for g in range(variant["key_groups"])]):
+            if kind == "climb":
+                assert "l" * (len(steps) // 2) in steps and steps[0] == "f", steps
+            elif kind == "stairs":
+                assert "ftt" in steps.replace("l", "") and steps.count("f") >= 2, steps
+            else:
+                assert steps.count("f") == 1 and steps[0] == "t", steps
         args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
         err = _max_err(got[b, :, sl], attention(*args, mask=one)[0])
-        assert err <= (2e-2 if dtype == torch.bfloat16 else TOL), (b, h, err)
+        assert err <= (2e-2 if bf16 else TOL), (b, h, err)
         # (one rounding of the probabilities, see test_split_and_group_kernels)
         want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
         off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
-        assert off.max().item() <= 2.0 ** (-8 if dtype == torch.bfloat16 else -10) * 1.01 + 1e-5, (b, h)
+        assert off.max().item() <= 2.0 ** (-8 if bf16 else -10) * 1.01 + 1e-5, (b, h)
+
+
+@pytest.mark.parametrize("H,mode,B,R,L,limit", [(16, "plain", 16, 12, 705, 1.33), (32, "causal", 6, 8, 2561, 1.28), (128, "plain", 1, 20, 1473, 1.22)])
+def test_scores_of_a_wide_spread_cost_little(gpu, H, mode, B, R, L, limit):
+    # The time with N(0, 10) inputs over that with N(0, 1) ones, half way between 1.21, 1.16 and 1.12 and what sub-tiles done
+    # again too often, and a loop for waves that look first that knew no ring slot, made of it: 1.45, 1.42 and 1.32.
+    assert capi.launch_variant(B, R, L, H, causal=mode == "causal")["kernel"] == "group"
+    q, k, v = (_rand((B, L, R * H), 6300 + L + i).to(torch.bfloat16).to(gpu) for i in range(3))
+    us = {std: [] for std in (1.0, 10.0)}
+    scaled, out = {std: [t * std for t in (q, k, v)] for std in us}, torch.empty_like(q)
+    for _ in range(9):
+        for std in us:
+            us[std].append(capi.forward_timed(*scaled[std], H, out, 50, causal=mode == "causal"))
+    assert min(us[10.0]) <= limit * min(us[1.0]), us
 
 
 def _block_mask(kind, B, L, seed):

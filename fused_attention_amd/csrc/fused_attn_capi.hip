@@ -261,16 +261,9 @@ struct Variant {
     int waves;
 };
 
-// (two divisions by run-time numbers are 0.05 to 0.1 us at the start of a workgroup)
-fa::Divisor divisor(int64_t d) {
-    if (d <= 1) return {0, 0};
-    uint32_t s = 0;
-    while (((int64_t)1 << s) < d) ++s;
-    return {(uint32_t)(((uint64_t)1 << (31 + s)) / (uint64_t)d + 1), s - 1};
-}
-
 fa::SplitParams split_params(const fa::FwdParams& p, bool bf16) {
-    fa::SplitParams params{p, divisor(p.n_qtiles), divisor(p.R), 0.f, 0.f};
+    // (two divisions by run-time numbers are 0.05 to 0.1 us at the start of a workgroup)
+    fa::SplitParams params{p, fa::divisor(p.n_qtiles), fa::divisor(p.R), 0.f, 0.f};
     params.leash = ((bf16 ? 10.f : 15.f) + p.bias) / p.scale_log2e;
     params.mask_scale = 1.4426950408889634f / p.scale_log2e;
     return params;
@@ -926,9 +919,9 @@ int use_qkv_kind(QkvKind kind, fa::qkv::Params* p) {
     if (tiles > 0x7fffffff - 8) return FA_ERR_TOO_LARGE;
     const int64_t band = (int64_t)fa::qkv::kBand * fa::qkv::kTileM / t.tm;
     p->tiles_m = (int)tiles_m;
-    p->by_band = divisor(band * tiles_n);
-    p->by_last = divisor(tiles_m % band != 0 ? tiles_m % band : band);
-    p->by_len = divisor(p->L);
+    p->by_band = fa::divisor(band * tiles_n);
+    p->by_last = fa::divisor(tiles_m % band != 0 ? tiles_m % band : band);
+    p->by_len = fa::divisor(p->L);
     p->tiles_n = (int)tiles_n;
     p->total_tiles = (int)tiles;
     p->total_wgs = (int)tiles;

@@ -50,14 +50,22 @@ typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 #define FA_LDS __attribute__((address_space(3)))
 
-// Division of numbers below 2^31 by d: the high half of n * mul, shifted (mul = 0: d is 1).  mul is
-// floor(2^(31 + s) / d) + 1 with s = ceil(log2 d), which exceeds 2^(31 + s) / d by less than 2^s / d <= 2, so that the
-// quotient is exact for n < 2^31.
+// Division of numbers below 2^31 by d <= 2^31 - 1: the high half of n * mul, shifted (mul = 0: d is 1).  mul is
+// floor(2^(31 + s) / d) + 1 with s = ceil(log2 d), which exceeds 2^(31 + s) / d by at most 1 <= 2^s / d, so that
+// n * mul / 2^(31 + s) exceeds n / d by at most n / (2^31 d) < 1 / d and has the same whole part.  (It fits 32 bits: d is
+// above 2^(s - 1), hence 2^(31 + s) / d below 2^32 by at least 2^32 / d > 2.)
 struct Divisor {
     uint32_t mul;
     uint32_t shift;
     __device__ __forceinline__ int of(int n) const { return mul == 0 ? n : (int)(__umulhi((uint32_t)n, mul) >> shift); }
 };
+
+inline Divisor divisor(int64_t d) {
+    if (d <= 1) return {0, 0};
+    uint32_t s = 0;
+    while (((int64_t)1 << s) < d) ++s;
+    return {(uint32_t)(((uint64_t)1 << (31 + s)) / (uint64_t)d + 1), s - 1};
+}
 
 struct FwdParams {
     const _Float16* q;

@@ -1,4 +1,5 @@
-"""What the compiler made of the kernels, read in the assembly it prints for them (no GPU needed)."""
+"""What the compiler made of the kernels, read in the assembly it prints for them, and the host side of what
+the kernels compute with (no GPU needed)."""
 import os
 import re
 import subprocess
@@ -57,3 +58,40 @@ def test_the_group_kernel_waits_for_its_queries_once(group_kernels, H, NQ, GK, w
     lines = group_kernels[H, NQ, GK, mode]
     assert any("s_barrier" in line for line in _loop_lines(lines))
     assert [line for line in _loop_lines(lines) if line.startswith("s_waitcnt") and "vmcnt" in line] == []
+
+
+def test_division_by_multiplication_is_exact(tmp_path):
+    # fa::Divisor as the kernels use it (the high half of n * mul, shifted), at every d up to 70, at every power of
+    # two and its neighbours, and at the largest one: n on both sides of multiples of d, over the whole range.
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    (tmp_path / "div.hip").write_text('#include "%s"\n' % os.path.join(build.CSRC, "fused_attn_kernel.hpp") + r"""
+#include <cstdio>
+int main() {
+    const int64_t most = 0x7fffffff;
+    auto check = [&](int64_t d) {
+        const fa::Divisor by = fa::divisor(d);
+        auto right = [&](int64_t n) {
+            const int64_t got = by.mul == 0 ? n : (int64_t)((((uint64_t)n * by.mul) >> 32) >> by.shift);
+            if (got != n / d) std::printf("%lld / %lld is not %lld\n", (long long)n, (long long)d, (long long)got);
+            return got == n / d;
+        };
+        const int64_t whole = most / d, step = whole / 1000 + 1;
+        for (int64_t i = 0; i <= whole; i += step)
+            for (int64_t n = i * d - 1; n <= i * d + 1; ++n)
+                if (n >= 0 && n <= most && !right(n)) return false;
+        for (int64_t n = whole * d - 1; n <= most && n <= whole * d + 1; ++n)
+            if (n >= 0 && !right(n)) return false;
+        return right(0) && right(d - 1) && right(most - 1) && right(most);
+    };
+    for (int64_t d = 1; d <= 70; ++d)
+        if (!check(d)) return 1;
+    for (int s = 1; s <= 31; ++s)
+        for (int64_t d = ((int64_t)1 << s) - 1; d <= ((int64_t)1 << s) + 1 && d <= most; ++d)
+            if (!check(d)) return 1;
+    return check(most) ? 0 : 1;
+}
+""")
+    subprocess.run([HIPCC] + build.HIPCC_FLAGS + [str(tmp_path / "div.hip"), "-o", str(tmp_path / "div")], check=True, capture_output=True)
+    ran = subprocess.run([str(tmp_path / "div")], capture_output=True, text=True)
+    assert ran.returncode == 0, ran.stdout

@@ -272,12 +272,12 @@ constexpr int split_lds_bytes(int waves) { return waves * (split_wave_bytes<H, M
 // barrier per sub-tile: +2 %), and ring slots (two where three would cost a resident workgroup: with the mask slabs
 // behind them a compute unit would hold two workgroups instead of three at head_dim 64, and the wait for a tile's
 // mask values is one for everything under way in any case).
-template <int H, int NQ, int GK>
+template <int H, int GK>
 constexpr int group_sub() { return GK == 1 && H <= 64 ? 2 : 1; }
-template <int H, int NQ, int GK, bool MASK>
+template <int H, int GK, bool MASK>
 constexpr int group_slots() { return (GK == 2 && H == 128) || MASK ? 2 : 3; }
-template <int H, int NQ, int GK, bool MASK>
-constexpr int group_ring_bytes() { return group_slots<H, NQ, GK, MASK>() * GK * group_sub<H, NQ, GK>() * 2 * 32 * H * 2; }
+template <int H, int GK, bool MASK>
+constexpr int group_ring_bytes() { return group_slots<H, GK, MASK>() * GK * group_sub<H, GK>() * 2 * 32 * H * 2; }
 // What the second key group's wave of a row group hands to the first one's: O as the lanes hold it, m and l.
 template <int H, int NQ>
 constexpr int group_part_bytes() { return NQ * (H / 16 * 1024 + 512); }
@@ -285,7 +285,7 @@ constexpr int group_part_bytes() { return NQ * (H / 16 * 1024 + 512); }
 // the second one's shares (whichever is larger).
 template <int H, int NQ, int GK, bool MASK>
 constexpr int group_lds_bytes() {
-    constexpr int ring = group_ring_bytes<H, NQ, GK, MASK>() + (MASK ? 8 * group_sub<H, NQ, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
+    constexpr int ring = group_ring_bytes<H, GK, MASK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
     return ring > part ? ring : part;
 }
 // (written in assembly so that the compiler does not see an LDS write, see RingLoader)

@@ -437,6 +437,9 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
 // when there were tile kernels only.  Those are padding and causal-pattern masks for the most part, whose
 // muted blocks the tile kernels skip at less cost: the same shape with a bias or documents is
 // 10 to 40 % faster on the group kernel.
+// The split and group kernels have become 3 to 18 % faster since.  On 700 calls drawn from the ranges of perf/cases.py the choice
+// now loses 2.1 % against the best kernel of each, more than 3 % on 132 of them and on 37 of the 103 that go to a tile
+// kernel (B8 R12 L1024 H64: 33.1 us there, 31.5 on 16-row waves of the group kernel).
 //   split:  kLaunch + a ceil(sub-tiles / waves)              the longest wave
 //                   + b sub-tiles of all workgroups / 256    one compute unit's share of the work
 //                   + c k                                    start and merge
@@ -490,7 +493,9 @@ constexpr GroupCost kCostGroup21[4][3] = {
 struct GroupShape {
     VariantKind kind;
     int nq, gk;
-    int resident[4];            // workgroups per compute unit, by head_dim
+    // workgroups per compute unit, by head_dim, as the estimates were fitted with (now 4, 4, 3, 2 / 4, 4, 3, 2 / 3, 3, 2, 1
+    // without a mask; a change here goes with a new fit)
+    int resident[4];
     const GroupCost (*cost)[3];
 };
 constexpr GroupShape kGroups[] = {

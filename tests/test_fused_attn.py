@@ -853,6 +853,40 @@ def test_eight_wave_kernel_on_adversarial_scores(gpu, B, R, L, H, kind):
     assert scores.abs().max() > 20
 
 
+@pytest.mark.parametrize("B,R,L,H,mode", [
+    (4, 16, 2048, 64, "plain"), (2, 64, 1024, 128, "plain"), (4, 16, 2048, 64, "causal"), (2, 64, 1024, 128, "causal"),    # 16-row blocks
+    (8, 12, 1024, 64, "plain"), (4, 32, 2048, 32, "plain"), (4, 16, 2048, 64, "mask"), (1, 12, 12288, 64, "causal"),        # 32-row blocks
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_some_blocks_of_a_wave_move_their_reference(gpu, B, R, L, H, mode, dtype):
+    # The tile kernels send only those blocks of 16 (32) query rows down the slow path that a row of theirs needs it for.
+    # A few rows, spread over the blocks and waves, meet late keys whose scores stand 40 log2 units and more above the
+    # rest (bf16's leash is 29), one after the other; every row around them keeps the reference it has.
+    assert capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")["kernel"] == "tile"
+    q, k, v = (_rand((B, L, R, H), 4150 + L + i) for i in range(3))
+    hot = torch.tensor([L - 1 - r for r in (0, 5, 21, 38, 63, 64, 130, 200, 259, 330, 511)])
+    q[..., 0] = 0.0
+    q[:, hot, :, 0] = 8.0
+    k[..., 0] = 0.0
+    for n, at in enumerate((L // 2, L // 2 + 70, L - 600)):
+        k[:, at, :, 0] = (40.0 + 35.0 * n) * 0.6931 * H ** 0.5 / 8.0
+    q, k, v = (t.reshape(B, L, R * H).to(dtype) for t in (q, k, v))
+    mask = torch.zeros(B, L, L, dtype=dtype, device=gpu) if mode == "mask" else None
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask, causal=mode == "causal", return_lse=True)
+    rows = torch.arange(L - 640, L)
+    one = causal_mask(1, L)[0] if mode == "causal" else None
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float())
+        s = args[0][0, rows] @ args[1][0].t() / H ** 0.5
+        s = s if one is None else s + one[rows].float()
+        tol = TOL if dtype == torch.float16 else BF16_TOL
+        assert (got[b, rows][:, sl].float().cpu() - torch.softmax(s, -1) @ args[2][0]).abs().max().item() <= tol, (b, h)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        off = (lse[b, h, rows].cpu() - torch.logsumexp(s, -1)).abs() - 2e-5 * s.abs().max()
+        assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
+
+
 @pytest.mark.parametrize("B,R,L", [(4, 16, 4096), (16, 16, 1024), (8, 16, 2000), (2, 40, 4096), (1, 122, 1005)])
 @pytest.mark.parametrize("kind", ["std3", "rising", "falling"])
 def test_causal_16_row_kernel_on_adversarial_scores(gpu, B, R, L, kind):

@@ -74,6 +74,11 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, const void* base, uint3
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
 }
+// ... and of lane 0's four bytes
+__device__ __forceinline__ void dma4(uint32_t lds_addr, const void* base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :: "s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");
+}
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
@@ -190,12 +195,29 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
         issue_part(slot, std::integral_constant<int, 1>{});
     };
 
-    // acc[nt][mt][r]: row m = m0 + wm 64 + mt 16 + c16, feature n = n0 + wn 128 + nt 16 + 4 g4 + r
+    // acc[nt][mt][r]: row m = m0 + wm 64 + mt 16 + c16, feature n = n0 + wn 128 + nt 16 + 4 g4 + r.  They start at the bias,
+    // which then costs nothing per value at the end of a tile, where it had to be widened and added for every row block.
     floatx4 acc[8][4];
+    u16x4 bias4[8];
+    auto request_bias = [&](int tile) __attribute__((always_inline)) {
+        int m0, n0;
+        tile_origin(tile, m0, n0);
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt)
+        for (int nt = 0; nt < 8; ++nt) {
+            const int n = n0 + wn * 128 + nt * 16 + 4 * g4;
+            bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
+        }
+    };
+    auto start_over = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < 8; ++nt) {
+            floatx4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = v;
+        }
+    };
 
     // ---- per-lane parts of the operand addresses (halves inside a slot) ---------------------------
     // B operand (x): row wm 64 + mt 16 + c16, logical chunk 4 s + g4 (k-slots 8 g4 ... of sub-step s are
@@ -232,16 +254,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
         int m0, n0;
         tile_origin(done_tile, m0, n0);
         const int nw = n0 + wn * 128;
-        // What is read from memory, in one go ahead of its use: the bias of the wave's runs, and per 16-row block
-        // the distinct runs of the tables.  Requested where they are used, one wait behind the other, they took
+        // What is read from memory, the next tile's bias and per 16-row block the distinct runs of the tables, is
+        // requested in one go ahead of its use.  Requested where they are used, one wait behind the other, they took
         // most of an epilogue's time: M 16384 N 3072 K 1024 with tables 103.9 -> 92.5 us on the same box,
         // without them 90.3 -> 84.5, M 14400 N 768 K 256 17.5 -> 13.0; at K 5120 it is 1 %.
-        u16x4 bias4[8];
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const int n = nw + nt * 16 + 4 * g4;
-            bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
-        }
+        // What is left of it is vector instructions, two waves' per SIMD, and the matrix core idle beside them.  The bias
+        // in the accumulators from the start, one decision per wave instead of one per run whether it rotates (whose two
+        // sides met in register copies), and places in the stage one XOR apart: with tables M 16384 N 3072 K 1024
+        // 96.8 -> 94.1 us, M 8000 N 2304 K 768 46.1 -> 43.7, M 16384 N 1536 K 512 38.0 -> 35.5, M 8192 N 15360 K 5120
+        // 1017 -> 998; without either 89.0 -> 88.8.
         constexpr int RUNS = HR == 0 ? 1 : HR <= 32 ? 1 : HR / 32;
         floatx4 cos4[RUNS], sin4[RUNS];
         const int at = HR > 0 ? m0 % p.L + wm * 64 + c16 : 0;
@@ -262,71 +283,58 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
             }
         };
         request(0);
-        // one run of four features of one row with the bias added
-        auto biased = [&](int nt, int mt) __attribute__((always_inline)) {
-            floatx4 v = acc[nt][mt];
-            if (p.bias != nullptr) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
-            }
-            return v;
-        };
         // The results leave through a private LDS tile of 16 rows x 128 features per wave, so that
         // every store instruction writes whole rows (16 lanes x 16 bytes = the wave's 256 bytes of a
         // row) as streaming stores.  A lane holds one row of a 16-row block and runs of four features;
-        // chunk c (16 bytes) of stage row r sits at c ^ r.
+        // chunk c (16 bytes) of stage row r sits at c ^ r, so that the run of feature block nt is the
+        // first one's place XOR 32 nt bytes.
+        const uint32_t stage0 = (uint32_t)(uintptr_t)(FA_LDS void*)stage;
+        uint32_t place = stage0 + (uint32_t)(c16 * 256 + ((g4 >> 1) ^ c16) * 16 + 8 * (g4 & 1));
         auto store_run = [&](floatx4 v, int nt) __attribute__((always_inline)) {
             u16x4 hv;
 #pragma unroll
             for (int e = 0; e < 4; ++e) hv[e] = BF ? bf16::float_to_elem(v[e]) : float_to_elem(v[e]);
-            // (the row index is made opaque per run: otherwise the swizzled addresses of a row are all
-            // computed ahead and held in registers through the whole epilogue)
-            int r = c16;
-            asm volatile("" : "+v"(r));
-            *reinterpret_cast<u32x2*>(stage + r * 128 + (((2 * nt + (g4 >> 1)) ^ r) * 8) + 4 * (g4 & 1)) = __builtin_bit_cast(u32x2, hv);
+            *(FA_LDS u32x2*)(uintptr_t)(place ^ (32u * nt)) = __builtin_bit_cast(u32x2, hv);
         };
+        // (2 F is a multiple of 128: a wave's features are all of q and k, or all of v)
+        const bool rotated = nw < 2 * p.F;
+        const int l4 = lane >> 4, ch = lane & 15, n_out = nw + ch * 8;
+        const uint32_t out_off = (uint32_t)l4 * (uint32_t)p.N * 2u + (uint32_t)ch * 16u;
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            if constexpr (HR >= 32) {
+            // (opaque, so that the places of all runs are not worked out ahead and held through the whole epilogue)
+            asm volatile("" : "+v"(place));
+            if (HR >= 32 && rotated) {
                 // rotate-half: within a head, feature i < HR / 2 pairs with feature i + HR / 2:
                 //   out[i] = y[i] cos_i - y[i + HR/2] sin_i,  out[i + HR/2] = y[i + HR/2] cos_i + y[i] sin_i
                 // with cos_i, sin_i taken at the row's position.  Only the q and k slices (n < 2 F).  The
                 // partner run sits in the same lane, HR / 32 feature blocks on.
-                constexpr int D = HR / 32;
+                constexpr int D = HR >= 32 ? HR / 32 : 1;
 #pragma unroll
                 for (int pr = 0; pr < 4; ++pr) {
                     const int nt_a = (pr / D) * 2 * D + pr % D, nt_b = nt_a + D;
-                    floatx4 a = biased(nt_a, mt);
-                    floatx4 b = biased(nt_b, mt);
-                    if (nw + nt_a * 16 < 2 * p.F) {
-                        const floatx4 c4 = cos4[pr % D], s4 = sin4[pr % D];
-                        const floatx4 ra = a * c4 - b * s4;
-                        const floatx4 rb = b * c4 + a * s4;
-                        a = ra;
-                        b = rb;
-                    }
-                    store_run(a, nt_a);
-                    store_run(b, nt_b);
+                    const floatx4 a = acc[nt_a][mt], b = acc[nt_b][mt], c4 = cos4[pr % D], s4 = sin4[pr % D];
+                    store_run(a * c4 - b * s4, nt_a);
+                    store_run(b * c4 + a * s4, nt_b);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-            } else if constexpr (HR == 16) {
+            } else if (HR == 16 && rotated) {
                 // head_dim 16: a head is one feature block and the partner of a run sits 32 lanes away
 #pragma unroll
                 for (int nt = 0; nt < 8; ++nt) {
-                    floatx4 a = biased(nt, mt);
+                    const floatx4 a = acc[nt][mt];
                     floatx4 b;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float ae = a[e];      // (a bit cast taken straight from a vector element reads element 0)
                         b[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, ae)));
                     }
-                    if (nw + nt * 16 < 2 * p.F) a = g4 < 2 ? a * cos4[0] - b * sin4[0] : a * cos4[0] + b * sin4[0];
-                    store_run(a, nt);
+                    store_run(g4 < 2 ? a * cos4[0] - b * sin4[0] : a * cos4[0] + b * sin4[0], nt);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
 #pragma unroll
-                for (int nt = 0; nt < 8; ++nt) store_run(biased(nt, mt), nt);
+                for (int nt = 0; nt < 8; ++nt) store_run(acc[nt][mt], nt);
             }
             if (mt < 3) request(mt + 1);
             // LDS operations of one wave complete in order; the waits keep the compiler from moving
@@ -334,19 +342,19 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int r = 4 * i + (lane >> 4), ch = lane & 15;
-                const u32x4 w = *reinterpret_cast<const u32x4*>(stage + r * 128 + ((ch ^ r) * 8));
-                const int mr = m0 + wm * 64 + mt * 16 + r;
-                const int n = nw + ch * 8;
-                if (mr < p.M && n < p.N)
-                    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p.out + (int64_t)mr * p.N + n));
+                const int r = 4 * i + l4, row0 = m0 + wm * 64 + mt * 16 + 4 * i;
+                const u32x4 w = *(FA_LDS const u32x4*)(uintptr_t)(stage0 + (uint32_t)(r * 256 + (ch ^ r) * 16));
+                char* const out = reinterpret_cast<char*>(p.out + (int64_t)row0 * p.N + nw);
+                if (row0 + l4 < p.M && n_out < p.N) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(out + out_off));
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (mt == (HR > 0 ? 2 : 1)) {      // (half of the accumulators are through: their registers hold the next tile's bias)
+                __builtin_amdgcn_sched_barrier(0);
+                request_bias(min(done_tile + p.total_wgs, p.total_tiles - 1));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt)
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        start_over();
     };
 
     const int my_tiles = (p.total_tiles - logical + p.total_wgs - 1) / p.total_wgs;
@@ -403,14 +411,25 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
     // are issued.
     static_assert(NSLOT == 2, "the waits below assume that only the next step's loads are in flight");
     static_assert(NSUB == 2, "eight units per step");
+    // The first tile's bias by a direct load into the wave's stage, ahead of everything else: the compiler, which knows
+    // nothing of the loads that follow, would make its wait for a load of its own one for all of them.
+    int first_m0, first_n0;
+    tile_origin(logical, first_m0, first_n0);
+    if (p.bias != nullptr) dma4((uint32_t)(uintptr_t)(FA_LDS void*)stage, p.bias, min(2u * (uint32_t)(first_n0 + wn * 128) + 4u * (uint32_t)lane, 2u * (uint32_t)p.N - 4u));
     aim();
     issue(0);
-    if (total_steps > 1) {
-        issue(1);
-        wait_loads<LX + LW>();      // loads complete in order: all but the second step's have landed
-    } else {
+    if (total_steps > 1) issue(1);
+    if (total_steps > 1)            // (loads complete in order)
+        wait_loads<2 * (LX + LW)>();
+    else
+        wait_loads<LX + LW>();
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) bias4[nt] = p.bias != nullptr ? *reinterpret_cast<const u16x4*>(stage + nt * 16 + 4 * g4) : u16x4{0, 0, 0, 0};
+    start_over();
+    if (total_steps > 1)
+        wait_loads<LX + LW>();      // all but the second step's have landed
+    else
         wait_loads<0>();
-    }
     ring_barrier();
     load_a(I<0>{}, 0, I<0>{}, I<0>{});
     load_b(I<0>{}, 0, I<0>{});

@@ -54,6 +54,31 @@ def test_projection_matches_the_oracle(gpu, B, L, Fin, R, H, mode):
     _close(got, want)
 
 
+@pytest.mark.parametrize("B,L,Fin,R,H", [
+    (1, 20000, 64, 3, 64),       # one tile of one slice per workgroup; 576 features, the last wave's 64 of its 128
+    (1, 30000, 128, 20, 16),     # a second tile in other columns, head_dim 16; q and k end inside a tile
+    (1, 9000, 64, 21, 64),       # a third one; 4032 features
+])
+@pytest.mark.parametrize("mode", ["bias", "bias+rope"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_large_tiles_start_at_the_bias(gpu, B, L, Fin, R, H, mode, dtype):
+    # The 256 x 256 kernel's accumulators start at the bias: the first tile's comes through LDS, the next ones' through registers
+    # while the tile before ends.  Every feature with a bias of its own, at an address that is a multiple of eight only.
+    v = capi.projection_variant(B, L, Fin, R, H, rope="rope" in mode)
+    assert (v["tile_m"], v["tile_n"]) == (256, 256)
+    F = R * H
+    x = _rand((B, L, Fin), 7300 + L).to(dtype)
+    w = _rand((Fin, 3 * F), 7301 + L, 1.0 / math.sqrt(Fin)).to(dtype)
+    store = torch.zeros(3 * F + 4, dtype=dtype)
+    store[4:] = (torch.arange(3 * F) % 97 - 48) / 16.0
+    rope = rope_tables(L, H) if "rope" in mode else None
+    want = qkv_projection(x, w, store[4:], R, H, *(rope or (None, None)))
+    on_gpu = store.to(gpu)[4:]
+    assert on_gpu.data_ptr() % 16 == 8
+    got = capi.qkv_project(x.to(gpu), w.to(gpu), R, H, bias=on_gpu, rope=tuple(t.to(gpu) for t in rope) if rope else None)
+    _close(got, want, *(() if dtype == torch.float16 else (1.6e-2, 8e-3)))
+
+
 @pytest.mark.parametrize("B,L,Fin,R,H,tile", [
     (1, 1, 64, 4, 16, (64, 64)),           # one row, one slice: most of the ring stays empty
     (5, 13, 256, 12, 16, (64, 64)),        # one row into the second row tile, sequences shorter than a tile

@@ -556,6 +556,7 @@ Variant pick_variant(int64_t B, int64_t R, int64_t L, int64_t H, bool has_mask, 
     }
     for (const GroupShape& g : kGroups) {
         if (g.nq == 2 && H == 128 && m != 0) continue;         // (group21_offered)
+        if (has_mask && L < 8) continue;                       // (SplitMask::load_any)
         const int rows = 16 * g.nq * (8 / g.gk);
         const float wgs = heads * (float)ceil_div(L, rows) / kNumCu, k = ceil_f(wgs);
         const float mean = causal ? 0.5f * (nsub + (float)rows / 32.f) : nsub;

@@ -1113,6 +1113,42 @@ def test_masked_tile_kernel(gpu, H, residue):
         assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
 
 
+@pytest.mark.parametrize("H,rows", [(16, 128), (32, 64), (64, 64), (64, 128), (128, 128), (64, 256)])
+@pytest.mark.parametrize("residue", [0, 1, 3, 7])
+def test_mask_ends_inside_a_chunk_in_the_group_kernel(gpu, H, rows, residue):
+    # Its mask values come 16 bytes at a time, from any address: where the tensor ends inside a chunk its last 16 bytes are
+    # fetched and shifted into place.  The last rows of the last sequence, whose last nine keys carry most of the weight and
+    # no two of them the same value, in the mask's very last elements.
+    B, R, L = _shape_on("group", H, "mask", [8 * n + residue for n in (1, 2, 4, 5, 8, 12, 16, 20, 27, 40, 56, 80)], rows)
+    dtype = torch.bfloat16 if (H // 16 + residue) % 2 else torch.float16
+    q, k, v = (_rand((B, L, R * H), 5400 + L + i).to(dtype) for i in range(3))
+    mask = torch.zeros(B, L, L)
+    mask[:, :, L - min(9, L - 1):] = torch.arange(min(9, L - 1)).float() * 0.75 + 2.0
+    mask[:, ::3, L - min(5, L - 1):] = float("-inf")
+    mask = mask.to(dtype)
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu), return_lse=True)
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        assert _max_err(got[b, :, sl], attention(*args, mask=mask[b:b + 1].float())[0]) <= (TOL if dtype == torch.float16 else BF16_TOL), (b, h)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        off = (lse[b, h].cpu() - attention_lse(args[0], args[1], H, mask=mask[b:b + 1].float())[0, 0]).abs()
+        assert off.max().item() <= 2.0 ** (-10 if dtype == torch.float16 else -8) * 1.01 + 1e-4, (b, h)
+
+
+def test_masks_of_less_than_eight_keys(gpu):
+    # (never on the group kernel, whose loads of 16 bytes they may not hold)
+    for B, R, L, H in [(1, 1, 1, 64), (3, 7, 2, 16), (1, 300, 3, 128), (700, 12, 5, 64), (2, 40, 7, 32)]:
+        assert capi.launch_variant(B, R, L, H, has_mask=True)["kernel"] == "split"
+        q, k, v = (_rand((B, L, R * H), 5450 + L + i) for i in range(3))
+        mask = torch.randn(B, L, L, generator=torch.Generator().manual_seed(5455)).half()
+        got = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, mask=mask.to(gpu))
+        for b, h in [(0, 0), (B - 1, R - 1)]:
+            sl = slice(h * H, (h + 1) * H)
+            want = attention(q[b:b + 1, :, sl], k[b:b + 1, :, sl], v[b:b + 1, :, sl], H, mask=mask[b:b + 1].float())
+            assert _max_err(got[b, :, sl], want[0]) <= TOL, (b, h)
+
+
 # One shape or two per kernel and head_dim, at the edges of their tiles: 16, 64 and 128 query rows (256: LAUNCHES
 # below), 32 keys per sub-tile, 64 keys per key tile and three key tiles per turn of the ring.
 SMALL_GRIDS = [(1, 1, 1), (2, 3, 17), (1, 5, 33), (2, 4, 129), (1, 3, 300), (3, 40, 130), (2, 40, 255), (2, 16, 513),

@@ -1607,3 +1607,35 @@ def test_binding_rejections_on_device_tensors(gpu):
     # a sequence length that is not a multiple of chunk_size is accepted (the reference rejects it)
     y = torch.zeros(1, 50, 64, dtype=torch.float16, device=gpu)
     assert fused_attn.attention_forward(64, 64, y, y, y).shape == y.shape
+
+
+@pytest.mark.parametrize("listen", ["", "mode", "inference"])
+def test_new_tensors_of_the_compiled_module(gpu, listen):
+    # They come from the allocator directly, through the dispatcher only where something listens there; either way
+    # dense tensors of their own, on the device of the inputs, without a gradient.
+    import contextlib
+
+    import fused_attn
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Listen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    q, k, v = (_rand((2, 33, 64), 8000 + i).to(gpu) for i in range(3))
+    want = fused_attn.attention_forward(32, 32, q, k, v, None)
+    mode = Listen()
+    with mode if listen == "mode" else torch.inference_mode() if listen == "inference" else contextlib.nullcontext():
+        got = fused_attn.attention_forward(32, 32, q.requires_grad_(listen == ""), k, v, None)
+        ex, lse = fused_attn.attention_forward_ex(q, k, v, 32, return_lse=True)
+    assert (len([f for f in mode.seen if "empty" in f]) == 3) == (listen == "mode")
+    for t, shape, dtype in ((got, (2, 33, 64), torch.float16), (ex, (2, 33, 64), torch.float16), (lse, (2, 2, 33), torch.float32)):
+        assert t.shape == shape and t.dtype == dtype and t.is_contiguous() and t.device == q.device and not t.requires_grad
+        assert t.is_inference() == (listen == "inference") and t.storage_offset() == 0
+    assert torch.equal(got, want) and torch.equal(ex, want)
+    assert len({t.data_ptr() for t in (q, k, v, got, ex, lse)}) == 6

@@ -1193,6 +1193,7 @@ def _whole_tile_steps(q, k, H, mode, bf16, variant, waves):
     done again) and 'l' (looked at first).  `waves`: (first row, key group) of those asked for."""
     L, GK = q.shape[0], variant["key_groups"]
     QW, SUB = variant["rows"] * GK // 8, 2 if GK == 1 and H <= 64 else 1
+    two = SUB if QW == 16 and H <= 32 else 1        # sub-tiles per step (split_two)
     c = 1.4426950408889634 / H ** 0.5
     bias = capi.load_library().fa_fwd_reference_bias(L)
     leash, keys = ((10.0 if bf16 else 15.0) + bias) / c, 32 * GK * SUB
@@ -1203,16 +1204,16 @@ def _whole_tile_steps(q, k, H, mode, bf16, variant, waves):
         m = torch.cat([sub(0, u) for u in range(SUB)], 1).max(1).values
         wary, steps = 0, ""
         whole = min(L, row + 1 if mode == "causal" else L) // keys
-        for t, u in ((t, u) for t in range(1, whole) for u in range(SUB)):
-            trusted = wary == 0
+        for t, u in ((t, u) for t in range(1, whole) for u in range(0, SUB, two)):
+            trusted, step = wary == 0, torch.cat([sub(t, u + i) for i in range(two)], 1)
             if trusted:
-                sums = torch.exp2((sub(t, u) - m[:, None]) * c - bias).sum(1)
+                sums = torch.exp2((step - m[:, None]) * c - bias).sum(1)
                 if sums.reshape(-1, 16).sum(0).max() < 32768.0:
                     steps += "t"
                     continue
             wary = 2 if trusted else wary - 1
             steps += "f" if trusted else "l"
-            new = sub(t, u).max(1).values
+            new = step.max(1).values
             if (new >= m + leash).any():
                 m = torch.maximum(m, new)
                 if not trusted:
@@ -1269,6 +1270,36 @@ def test_whole_key_tiles_of_the_group_kernel(gpu, H, mode, rows, kind, dtype):
         want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
         off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
         assert off.max().item() <= 2.0 ** (-8 if bf16 else -10) * 1.01 + 1e-5, (b, h)
+
+
+@pytest.mark.parametrize("H", [16, 32])
+@pytest.mark.parametrize("mode", ["plain", "causal"])
+@pytest.mark.parametrize("L", [128, 704, 769, 865, 1087])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_two_sub_tiles_at_a_time(gpu, H, mode, L, dtype):
+    # 16-row waves at head_dim 16 and 32 take the sub-tiles of a whole key tile two at a time: one whole tile behind the
+    # first, an odd and an even number of them, remainders of 0, 1, 33 and 63 keys.  The scores of some rows leave
+    # the reference in the first sub-tile of a pair, those of others in the second one.
+    B, R, L = _shape_on("group", H, mode, [L], 128)
+    q, k, v = (_rand((B, L, R, H), 6250 + L + i) for i in range(3))
+    up = torch.arange(L) // 32
+    q[..., 0], q[..., 1] = 4.0, 4.0
+    q[:, 1::2, :, 0] = 0.0
+    q[:, ::3, :, 1] = 0.0
+    k[..., 0] = ((up // 10 * 40.0) * 0.6931 * H ** 0.5 / 4.0)[None, :, None]           # first sub-tiles of a pair
+    k[..., 1] = (((up + 5) // 8 * 40.0) * 0.6931 * H ** 0.5 / 4.0)[None, :, None]      # second ones
+    q, k, v = (t.reshape(B, L, R * H).to(dtype) for t in (q, k, v))
+    got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, causal=mode == "causal", return_lse=True)
+    one = causal_mask(1, L).float() if mode == "causal" else None
+    for b, h in [(0, 0), (B - 1, R - 1)]:
+        sl = slice(h * H, (h + 1) * H)
+        args = (q[b:b + 1, :, sl].float(), k[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H)
+        err = _max_err(got[b, :, sl], attention(*args, mask=one)[0])
+        assert err <= (2e-2 if dtype == torch.bfloat16 else TOL), (b, h, err)
+        # (one rounding of the probabilities, see test_split_and_group_kernels)
+        want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
+        off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
+        assert off.max().item() <= 2.0 ** (-8 if dtype == torch.bfloat16 else -10) * 1.01 + 1e-5, (b, h)
 
 
 @pytest.mark.parametrize("H,mode,B,R,L,limit", [(16, "plain", 16, 12, 705, 1.33), (32, "causal", 6, 8, 2561, 1.28), (128, "plain", 1, 20, 1473, 1.22)])

@@ -10,8 +10,9 @@ from fused_attention_amd import build
 
 HIPCC = os.path.join(build.ROCM, "bin", "hipcc")
 
-# (head_dim, blocks of 16 rows per wave, key groups, waves per SIMD): two and three ring slots, one and two key groups
-GROUP_KERNELS = [(16, 1, 2, 6), (32, 2, 1, 4), (64, 1, 1, 6), (128, 1, 1, 4), (128, 1, 2, 4)]
+# (head_dim, blocks of 16 rows per wave, key groups, waves per SIMD): two and three ring slots, one and two key groups, one
+# sub-tile at a time and two
+GROUP_KERNELS = [(16, 1, 2, 6), (32, 1, 1, 8), (32, 2, 1, 4), (64, 1, 1, 6), (128, 1, 1, 4), (128, 1, 2, 4)]
 
 
 @pytest.fixture(scope="module")

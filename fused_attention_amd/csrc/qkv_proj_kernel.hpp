@@ -195,28 +195,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
         issue_part(slot, std::integral_constant<int, 1>{});
     };
 
-    // acc[nt][mt][r]: row m = m0 + wm 64 + mt 16 + c16, feature n = n0 + wn 128 + nt 16 + 4 g4 + r.  They start at the bias,
-    // which then costs nothing per value at the end of a tile, where it had to be widened and added for every row block.
+    // acc[nt][mt][r]: row m = m0 + wm 64 + mt 16 + c16, feature n = n0 + wn 128 + nt 16 + 4 g4 + r
     floatx4 acc[8][4];
-    u16x4 bias4[8];
+    auto start_over = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    // The bias of a tile's features by a direct load into the wave's stage, which is idle until the tile ends: it has landed
+    // with the first slice that is waited for, and takes no register meanwhile.
     auto request_bias = [&](int tile) __attribute__((always_inline)) {
         int m0, n0;
         tile_origin(tile, m0, n0);
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const int n = n0 + wn * 128 + nt * 16 + 4 * g4;
-            bias4[nt] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const u16x4*>(p.bias + n) : u16x4{0, 0, 0, 0};
-        }
-    };
-    auto start_over = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            floatx4 v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = v;
-        }
+        if (p.bias != nullptr) dma4((uint32_t)(uintptr_t)(FA_LDS void*)stage, p.bias, min(2u * (uint32_t)(n0 + wn * 128) + 4u * (uint32_t)lane, 2u * (uint32_t)p.N - 4u));
     };
 
     // ---- per-lane parts of the operand addresses (halves inside a slot) ---------------------------
@@ -248,21 +240,21 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
     }
 
     // ---- end of a tile: bias, rotation, one rounding, whole-row stores; the accumulators start over ---
-    // The accumulators are only read here (results are formed in temporaries): modifying them in
-    // place inside the step loop makes the compiler carry a second copy of all of them.
+    // The rotation only reads the accumulators (results are formed in temporaries): done in place inside
+    // the step loop it makes the compiler carry a second copy of all of them.
     auto finish_tile = [&](int done_tile) __attribute__((always_inline)) {
         int m0, n0;
         tile_origin(done_tile, m0, n0);
         const int nw = n0 + wn * 128;
-        // What is read from memory, the next tile's bias and per 16-row block the distinct runs of the tables, is
-        // requested in one go ahead of its use.  Requested where they are used, one wait behind the other, they took
-        // most of an epilogue's time: M 16384 N 3072 K 1024 with tables 103.9 -> 92.5 us on the same box,
+        // What is read from memory, per 16-row block the distinct runs of the tables, is requested in one go ahead of its
+        // use.  Requested where they are used, one wait behind the other, they and the bias took most of an
+        // epilogue's time: M 16384 N 3072 K 1024 with tables 103.9 -> 92.5 us on the same box,
         // without them 90.3 -> 84.5, M 14400 N 768 K 256 17.5 -> 13.0; at K 5120 it is 1 %.
-        // What is left of it is vector instructions, two waves' per SIMD, and the matrix core idle beside them.  The bias
-        // in the accumulators from the start, one decision per wave instead of one per run whether it rotates (whose two
-        // sides met in register copies), and places in the stage one XOR apart: with tables M 16384 N 3072 K 1024
-        // 96.8 -> 94.1 us, M 8000 N 2304 K 768 46.1 -> 43.7, M 16384 N 1536 K 512 38.0 -> 35.5, M 8192 N 15360 K 5120
-        // 1017 -> 998; without either 89.0 -> 88.8.
+        // What is left of it is vector instructions, two waves' per SIMD, and the matrix core idle beside them.
+        // The bias from LDS, widened once per run of features instead of once per row block, one decision per row block
+        // instead of one per run whether it rotates (whose two sides met in register copies), and places in the stage one
+        // XOR apart: with tables M 16384 N 3072 K 1024 92.7 -> 89.2 us, at head_dim 128 100.1 -> 93.8, M 8192 N 15360 K 5120
+        // 943 -> 922, M 9000 N 4032 K 64 26.7 -> 24.2, M 8000 N 2304 K 768 41.2 -> 41.4; without tables 86.0 -> 85.5.
         constexpr int RUNS = HR == 0 ? 1 : HR <= 32 ? 1 : HR / 32;
         floatx4 cos4[RUNS], sin4[RUNS];
         const int at = HR > 0 ? m0 % p.L + wm * 64 + c16 : 0;
@@ -283,6 +275,25 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
             }
         };
         request(0);
+        // The bias comes last, on top of the finished sum and rounded once.  Accumulators that start at it round every
+        // partial sum at its magnitude: M 4096 N 3840 K 5120 with a bias of 256, whose q and k a rotation by 45 degrees
+        // brings back to 0.02, was 1.8e-4 (rms) off float64 that way and is 9.4e-6 off now, as on small tiles; one more matrix
+        // instruction of bias times one, which does not round to nearest, 1.1e-5.
+        if (p.bias != nullptr) {
+            u16x4 bias4[8];
+#pragma unroll
+            for (int nt = 0; nt < 8; ++nt) bias4[nt] = *reinterpret_cast<const u16x4*>(stage + nt * 16 + 4 * g4);
+            asm volatile("" ::: "memory");      // (the results pass through the same place)
+#pragma unroll
+            for (int nt = 0; nt < 8; ++nt) {
+                floatx4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = BF ? bf16::elem_to_float(bias4[nt][e]) : elem_to_float(bias4[nt][e]);
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt) acc[nt][mt] += v;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         // The results leave through a private LDS tile of 16 rows x 128 features per wave, so that
         // every store instruction writes whole rows (16 lanes x 16 bytes = the wave's 256 bytes of a
         // row) as streaming stores.  A lane holds one row of a 16-row block and runs of four features;
@@ -348,12 +359,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
                 if (row0 + l4 < p.M && n_out < p.N) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(out + out_off));
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (mt == (HR > 0 ? 2 : 1)) {      // (half of the accumulators are through: their registers hold the next tile's bias)
-                __builtin_amdgcn_sched_barrier(0);
-                request_bias(min(done_tile + p.total_wgs, p.total_tiles - 1));
-                __builtin_amdgcn_sched_barrier(0);
-            }
         }
+        if (done_tile + p.total_wgs < p.total_tiles) request_bias(done_tile + p.total_wgs);
         start_over();
     };
 
@@ -411,25 +418,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qkv_proj_kernel(const Params p
     // are issued.
     static_assert(NSLOT == 2, "the waits below assume that only the next step's loads are in flight");
     static_assert(NSUB == 2, "eight units per step");
-    // The first tile's bias by a direct load into the wave's stage, ahead of everything else: the compiler, which knows
-    // nothing of the loads that follow, would make its wait for a load of its own one for all of them.
-    int first_m0, first_n0;
-    tile_origin(logical, first_m0, first_n0);
-    if (p.bias != nullptr) dma4((uint32_t)(uintptr_t)(FA_LDS void*)stage, p.bias, min(2u * (uint32_t)(first_n0 + wn * 128) + 4u * (uint32_t)lane, 2u * (uint32_t)p.N - 4u));
+    request_bias(logical);      // (loads complete in order: landed with the first slice)
     aim();
     issue(0);
-    if (total_steps > 1) issue(1);
-    if (total_steps > 1)            // (loads complete in order)
-        wait_loads<2 * (LX + LW)>();
-    else
-        wait_loads<LX + LW>();
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) bias4[nt] = p.bias != nullptr ? *reinterpret_cast<const u16x4*>(stage + nt * 16 + 4 * g4) : u16x4{0, 0, 0, 0};
-    start_over();
-    if (total_steps > 1)
-        wait_loads<LX + LW>();      // all but the second step's have landed
-    else
+    if (total_steps > 1) {
+        issue(1);
+        wait_loads<LX + LW>();      // loads complete in order: all but the second step's have landed
+    } else {
         wait_loads<0>();
+    }
+    start_over();
     ring_barrier();
     load_a(I<0>{}, 0, I<0>{}, I<0>{});
     load_b(I<0>{}, 0, I<0>{});

@@ -61,9 +61,9 @@ def test_projection_matches_the_oracle(gpu, B, L, Fin, R, H, mode):
 ])
 @pytest.mark.parametrize("mode", ["bias", "bias+rope"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_large_tiles_start_at_the_bias(gpu, B, L, Fin, R, H, mode, dtype):
-    # The 256 x 256 kernel's accumulators start at the bias: the first tile's comes through LDS, the next ones' through registers
-    # while the tile before ends.  Every feature with a bias of its own, at an address that is a multiple of eight only.
+def test_bias_of_large_tiles(gpu, B, L, Fin, R, H, mode, dtype):
+    # The 256 x 256 kernel's bias comes through LDS, requested when the tile before has ended.  Every feature with a bias
+    # of its own, at an address that is a multiple of eight only.
     v = capi.projection_variant(B, L, Fin, R, H, rope="rope" in mode)
     assert (v["tile_m"], v["tile_n"]) == (256, 256)
     F = R * H
@@ -77,6 +77,43 @@ def test_large_tiles_start_at_the_bias(gpu, B, L, Fin, R, H, mode, dtype):
     assert on_gpu.data_ptr() % 16 == 8
     got = capi.qkv_project(x.to(gpu), w.to(gpu), R, H, bias=on_gpu, rope=tuple(t.to(gpu) for t in rope) if rope else None)
     _close(got, want, *(() if dtype == torch.float16 else (1.6e-2, 8e-3)))
+
+
+@pytest.mark.parametrize("L,R,H,tile", [
+    (4096, 20, 64, (256, 256)), (4096, 10, 128, (256, 256)), (4096, 80, 16, (256, 256)), (300, 20, 64, (64, 128)), (300, 80, 16, (64, 128)),
+])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_large_bias_costs_one_rounding(gpu, L, R, H, tile, rope, dtype):
+    # 4096 products under a bias of 256, against float64: the bias is added to the finished sum, so that its magnitude is
+    # rounded at once and not with every partial sum.  Rotated by 45 degrees the biases of a pair cancel and what is
+    # left shows it; without a rotation it shows where the result lies half way between two values of `dtype`.
+    Fin, F, big = 4096, R * H, 256.0
+    v = capi.projection_variant(1, L, Fin, R, H, rope=rope)
+    assert (v["tile_m"], v["tile_n"]) == tile
+    x = _rand((1, L, Fin), 7350 + L).to(dtype)
+    w = _rand((Fin, 3 * F), 7351 + H, 3e-4 if rope else 1.0 / math.sqrt(Fin)).to(dtype)
+    b = torch.full((3 * F,), big, dtype=dtype)
+    cos = torch.full((L, H // 2), math.sqrt(0.5))
+    got = capi.qkv_project(x.to(gpu), w.to(gpu), R, H, bias=b.to(gpu), rope=(cos.to(gpu), cos.to(gpu)) if rope else None).cpu()
+    rows = torch.randperm(L, generator=torch.Generator().manual_seed(7352))[:48]
+    y = x[0, rows].double() @ w.double()
+    sums = y.abs().max().item()
+    y = y + big
+    got = got[0, rows].double()
+    # sums: 32-wide instructions, four roundings in each at most; one rounding on top of the bias (half an ulp at 256)
+    off = Fin / 32 * 4 * 2.0 ** -25 * 2.0 ** math.ceil(math.log2(sums)) + 2.0 ** -16
+    if rope:
+        want = (y.view(-1, 3, R, 2, H // 2)[:, :2, :, 0] - y.view(-1, 3, R, 2, H // 2)[:, :2, :, 1]) * cos[0, 0].double()
+        got = got.view(-1, 3, R, 2, H // 2)[:, :2, :, 0]
+        off = 2 * off * 0.7072 + 2 * 2.0 ** -17       # two of them, and the two products (below 256) rounded
+    else:
+        want = y.view(-1, 3, F)
+    ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    # half an ulp of what is rounded, which is up to `off` larger than the exact value
+    final = ulp * 2.0 ** torch.floor(torch.log2((want.abs() + off).clamp_min(2.0 ** -14)))
+    excess = ((got - want).abs() - final - off).max().item()
+    assert excess <= 0, excess
 
 
 @pytest.mark.parametrize("B,L,Fin,R,H,tile", [

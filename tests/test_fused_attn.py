@@ -1670,3 +1670,21 @@ def test_new_tensors_of_the_compiled_module(gpu, listen):
         assert t.is_inference() == (listen == "inference") and t.storage_offset() == 0
     assert torch.equal(got, want) and torch.equal(ex, want)
     assert len({t.data_ptr() for t in (q, k, v, got, ex, lse)}) == 6
+
+
+@pytest.mark.parametrize("listen", [False, True])
+def test_output_keeps_the_strides_of_the_queries(gpu, listen):
+    # attention_forward's output is laid out like the queries, which are contiguous: a dimension of one element may have any stride
+    import fused_attn
+
+    x = _rand((33, 1, 64), 8120).to(gpu).transpose(0, 1)
+    assert x.is_contiguous() and x.stride() == (64, 64, 1)
+    dense = x.clone(memory_format=torch.contiguous_format).view(-1).view(1, 33, 64)
+    torch.use_deterministic_algorithms(listen)
+    try:
+        got = fused_attn.attention_forward(32, 32, x, x, x, None)
+        assert fused_attn.attention_forward_ex(x, x, x, 32).stride() == (2112, 64, 1)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert got.stride() == x.stride() == torch.empty_like(x).stride()
+    assert torch.equal(got, fused_attn.attention_forward(32, 32, dense, dense, dense, None))

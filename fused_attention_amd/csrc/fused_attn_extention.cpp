@@ -23,9 +23,10 @@
 //     terminating the process (reference include/fused_attn.cuh:17-42 calls std::exit).
 #include <torch/extension.h>
 
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
-#include <c10/core/impl/TorchDispatchModeTLS.h>
 
 // PyTorch-ROCm presents its HIP devices under the device type "cuda"; these are the guard and
 // stream accessors that understand that.
@@ -51,20 +52,23 @@ void check_qkv(const torch::Tensor& t, const char* name) {
     TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
 }
 
-// The device of `t` made current for the launch, if it is not (a guard of its own costs 0.1 us of a call's 4.5).
+// The device of `t` made current for the launch, if it is not.
 std::optional<c10::hip::HIPGuardMasqueradingAsCUDA> on_device_of(const torch::Tensor& t) {
     if (c10::hip::current_device() == t.device().index()) return std::nullopt;
     return std::optional<c10::hip::HIPGuardMasqueradingAsCUDA>(t.device());
 }
 
-// A new dense tensor on the device of `like`.  Small calls come as fast as the host launches them, and the way
-// through the dispatcher is 0.4 us of that: it is taken where something may listen there (a dispatch mode, a
-// tensor subclass, a tracer), otherwise the memory comes from the allocator directly.  B1 R4 L256 H64, launches of 3.6 us:
-// 4.9 -> 4.5 us per call.
+// Whether an allocation has to go through the dispatcher: a mode, a tracer or a functional transform (keys that this
+// thread does not usually include), a tensor subclass or wrapper, the callbacks of a profiler, or the fill of new memory
+// that deterministic algorithms ask for.  Small calls come as fast as the host launches them: where nothing listens the
+// memory comes from the allocator directly, and no guard is made for a device that is current (B1 R4 L256 H64, medians of five
+// processes each, in turn: 4.80 -> 4.40 us per call, a single process 3.75 or 4.4; the questions asked here are 0.05 of it).
 bool allocation_is_watched(const torch::Tensor& like) {
-    return c10::impl::dispatch_mode_enabled() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
-           like.key_set().has(c10::DispatchKey::Python);
+    return !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() ||
+           at::isTensorSubclassLike(like) || at::hasCallbacks() || at::globalContext().deterministicAlgorithms();
 }
+
+// A new dense tensor on the device of `like`.
 torch::Tensor new_dense(const torch::Tensor& like, c10::IntArrayRef sizes, c10::ScalarType dtype) {
     if (allocation_is_watched(like)) return torch::empty(sizes, like.options().dtype(dtype));
     return at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt);

@@ -1642,8 +1642,8 @@ def test_binding_rejections_on_device_tensors(gpu):
 
 @pytest.mark.parametrize("listen", ["", "mode", "inference"])
 def test_new_tensors_of_the_compiled_module(gpu, listen):
-    # They come from the allocator directly, through the dispatcher only where something listens there; either way
-    # dense tensors of their own, on the device of the inputs, without a gradient.
+    # They come from the allocator directly, through the dispatcher only where something listens there (more of that below);
+    # either way dense tensors of their own, on the device of the inputs, without a gradient.
     import contextlib
 
     import fused_attn
@@ -1670,6 +1670,36 @@ def test_new_tensors_of_the_compiled_module(gpu, listen):
         assert t.is_inference() == (listen == "inference") and t.storage_offset() == 0
     assert torch.equal(got, want) and torch.equal(ex, want)
     assert len({t.data_ptr() for t in (q, k, v, got, ex, lse)}) == 6
+
+
+def test_functional_transforms_refuse_the_compiled_module(gpu):
+    # A call of these modules has no gradient or tangent, so grad and jvp must not walk past it: the output is theirs
+    # (a wrapper without memory), and the call ends in an error instead of a result that lacks its share.
+    import fused_attn
+
+    q, k, v = (_rand((2, 33, 64), 8100 + i).to(gpu) for i in range(3))
+    x, w = _rand((2, 33, 64), 8105).to(gpu), _rand((64, 192), 8106, 0.1).to(gpu)
+    one = torch.ones(1, device=gpu)
+    for call in (lambda: fused_attn.attention_forward(32, 32, q, k, v, None), lambda: fused_attn.attention_forward_ex(q, k, v, 32),
+                 lambda: fused_attn.qkv_projection(x, w, None, 1, 64, None, None)):
+        call()
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda z: (z * call().float().sum()).sum())(one)
+        with pytest.raises(RuntimeError):
+            torch.func.jvp(lambda z: call(), (one,), (one,))
+    with pytest.raises(RuntimeError):
+        torch.func.functionalize(lambda z: fused_attn.attention_forward_ex(q, k, v, 32))(one)
+
+
+def test_profiler_sees_the_tensors_of_the_compiled_module(gpu):
+    import fused_attn
+
+    q, k, v = (_rand((2, 33, 64), 8110 + i).to(gpu) for i in range(3))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        fused_attn.attention_forward(32, 32, q, k, v, None)
+        fused_attn.attention_forward_ex(q, k, v, 32, return_lse=True)
+    seen = {e.key: e.count for e in prof.key_averages()}
+    assert seen.get("aten::empty_like") == 1 and seen.get("aten::empty") == 2
 
 
 @pytest.mark.parametrize("listen", [False, True])

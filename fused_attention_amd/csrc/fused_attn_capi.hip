@@ -290,13 +290,7 @@ template <int H, int NQ, int GK, int MODE, bool BF>
 hipError_t launch_group(const fa::FwdParams& p, hipStream_t stream) {
     constexpr int lds = fa::group_lds_bytes<H, NQ, GK, MODE == fa::kAdditive>();
     static_assert(lds <= 160 * 1024, "fits a compute unit");
-    // 16-row waves: six per SIMD, three workgroups per compute unit.  Masked launches with the two that three ring
-    // slots left room for: B2 R12 L2048 H64 bias (768 workgroups) took 52.7 us instead of 44.3, B16 R12 L381
-    // padding (576) 21.0 instead of 18.6, B14 R8 L576 (bf16) 23.2 instead of 20.0.  Launches without a mask stay below the 80
-    // registers of six by themselves: 260 shapes, plain and causal, take the time that they take with a bound of four
-    // (1.000 in the mean for one and for two key groups).  At head_dim 16 and 32 without a mask eight, four workgroups: two
-    // sub-tiles at a time (split_two) take 65 registers if they are let.
-    constexpr int WPE = NQ == 1 && H <= 32 && MODE != fa::kAdditive ? 8 : NQ == 1 && H <= 64 ? 6 : NQ == 1 || H <= 64 ? 4 : 2;
+    constexpr int WPE = fa::group_waves_per_simd<H, NQ, MODE == fa::kAdditive>();
     auto kernel = BF ? fa::bf16::fwd_kernel_group<H, NQ, GK, MODE, WPE> : fa::fwd_kernel_group<H, NQ, GK, MODE, WPE>;
     if constexpr (lds > 64 * 1024) {
         const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), lds);

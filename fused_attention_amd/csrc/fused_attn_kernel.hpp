@@ -288,6 +288,14 @@ constexpr int group_lds_bytes() {
     constexpr int ring = group_ring_bytes<H, GK, MASK>() + (MASK ? 8 * group_sub<H, GK>() * NQ * 1024 : 0), part = GK == 1 ? 8 * 16 * (H + 8) * 2 : 8 / GK * group_part_bytes<H, NQ>();
     return ring > part ? ring : part;
 }
+// Waves per SIMD that the group kernel's registers are to last for.  16-row waves: six, three workgroups per compute unit.
+// Masked launches with the two that three ring slots left room for: B2 R12 L2048 H64 bias (768 workgroups) took
+// 52.7 us instead of 44.3, B16 R12 L381 padding (576) 21.0 instead of 18.6, B14 R8 L576 (bf16) 23.2 instead of 20.0.
+// Launches without a mask stay below the 80 registers of six by themselves: 260 shapes, plain and causal, take the
+// time that they take with a bound of four (1.000 in the mean for one and for two key groups).  At head_dim 16 and 32
+// without a mask eight, four workgroups: two sub-tiles at a time (split_two) take 65 registers if they are let.
+template <int H, int NQ, bool MASK>
+constexpr int group_waves_per_simd() { return NQ == 1 && H <= 32 && !MASK ? 8 : NQ == 1 && H <= 64 ? 6 : NQ == 1 || H <= 64 ? 4 : 2; }
 // (written in assembly so that the compiler does not see an LDS write, see RingLoader)
 __device__ __forceinline__ void group_dma16(uint32_t lds_addr, const _Float16* base, uint32_t voff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(base) : "memory", "m0");

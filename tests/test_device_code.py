@@ -1,5 +1,6 @@
 """What the compiler made of the kernels, read in the assembly it prints for them, and the host side of what
 the kernels compute with (no GPU needed)."""
+import concurrent.futures
 import os
 import re
 import subprocess
@@ -10,32 +11,49 @@ from fused_attention_amd import build
 
 HIPCC = os.path.join(build.ROCM, "bin", "hipcc")
 
-# (head_dim, blocks of 16 rows per wave, key groups, waves per SIMD): two and three ring slots, one and two key groups, one
-# sub-tile at a time and two
-GROUP_KERNELS = [(16, 1, 2, 6), (32, 1, 1, 8), (32, 2, 1, 4), (64, 1, 1, 6), (128, 1, 1, 4), (128, 1, 2, 4)]
+# (head_dim, blocks of 16 rows per wave, key groups): two and three ring slots, one and two key groups, one sub-tile at a time
+# and two.  The registers that a kernel may have come from where the launcher takes them.
+GROUP_KERNELS = [(16, 1, 1), (16, 1, 2), (32, 1, 1), (32, 1, 2), (32, 2, 1), (64, 1, 1), (128, 1, 1), (128, 1, 2)]
+ELEMENTS = ["fp16", "bf16"]
 
 
 @pytest.fixture(scope="module")
 def group_kernels(tmp_path_factory):
-    """{(head_dim, NQ, GK, mode): [lines of the kernel's assembly]}, unmasked (mode 0) and causal (2), fp16."""
+    """{(element, head_dim, NQ, GK, mode): ([lines of the kernel's assembly], {what its metadata say})}, unmasked (mode 0) and
+    causal (2)."""
     if not os.path.exists(HIPCC):
         pytest.skip("no hipcc")
     where = tmp_path_factory.mktemp("asm")
-    source = ['#include "%s"' % os.path.join(build.CSRC, "fused_attn_kernel.hpp")]
-    source += ["template __global__ void fa::fwd_kernel_group<%d, %d, %d, fa::%s, %d>(const fa::SplitParams);" % (h, nq, gk, mode, wpe)
-               for h, nq, gk, wpe in GROUP_KERNELS for mode in ("kPlain", "kCausal")]
-    (where / "one.hip").write_text("\n".join(source) + "\n")
-    subprocess.run([HIPCC] + build.HIPCC_FLAGS + ["--cuda-device-only", "-S", str(where / "one.hip"), "-o", str(where / "one.s")],
-                   check=True, capture_output=True)
-    kernels, lines = {}, None
-    for line in (where / "one.s").read_text().splitlines():
-        found = re.match(r"_ZN2fa16fwd_kernel_groupILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E\w+:", line)
-        if found:
-            lines = kernels[tuple(int(n) for n in found.groups())] = []
-        elif line.startswith(".Lfunc_end"):
-            lines = None
-        elif lines is not None:
-            lines.append(line.strip())
+
+    def compiled(element):
+        space = "fa::bf16" if element == "bf16" else "fa"
+        source = ['#include "%s"' % os.path.join(build.CSRC, "fused_attn_kernel.hpp")]
+        source += ["template __global__ void %s::fwd_kernel_group<%d, %d, %d, fa::%s, fa::group_waves_per_simd<%d, %d, false>()>(const fa::SplitParams);"
+                   % (space, h, nq, gk, mode, h, nq) for h, nq, gk in GROUP_KERNELS for mode in ("kPlain", "kCausal")]
+        (where / (element + ".hip")).write_text("\n".join(source) + "\n")
+        subprocess.run([HIPCC] + build.HIPCC_FLAGS + ["--cuda-device-only", "-S", str(where / (element + ".hip")), "-o", str(where / (element + ".s"))],
+                       check=True, capture_output=True)
+        return (where / (element + ".s")).read_text()
+
+    with concurrent.futures.ThreadPoolExecutor() as pool:
+        texts = dict(zip(ELEMENTS, pool.map(compiled, ELEMENTS)))
+    kernels = {}
+    name = r"_ZN2fa(?:4bf16)?16fwd_kernel_groupILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E"
+    for element, text in texts.items():
+        lines = None
+        for line in text.splitlines():
+            found = re.match(name + r"\w+:", line)
+            if found:
+                lines = []
+                kernels[(element,) + tuple(int(n) for n in found.groups())] = lines, {}
+            elif line.startswith(".Lfunc_end"):
+                lines = None
+            elif lines is not None:
+                lines.append(line.strip())
+        for entry in text[text.index("amdhsa.kernels:"):].split("  - .agpr_count:")[1:]:
+            found = re.search(r"\.name: +" + name, entry)
+            kernels[(element,) + tuple(int(n) for n in found.groups())][1].update(
+                (key, int(n)) for key, n in re.findall(r"\.(private_segment_fixed_size|vgpr_spill_count|vgpr_count): +(\d+)", entry))
     return kernels
 
 
@@ -52,13 +70,25 @@ def _loop_lines(lines):
 
 
 @pytest.mark.parametrize("mode", [0, 2])
-@pytest.mark.parametrize("H,NQ,GK,wpe", GROUP_KERNELS)
-def test_the_group_kernel_waits_for_its_queries_once(group_kernels, H, NQ, GK, wpe, mode):
+@pytest.mark.parametrize("H,NQ,GK", GROUP_KERNELS)
+@pytest.mark.parametrize("element", ELEMENTS)
+def test_the_group_kernel_waits_for_its_queries_once(group_kernels, H, NQ, GK, mode, element):
     # The key tiles come by loads written in assembly, with exact waits of their own, so that the only loads the compiler
     # knows of are the queries'.  A wait of its making inside a loop would be one for the key tiles on their way, in every pass.
-    lines = group_kernels[H, NQ, GK, mode]
+    lines, _ = group_kernels[element, H, NQ, GK, mode]
     assert any("s_barrier" in line for line in _loop_lines(lines))
     assert [line for line in _loop_lines(lines) if line.startswith("s_waitcnt") and "vmcnt" in line] == []
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("H,NQ,GK", GROUP_KERNELS)
+@pytest.mark.parametrize("element", ELEMENTS)
+def test_the_group_kernel_keeps_its_values_in_registers(group_kernels, H, NQ, GK, mode, element):
+    # None of its values pass through memory, with as many waves per SIMD as the launcher compiles it for (64 registers with
+    # eight, 80 with six, 128 with four).
+    _, said = group_kernels[element, H, NQ, GK, mode]
+    assert said["private_segment_fixed_size"] == said["vgpr_spill_count"] == 0
+    assert said["vgpr_count"] <= (64 if NQ == 1 and H <= 32 else 80 if NQ == 1 and H <= 64 else 128)
 
 
 def test_division_by_multiplication_is_exact(tmp_path):

@@ -853,16 +853,14 @@ def test_eight_wave_kernel_on_adversarial_scores(gpu, B, R, L, H, kind):
     assert scores.abs().max() > 20
 
 
-@pytest.mark.parametrize("B,R,L,H,mode", [
-    (4, 16, 2048, 64, "plain"), (2, 64, 1024, 128, "plain"), (4, 16, 2048, 64, "causal"), (2, 64, 1024, 128, "causal"),    # 16-row blocks
-    (8, 12, 1024, 64, "plain"), (4, 32, 2048, 32, "plain"), (4, 16, 2048, 64, "mask"), (1, 12, 12288, 64, "causal"),        # 32-row blocks
-])
+@pytest.mark.parametrize("H,mode,edge", [(64, "plain", 16), (128, "plain", 16), (64, "causal", 16), (128, "causal", 16),
+                                         (64, "plain", 32), (32, "plain", 32), (64, "mask", 32), (64, "causal", 32)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_some_blocks_of_a_wave_move_their_reference(gpu, B, R, L, H, mode, dtype):
+def test_some_blocks_of_a_wave_move_their_reference(gpu, H, mode, edge, dtype):
     # The tile kernels send only those blocks of 16 (32) query rows down the slow path that a row of theirs needs it for.
     # A few rows, spread over the blocks and waves, meet late keys whose scores stand 40 log2 units and more above the
     # rest (bf16's leash is 29), one after the other; every row around them keeps the reference it has.
-    assert capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")["kernel"] == "tile"
+    B, R, L = _shape_on("tile", H, mode, [2048, 1024, 4096, 12288], edge=edge)
     q, k, v = (_rand((B, L, R, H), 4150 + L + i) for i in range(3))
     hot = torch.tensor([L - 1 - r for r in (0, 5, 21, 38, 63, 64, 130, 200, 259, 330, 511)])
     q[..., 0] = 0.0
@@ -1078,13 +1076,14 @@ def test_mask_rows_at_any_alignment(gpu, L, H):
         assert _max_err(got[b, :, sl], want[0]) <= TOL, (b, h)
 
 
-def _shape_on(kernel, H, mode, lengths, rows=None, fits=lambda v: True):
+def _shape_on(kernel, H, mode, lengths, rows=None, fits=lambda v: True, edge=None):
     """The first (B, R, L) of a small grid of problems, of one of these lengths, that the library runs on this
-    kernel (and, if given, with this many query rows per workgroup and a launch that `fits`)."""
+    kernel (and, if given, with this many query rows per workgroup, a launch that `fits` and matrix tiles of this edge)."""
     for L in lengths:
         for B, R in [(1, r) for r in range(1, 64)] + [(2, 40), (1, 96), (1, 128), (1, 160), (2, 120), (1, 320)]:
             v = capi.launch_variant(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")
-            if v["kernel"] == kernel and (rows is None or v["rows"] == rows) and fits(v):
+            if v["kernel"] == kernel and (rows is None or v["rows"] == rows) and fits(v) and (
+                    edge is None or capi.launch_plan(B, R, L, H, causal=mode == "causal", has_mask=mode == "mask")["matrix_tile"] == edge):
                 return B, R, L
     raise AssertionError((kernel, H, mode, lengths, rows))
 
@@ -1274,13 +1273,14 @@ def test_whole_key_tiles_of_the_group_kernel(gpu, H, mode, rows, kind, dtype):
 
 @pytest.mark.parametrize("H", [16, 32])
 @pytest.mark.parametrize("mode", ["plain", "causal"])
-@pytest.mark.parametrize("L", [128, 704, 769, 865, 1087])
+@pytest.mark.parametrize("L", ["short", 704, 769, 865, 1087])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_two_sub_tiles_at_a_time(gpu, H, mode, L, dtype):
     # 16-row waves at head_dim 16 and 32 take the sub-tiles of a whole key tile two at a time: one whole tile behind the
-    # first, an odd and an even number of them, remainders of 0, 1, 33 and 63 keys.  The scores of some rows leave
-    # the reference in the first sub-tile of a pair, those of others in the second one.
-    B, R, L = _shape_on("group", H, mode, [L], 128)
+    # first ("short"; causal: below the diagonal of the wave from row 144 on), an odd and an even number of them, remainders of 0,
+    # 1, 33 and 63 keys.  The scores of some rows leave the reference in the first sub-tile of a pair, those of others in the second one.
+    short = L == "short"
+    B, R, L = _shape_on("group", H, mode, [L] if not short else [128] if mode == "plain" else [160, 192, 224, 256, 320, 384], 128)
     q, k, v = (_rand((B, L, R, H), 6250 + L + i) for i in range(3))
     up = torch.arange(L) // 32
     q[..., 0], q[..., 1] = 4.0, 4.0
@@ -1289,6 +1289,11 @@ def test_two_sub_tiles_at_a_time(gpu, H, mode, L, dtype):
     k[..., 0] = ((up // 10 * 40.0) * 0.6931 * H ** 0.5 / 4.0)[None, :, None]           # first sub-tiles of a pair
     k[..., 1] = (((up + 5) // 8 * 40.0) * 0.6931 * H ** 0.5 / 4.0)[None, :, None]      # second ones
     q, k, v = (t.reshape(B, L, R * H).to(dtype) for t in (q, k, v))
+    # pairs of that wave, or the last whole one: the reference fails, is looked at first and, given time, is trusted and holds
+    variant = capi.launch_variant(B, R, L, H, causal=mode == "causal")
+    row = 144 if short and mode == "causal" else L // 16 * 16 - 16
+    steps = _whole_tile_steps(q[0, :, :H], k[0, :, :H], H, mode, dtype == torch.bfloat16, variant, [(row, 0)])[0]
+    assert steps == "f" if short else steps.startswith("flltfl"), steps
     got, lse = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, causal=mode == "causal", return_lse=True)
     one = causal_mask(1, L).float() if mode == "causal" else None
     for b, h in [(0, 0), (B - 1, R - 1)]:
@@ -1300,6 +1305,37 @@ def test_two_sub_tiles_at_a_time(gpu, H, mode, L, dtype):
         want = attention_lse(args[0], args[1], H, mask=one)[0, 0]
         off = (lse[b, h].cpu() - want).abs() - 2e-5 * want.abs()
         assert off.max().item() <= 2.0 ** (-8 if dtype == torch.bfloat16 else -10) * 1.01 + 1e-5, (b, h)
+
+
+@pytest.mark.parametrize("H", [16, 32])
+@pytest.mark.parametrize("mode", ["plain", "causal"])
+@pytest.mark.parametrize("at", [64 + 3, 64 + 32 + 21, 320 + 9])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_non_finite_inputs_in_two_sub_tiles(gpu, H, mode, at, dtype):
+    # An inf in a key of the first or the second sub-tile of a pair (score +inf for some rows: NaN; -inf for the others:
+    # no weight) and a NaN in a query: the rows that the oracle leaves finite match it, the others are not finite, and the
+    # heads without any do not change a bit.
+    B, R, L = _shape_on("group", H, mode, [704], 128)
+    q, k, v = (_rand((B, L, R * H), 6350 + i).to(dtype) for i in range(3))
+    clean = capi.forward(q.to(gpu), k.to(gpu), v.to(gpu), H, causal=mode == "causal").cpu()
+    q2, k2 = q.clone(), k.clone()
+    q2[0, 437, 3] = float("nan")                      # head 0, query 437
+    k2[B - 1, at, H + 1] = float("inf")               # head 1 of the last batch
+    got = capi.forward(q2.to(gpu), k2.to(gpu), v.to(gpu), H, causal=mode == "causal").cpu()
+    one = causal_mask(1, L).float() if mode == "causal" else None
+    same = (got == clean).view(B, L, R, H).all(-1).all(1)
+    same[0, 0] = same[B - 1, 1] = True
+    assert same.all()
+    for b, h in ((0, 0), (B - 1, 1)):
+        sl = slice(h * H, (h + 1) * H)
+        want = attention(q2[b:b + 1, :, sl].float(), k2[b:b + 1, :, sl].float(), v[b:b + 1, :, sl].float(), H, mask=one)[0]
+        if mode == "causal":        # rows ahead of the key do not see it (the oracle's mask added to it is no number)
+            want[:at] = attention(q2[b:b + 1, :at, sl].float(), k[b:b + 1, :at, sl].float(), v[b:b + 1, :at, sl].float(), H, mask=one[:, :at, :at])[0]
+        mine = got[b, :, sl].float()
+        bad = ~torch.isfinite(want).all(dim=-1)
+        assert bad.sum() == 1 if h == 0 else 10 < bad.sum() < L - 10
+        assert (~torch.isfinite(mine[bad])).any(dim=-1).all()
+        assert (mine[~bad] - want[~bad]).abs().max().item() <= (2e-2 if dtype == torch.bfloat16 else TOL)
 
 
 @pytest.mark.parametrize("H,mode,B,R,L,limit", [(16, "plain", 16, 12, 705, 1.33), (32, "causal", 6, 8, 2561, 1.28), (128, "plain", 1, 20, 1473, 1.22)])

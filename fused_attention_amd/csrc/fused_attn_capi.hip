@@ -425,11 +425,17 @@ int validate(const void* q, const void* k, const void* v, const void* mask, void
 // causal ones in part behind a producer of q, k and v.  What counts is the order of the estimates, so that is what
 // was fitted: the time lost against the best kernel of each call, with a share of the estimates' own error.  Choosing the
 // smallest one loses 0.9 % on these calls, more than 3 % on 10 % of them, and 0.9 % on 600 left out of the fit (the fit
-// before, of the kernels as they were then: 1.9, 20 and 1.7 %).  The 600 take 0.8 % less time than with that fit, 61 of them
-// more than 3 % less and five 3 to 14 % more.  Calls whose kernel the tests name were held where they are: without that the
-// loss is 0.6 % (B8 R12 L1024 H64: 32.2 us on the tile kernel, 30.4 on 16-row waves of the group kernel).  Two key groups
-// read K and V twice as often and lose their lead behind the projection, whose stores pass L2 (B1 R40 L512 H128 causal:
-// 12.6 us against 12.9 alone, 2 us more in the block); the fit counts that.
+// before, of the kernels as they were then: 1.9, 20 and 1.7 %).  Two things in the fit are not measured times.  The 93 problems
+// whose kernel the tests name were held where they are, by a penalty: without it the loss is 0.6 % (B8 R12 L1024 H64: 32.2 us
+// on the tile kernel, 30.4 on 16-row waves of the group kernel).  And the times of two key groups behind a producer were taken
+// 1.1 times as long: the producer that was timed is a copy, and behind the projection, whose stores pass L2, K and V
+// are read twice as often from further away (measured on one call, B1 R40 L512 H128 causal: 12.6 us against 12.9 alone, 2 us
+// more in the block).
+// Against the choice before, of all 7271 calls 794 take over 3 % less time and 69 over 3 % more, scattered over the ranges; the
+// furthest, timed again: B1 R16 L9344 H64 causal 209 -> 252 us (two key groups before, the tile kernel now), B11 R12 L397 H128
+// causal 19.8 -> 23.7 (two key groups, 16 rows), B6 R40 L2924 H16 padding 584 -> 697 (tile, 16 rows).  Other weights in the fit move
+// them elsewhere (10 to 15 of 1000 calls outside a fit, with eight times the weight on calls that get slower or without the
+// tests' problems): estimates of four terms cannot tell these calls from their neighbours.
 //   split:  kLaunch + a ceil(sub-tiles / waves)              the longest wave
 //                   + b sub-tiles of all workgroups / 256    one compute unit's share of the work
 //                   + c k                                    start and merge
